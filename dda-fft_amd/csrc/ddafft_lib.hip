@@ -197,7 +197,7 @@ struct ddafft_ctx {
     bool have_target = false;
 
     // matvec scratch
-    float2 *b1 = nullptr, *b2 = nullptr, *b3 = nullptr;
+    float2 *b1 = nullptr, *b2 = nullptr, *b3 = nullptr;   // b3: kInPlaceBytes at most (launch_matvec)
     // solver fields [nrhs][3][n]
     float2 *P = nullptr, *Pmin = nullptr, *R = nullptr, *S = nullptr, *G = nullptr, *H = nullptr, *W = nullptr;
     float2 *X = nullptr, *Y = nullptr;
@@ -425,9 +425,16 @@ int zi_blocks(const Dims& d) {
         default: return fail(DDAFFT_EINVAL, "unsupported line length");                                 \
     }
 
-struct PassEvents {
-    hipEvent_t* ev;  // 6 events bracketing the 5 passes, or nullptr
-};
+// The X pass writes over its input (B3 is B2) where one of them is larger
+// than this, the 8 x 4 MB of L2: the write then hits the lines the tile has
+// just read, and a matvec touches 192 N bytes a right-hand side less, so that
+// more of Â stays in the 256 MB memory-side cache.  X pass, MI355X, against
+// separate buffers: 64^3, 2 RHS (50 MB) 49.5 -> 41.8 us; 32x32x64, 16 RHS
+// (101 MB) 66.9 -> 60.1; 256^3, 2 RHS 4.11 -> 3.22 ms.  Smaller ones keep two
+// buffers: in place, every line changes its writer twice a matvec, and the
+// forward pass that fills it from another XCD pays for that (64x32x64, 1 RHS,
+// 13 MB: fused forward pass 13.2 -> 18.5 us, X pass 20.4 -> 19.6).
+constexpr size_t kInPlaceBytes = (size_t)32 << 20;
 
 // Host-side check that every pointer a pass will dereference is set, so that
 // a sequencing mistake returns an error instead of faulting the GPU.
@@ -501,6 +508,7 @@ int launch_matvec(ddafft_ctx* c, int nrhs, const ProArgs& pa, SolveState* st, in
     const int C = 3 * nrhs;
     hipStream_t s = c->stream;
     const Schedule sch = schedule(c, nrhs);
+    float2* b3 = (size_t)4 * d.n * C * sizeof(float2) <= kInPlaceBytes ? c->b3 : c->b2;
     if (ev) HIPCHECK(hipEventRecord(ev[0], s));
     // z and y forward: fused per i-plane for planes up to 64 x 64, else ZF then YF
     if (sch.fuse && zyf_launch(c, d, pa, st, C, s)) {
@@ -534,8 +542,8 @@ int launch_matvec(ddafft_ctx* c, int nrhs, const ProArgs& pa, SolveState* st, in
         const int gpb = (ngroups + ysets - 1) / ysets;
         dim3 grid(ntile, (ngroups + gpb - 1) / gpb);
 #define DDA_KX(SW, RB, RUN, CP)                                                                           \
-    SW(d.ni, hipLaunchKernelGGL((k_x<NN, RB, RUN, CP>), grid, kBlock, 0, s, d, st, c->b2, c->b3, c->ahat, conj, \
-                                c->wpre_i, c->tw_i, c->tw_2i, gpb))
+    SW(d.ni, hipLaunchKernelGGL((k_x<NN, RB, RUN, CP>), grid, kBlock, 0, s, d, st, c->b2, b3, c->ahat, conj, c->wpre_i, \
+                                c->tw_2i, gpb))
 #define DDA_KX_RB(RUN, CP)                              \
     {                                                   \
         if (rb == 4) DDA_KX(DDA_SWITCH_X, 4, RUN, CP)      \
@@ -557,7 +565,7 @@ int launch_matvec(ddafft_ctx* c, int nrhs, const ProArgs& pa, SolveState* st, in
     {
         const int tl = std::min(tile_yi(2 * d.nj), 2 * d.nl);
         dim3 grid(d.ni * (2 * d.nl / tl), C);
-        DDA_SWITCH_LARGE(2 * d.nj, hipLaunchKernelGGL((k_yi<NN>), grid, kBlock, 0, s, d, st, c->b3, c->b1, c->tw_2j));
+        DDA_SWITCH_LARGE(2 * d.nj, hipLaunchKernelGGL((k_yi<NN>), grid, kBlock, 0, s, d, st, b3, c->b1, c->tw_2j));
     }
     if (ev) HIPCHECK(hipEventRecord(ev[4], s));
     {
@@ -991,7 +999,7 @@ int ddafft_create(int ni, int nj, int nl, float kd, int nrhs_max, ddafft_ctx** o
     if (!rc) rc = dev_alloc(&c->ahat, (size_t)P * 6);
     if (!rc) rc = dev_alloc(&c->b1, (size_t)(2 * n * C));
     if (!rc) rc = dev_alloc(&c->b2, (size_t)(4 * n * C));
-    if (!rc) rc = dev_alloc(&c->b3, (size_t)(4 * n * C));
+    if (!rc) rc = dev_alloc(&c->b3, std::min((size_t)(4 * n * C), kInPlaceBytes / sizeof(float2)));
     float2** fields[] = {&c->P, &c->Pmin, &c->R, &c->S, &c->G, &c->H, &c->W, &c->X, &c->Y};
     for (float2** f : fields)
         if (!rc) rc = dev_alloc(f, (size_t)(n * C));

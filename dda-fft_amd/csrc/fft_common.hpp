@@ -203,7 +203,10 @@ __device__ __forceinline__ int rest_natural(int g) {
     return (int)j;
 }
 
-template <int N, int T>
+// TWS: stride of the line's twiddles in `tw` (W_N^q at tw[q TWS]), so that
+// transforms of N points can use a longer plan's table: W_N^q and W_2N^2q are
+// the same floats (their double arguments are equal).
+template <int N, int T, int TWS = 1>
 struct StageRunner {
     static __device__ __forceinline__ void run(float2* s, const LineWalk& w, int ls, const float2* __restrict__ tw,
                                                int span_prev) {
@@ -223,7 +226,7 @@ struct StageRunner {
 #pragma unroll
                 for (int q = 0; q < R; ++q) z[q] = v[q * H];
                 if (R > 2 && i > 0) {
-                    const int ts = i * step;
+                    const int ts = i * step * TWS;
                     int tq = 0;
 #pragma unroll
                     for (int q = 1; q < R; ++q) {
@@ -240,7 +243,7 @@ struct StageRunner {
                 w.step(b, line);
             }
             __syncthreads();
-            StageRunner<N, T + 1>::run(s, w, ls, tw, span);
+            StageRunner<N, T + 1, TWS>::run(s, w, ls, tw, span);
         }
     }
 };
@@ -271,8 +274,9 @@ __device__ __forceinline__ void lane_pos(unsigned f, unsigned& line, unsigned& b
     }
 }
 
-// TEND: the stage to stop before (the caller runs the stages from TEND on).
-template <int N, int NL, int LS, int T, int BT = kBlock, int TEND = Plan<N>::NST>
+// TEND: the stage to stop before (the caller runs the stages from TEND on);
+// TWS: twiddle stride, as in StageRunner.
+template <int N, int NL, int LS, int T, int BT = kBlock, int TEND = Plan<N>::NST, int TWS = 1>
 struct FixedStage {
     static __device__ __forceinline__ void run(float2* s, const float2* __restrict__ tw) {
         if constexpr (T < TEND) {
@@ -297,7 +301,7 @@ struct FixedStage {
 #pragma unroll
                     for (int q = 0; q < R; ++q) z[q] = v[q * H];
                     if (R > 2 && i > 0) {
-                        const unsigned ts = i * step;
+                        const unsigned ts = i * step * TWS;
                         unsigned tq = 0;
 #pragma unroll
                         for (int q = 1; q < R; ++q) {
@@ -314,13 +318,14 @@ struct FixedStage {
                 }
             }
             __syncthreads();
-            FixedStage<N, NL, LS, T + 1, BT, TEND>::run(s, tw);
+            FixedStage<N, NL, LS, T + 1, BT, TEND, TWS>::run(s, tw);
         }
     }
 };
 
-// BT: threads per block; TEND: the stage to stop before (Plan<N>::NST: all)
-template <int N, int NL, int LS, int BT = kBlock, int TEND = Plan<N>::NST>
+// BT: threads per block; TEND: the stage to stop before (Plan<N>::NST: all);
+// TWS: twiddle stride
+template <int N, int NL, int LS, int BT = kBlock, int TEND = Plan<N>::NST, int TWS = 1>
 __device__ __forceinline__ void fft_lds_fixed(float2* s, const float2* __restrict__ tw) {
     constexpr int K = Plan<N>::K;
     constexpr int R0 = plan_radix(K, 0);
@@ -354,7 +359,7 @@ __device__ __forceinline__ void fft_lds_fixed(float2* s, const float2* __restric
         }
     }
     __syncthreads();
-    FixedStage<N, NL, LS, 1, BT, TEND>::run(s, tw);
+    FixedStage<N, NL, LS, 1, BT, TEND, TWS>::run(s, tw);
 }
 
 // The last stage of NLINES line transforms of N points in LDS (stride LS),
@@ -401,12 +406,12 @@ __device__ __forceinline__ void fft_last_stage_out(const float2* s, const float2
 
 // MAXL: the most lines any call of this instance passes (sizes the registers
 // that carry stage 0 across its barrier); LS: the line stride in float2.
-// Ends with a __syncthreads.
-template <int N, int MAXL, int LS>
+// TWS: twiddle stride.  Ends with a __syncthreads.
+template <int N, int MAXL, int LS, int TWS = 1>
 __device__ __forceinline__ void fft_lds(float2* s, int nlines, const float2* __restrict__ tw) {
     constexpr int ls = LS;
     if (nlines == MAXL) {   // the usual case: full tiles
-        fft_lds_fixed<N, MAXL, LS>(s, tw);
+        fft_lds_fixed<N, MAXL, LS, kBlock, Plan<N>::NST, TWS>(s, tw);
         return;
     }
     constexpr int K = Plan<N>::K;
@@ -442,7 +447,7 @@ __device__ __forceinline__ void fft_lds(float2* s, int nlines, const float2* __r
         }
     }
     __syncthreads();
-    StageRunner<N, 1>::run(s, w, ls, tw, R0);
+    StageRunner<N, 1, TWS>::run(s, w, ls, tw, R0);
 }
 
 // ---------------------------------------------------------------------------

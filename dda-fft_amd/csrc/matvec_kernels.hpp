@@ -5,7 +5,9 @@
 // HBM layouts (float2 = complex64, C = 3*nrhs component planes):
 //   field x, out : [C][ni][nj][nl]            (one plane per component)
 //   B1 / B4      : [C][ni][2nl'][nj] / [C][ni][nj][2nl']
-//   B2 / B3      : [C][2nj][ni][2nl']         (an X tile's i rows 2nl apart)
+//   B2 / B3      : [C][2nj][ni][2nl']         (an X tile's i rows 2nl apart);
+//                  one buffer, the X pass in place, where it is larger than
+//                  the L2 caches, else two
 //   Â            : [2nj][2nl][2ni][6]         (e00 e01 e02 e11 e12 e22)
 // L' is the z-frequency in parity-split order: L' = L / 2 for even L and
 // n_l + L / 2 for odd L, the order in which the pruned z transform produces
@@ -521,10 +523,9 @@ __device__ __forceinline__ unsigned long long x_active(const Dims& d, const Solv
 // constant and the index arithmetic reduces to shifts and masks; otherwise
 // tj = 2 n_j.
 template <int NI, int RB, bool FULL, bool RUN, bool COMPACT>
-__device__ __forceinline__ void x_tile(const Dims& d, unsigned long long amask, int g0, int g1, int tj_small, const float2* __restrict__ b2, float2* __restrict__ b3,
+__device__ __forceinline__ void x_tile(const Dims& d, unsigned long long amask, int g0, int g1, int tj_small, const float2* b2, float2* b3,
                                        const float2* __restrict__ ahat, int conj, const float2* __restrict__ wpre,
-                                       const float2* __restrict__ tw1, const float2* __restrict__ tw2, float2* s,
-                                       float2* stw1, float2* stw2) {
+                                       const float2* __restrict__ tw2, float2* s, float2* stw2) {
     // conj: the conjugate convolution (Â at -k, conjugated).  COMPACT: Â
     // stored as one octant (the reference's padded A(r) with its Nyquist
     // planes zeroed, so that Â is even or odd along every axis).
@@ -604,7 +605,6 @@ __device__ __forceinline__ void x_tile(const Dims& d, unsigned long long amask, 
         // every load in flight first)
         auto stage_twiddles = [&]() {
             if (!staged) {
-                for (int f = threadIdx.x; f < NI; f += kBlock) stw1[f] = tw1[f];
                 for (int f = threadIdx.x; f < NI2; f += kBlock) stw2[f] = tw2[f];
                 staged = true;
             }
@@ -658,7 +658,7 @@ __device__ __forceinline__ void x_tile(const Dims& d, unsigned long long amask, 
                 }
             }
             __syncthreads();
-            FixedStage<NI, 2 * NCOL, LS1, 1>::run(s, stw1);
+            FixedStage<NI, 2 * NCOL, LS1, 1, kBlock, Plan<NI>::NST, 2>::run(s, stw2);
         } else {
             {
                 // all loads of this thread are issued before the first is used;
@@ -688,7 +688,7 @@ __device__ __forceinline__ void x_tile(const Dims& d, unsigned long long amask, 
                 }
             }
             __syncthreads();
-            fft_lds<NI, 2 * CB * TJ, LS1>(s, 2 * CB * tj, stw1);
+            fft_lds<NI, 2 * CB * TJ, LS1, 2>(s, 2 * CB * tj, stw2);
         }
 
         // Â multiply in natural order of I, one Â read for every right-hand
@@ -721,7 +721,7 @@ __device__ __forceinline__ void x_tile(const Dims& d, unsigned long long amask, 
             }
         }
         __syncthreads();
-        // B3 [C][J][i][L'], as B2
+        // B3 [C][J][i][L'], as B2 (in place: the cells the tile was read from)
         float2* dst = b3 + ((long long)(rhs0 * 3) * NJ2 + J) * NI * NL2 + L0;
         constexpr int NSTI = Plan<NI2>::NST;
         if constexpr (FULL && NSTI >= 2 && XRegStages<NI, RB>::INV) {
@@ -778,21 +778,24 @@ __device__ __forceinline__ void x_tile(const Dims& d, unsigned long long amask, 
     }
 }
 
+// b3 may be b2: a block reads all of its tile before it writes it, and no
+// other block touches those cells (so neither pointer is __restrict__).  The
+// 2 n_i-point twiddles serve the n_i-point lines too, at twice the stride
+// (256^3: the tile and they leave three blocks per CU instead of two).
+//
 // Grid: x over (J, L) tiles, y over sets of `gpb` consecutive right-hand-side
 // groups of RB (RUN; otherwise gpb = 1); each block reads its tile's Â once
 // for all of its groups.
 template <int NI, int RB, bool RUN, bool COMPACT>
 __global__ __launch_bounds__(kBlock) DDA_WAVES_PER_EU(XWaves<NI, RB, RUN, COMPACT>::W) void k_x(Dims d, const SolveState* __restrict__ st,
-                                              const float2* __restrict__ b2, float2* __restrict__ b3,
-                                              const float2* __restrict__ ahat, int conj,
-                                              const float2* __restrict__ wpre, const float2* __restrict__ tw1,
-                                              const float2* __restrict__ tw2, int gpb) {
+                                              const float2* b2, float2* b3, const float2* __restrict__ ahat, int conj,
+                                              const float2* __restrict__ wpre, const float2* __restrict__ tw2,
+                                              int gpb) {
     static_assert(RB == 1 || RB == 2 || RB == 4, "one, two or four right-hand sides per X tile");
     constexpr int TJ = TileX<NI, RB>::T;
     constexpr int LS1 = XStride<NI, RB>::S1, LS2 = XStride<NI, RB>::S2;
     static_assert(LS2 <= 2 * LS1, "the inverse lines fit the forward tile's LDS");
     __shared__ float2 s[3 * RB * TJ * 2 * LS1];
-    __shared__ float2 stw1[NI];
     __shared__ float2 stw2[2 * NI];
     const int ngroups = (d.nrhs + RB - 1) / RB;
     const int g0 = blockIdx.y * gpb, g1 = RUN ? min(g0 + gpb, ngroups) : g0 + 1;
@@ -805,9 +808,9 @@ __global__ __launch_bounds__(kBlock) DDA_WAVES_PER_EU(XWaves<NI, RB, RUN, COMPAC
     // 6571 -> 5688 us.
     const int tj = min(TJ, 2 * d.nl);
     if (tj == TJ)
-        x_tile<NI, RB, true, RUN, COMPACT>(d, amask, g0, g1, TJ, b2, b3, ahat, conj, wpre, tw1, tw2, s, stw1, stw2);
+        x_tile<NI, RB, true, RUN, COMPACT>(d, amask, g0, g1, TJ, b2, b3, ahat, conj, wpre, tw2, s, stw2);
     else
-        x_tile<NI, RB, false, RUN, COMPACT>(d, amask, g0, g1, tj, b2, b3, ahat, conj, wpre, tw1, tw2, s, stw1, stw2);
+        x_tile<NI, RB, false, RUN, COMPACT>(d, amask, g0, g1, tj, b2, b3, ahat, conj, wpre, tw2, s, stw2);
 }
 
 // ---------------------------------------------------------------------------
