@@ -4,6 +4,7 @@
 // pass over lattice-sized data runs on the GPU.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <complex>
 #include <cstdio>
@@ -190,8 +191,18 @@ struct ddafft_ctx {
     int nmat = 0;
     int* cells = nullptr;   // dipole cell indices (far field)
     int ncells = 0;
-    int2* ffseg = nullptr;  // far-field column segments {first dipole, (i nj + j) << 6 | count}
+    int* ffcol = nullptr;     // (i nj + j) of the columns that hold dipoles, each plane i padded to 8 with -1
+    int2* ffpiece = nullptr;  // 8 columns each over a range of l (k_far_field_cols), padded to 4
+    int nffpiece = 0;
+    // the S11 gradients' far field (k_far_field_grp): column segments
+    // {first dipole, (i nj + j) << 6 | count}, built by the first such call on a
+    // target, and the dipole moments in list order
+    int2* ffseg = nullptr;
     int nseg = 0;
+    float2* ffpc = nullptr;
+    size_t ffpc_cap = 0;
+    bool ff_s11 = false;      // such a call's forward solve is running
+    int ffs_n = 0, ffs_S = 1; // its split of the direction set, groups of at most kFFDirs
     long long ndip = 0;
     std::vector<long long> mat_count;  // dipoles per material index
     bool have_target = false;
@@ -235,11 +246,9 @@ struct ddafft_ctx {
     int sum_mode = 0;                  // observables: 0 FP64 sums, 1 the reference's sequential float sums
     int ahat_mode = 0;                 // 0: full Â as the reference builds it; 1: one octant (Nyquist planes zeroed)
     int ff_mfma = -1;                  // far field on the matrix cores: -1 default, 0 off, 1 on
-    int ff_group = -1;                 // far field by groups of directions sharing z: -1 default (on), 0 off, 1 on
-    int ffg_n = 0, ffg_S = 0;          // the resident direction set as ffg_n groups of ffg_S (0: no such split)
-    bool ffg_off_call = false;         // set by an allocation-free solve whose scratch cannot hold the grouped form
-    float2* ffpc = nullptr;            // dipole moments in dipole-list order for the grouped far field
-    size_t ffpc_cap = 0;
+    int ff_group = -1;                 // far field by columns: -1 default (on), 0 off, 1 on
+    int ffg_n = 0, ffg_S = 1;          // the direction set as ffg_n groups of ffg_S sharing z (dir_groups)
+    int ff_chunk_max = 0;              // set by an allocation-free solve: column chunks that its scratch has room for
     // launch schedule, 0 / -1: from the tuned table, else the built-in rule
     int x_blocks = 0;                  // X pass: blocks per launch up to which right-hand-side groups are spread
     int x_rb = 0;                      // X pass: right-hand sides per tile
@@ -942,7 +951,7 @@ int ddafft_destroy(ddafft_ctx* c) {
     void* bufs[] = {c->ahat, c->tables, c->occ, c->dipf, c->mv, c->cells, c->b1, c->b2, c->b3, c->P, c->Pmin, c->R,
                     c->S, c->G, c->H, c->W, c->X, c->Y, c->small, c->hist, c->partials,
                     c->dirs, c->esc, c->fftab, c->Pf, c->phase, c->gaux, c->inc_cell, c->seqbuf,
-                    c->ffseg, c->ffpc};
+                    c->ffcol, c->ffpiece, c->ffseg, c->ffpc};
     for (void* b : bufs)
         if (b) hipFree(b);
     if (c->state_ring) hipHostFree(c->state_ring);
@@ -1083,6 +1092,12 @@ int ddafft_get_ahat(ddafft_ctx* c, float* out) {
     return DDAFFT_OK;
 }
 
+// Far-field pieces that a target is cut into at least, where it spans that
+// many 16-point chunks: two batches of four for each of 256 CUs, so that a
+// long axis fills the chip (16x32x128, 400 columns: 39.8 -> 11.7 us against
+// whole columns); 1024 and 4096 measured the same within 2 us.
+static constexpr long long kFFPieces = 2048;
+
 int ddafft_set_target(ddafft_ctx* c, const signed char* occ, int nmat, const int* mv) {
     if (!c || !occ || !mv || nmat < 1 || nmat > 128) return fail(DDAFFT_EINVAL, "bad target arguments");
     const long long n = c->d.n;
@@ -1094,36 +1109,55 @@ int ddafft_set_target(ddafft_ctx* c, const signed char* occ, int nmat, const int
         if (mv[m]) cells.push_back((int)k);
     }
     if (cells.empty()) return fail(DDAFFT_EINVAL, "target has no dipoles");
-    // far-field segments: each run of dipoles in one (i, j) column, cut into
-    // near-equal pieces of at most kFFSeg
-    std::vector<int2> segs;
+    // far-field columns: the (i, j) that hold dipoles, and 8 of them at a time
+    // the 16-point chunks of l that their dipoles span, cut into pieces
+    std::vector<int> fcol;
+    std::vector<int2> fpiece;
     {
         const int lnl = __builtin_ctz(c->d.nl);
-        size_t e = 0;
-        while (e < cells.size()) {
-            const int ij = cells[e] >> lnl;
-            size_t e1 = e + 1;
-            while (e1 < cells.size() && (cells[e1] >> lnl) == ij) ++e1;
-            const int len = (int)(e1 - e), np = (len + kFFSeg - 1) / kFFSeg;
-            for (int q = 0, at = 0; q < np; ++q) {
-                const int cnt = (len - at) / (np - q);
-                segs.push_back(make_int2((int)e + at, (ij << 6) | cnt));
-                at += cnt;
+        const int lnj = __builtin_ctz(c->d.nj);
+        std::vector<std::pair<int, int>> span;   // chunks [lo, hi) of 8 columns of one plane i
+        for (const int k : cells) {
+            const int ij = k >> lnl, u = (k & (c->d.nl - 1)) >> 4;
+            if (fcol.empty() || fcol.back() != ij) {
+                if (!fcol.empty() && (fcol.back() >> lnj) != (ij >> lnj))
+                    fcol.resize((fcol.size() + kFFCols - 1) / kFFCols * kFFCols, -1);
+                if (fcol.size() % kFFCols == 0) span.emplace_back(u, u + 1);
+                fcol.push_back(ij);
             }
-            e = e1;
+            span.back().first = std::min(span.back().first, u);
+            span.back().second = std::max(span.back().second, u + 1);
+        }
+        fcol.resize((fcol.size() + kFFCols - 1) / kFFCols * kFFCols, -1);
+        // a piece is short where there are few of them (parallelism) and long
+        // where there are many (fewer T for stage 2): see kFFPieces
+        long long chunks = 0;
+        for (const auto& w : span) chunks += w.second - w.first;
+        const int most = (int)std::min<long long>(32, std::max<long long>(1, chunks / kFFPieces));
+        for (size_t g = 0; g < span.size(); ++g) {
+            const int lo = span[g].first, len = span[g].second - lo, np = (len + most - 1) / most;
+            for (int q = 0; q < np; ++q)
+                fpiece.push_back(make_int2((int)g, (lo + len * q / np) | (lo + len * (q + 1) / np) << 16));
         }
     }
+    const int npiece = (int)fpiece.size();
+    while (fpiece.size() % kFFWaves) fpiece.push_back(make_int2(0, 0));
     HIPCHECK(hipStreamSynchronize(c->stream));
     if (c->mv) hipFree(c->mv);
     if (c->cells) hipFree(c->cells);
+    if (c->ffcol) hipFree(c->ffcol);
+    if (c->ffpiece) hipFree(c->ffpiece);
     if (c->ffseg) hipFree(c->ffseg);
     c->mv = nullptr;
     c->cells = nullptr;
+    c->ffcol = nullptr;
+    c->ffpiece = nullptr;
     c->ffseg = nullptr;
-    c->nseg = 0;
+    c->nffpiece = c->nseg = 0;
     int rc = dev_alloc(&c->mv, (size_t)nmat);
     if (!rc) rc = dev_alloc(&c->cells, cells.size());
-    if (!rc) rc = dev_alloc(&c->ffseg, segs.size());
+    if (!rc) rc = dev_alloc(&c->ffcol, fcol.size());
+    if (!rc) rc = dev_alloc(&c->ffpiece, fpiece.size());
     if (rc) return rc;
     c->nmat = nmat;
     c->mat_count.assign(nmat, 0);
@@ -1136,8 +1170,9 @@ int ddafft_set_target(ddafft_ctx* c, const signed char* occ, int nmat, const int
     if ((rc = upload(c, c->dipf, c->dipf_h.data(), (size_t)n))) return rc;
     if ((rc = upload(c, c->mv, mv, (size_t)nmat * sizeof(int)))) return rc;
     if ((rc = upload(c, c->cells, cells.data(), cells.size() * sizeof(int)))) return rc;
-    if ((rc = upload(c, c->ffseg, segs.data(), segs.size() * sizeof(int2)))) return rc;
-    c->nseg = (int)segs.size();
+    if ((rc = upload(c, c->ffcol, fcol.data(), fcol.size() * sizeof(int)))) return rc;
+    if ((rc = upload(c, c->ffpiece, fpiece.data(), fpiece.size() * sizeof(int2)))) return rc;
+    c->nffpiece = npiece;
     HIPCHECK(hipStreamSynchronize(c->stream));
     c->have_target = true;
     return DDAFFT_OK;
@@ -1199,11 +1234,11 @@ namespace {
 // A set of ng * S directions whose z components repeat with period ng
 // (directions d and d + ng share z bit for bit) splits into ng groups of S
 // (group g: g, g + ng, ..., g + (S - 1) ng).  Returns ng of the smallest
-// such period with 2 <= S <= kFFDirs (S in *S), else 0.
-int dir_groups(const float* dirs, int ndirs, int* S) {
-    *S = 0;
-    if (!dirs || ndirs < 2) return 0;
-    for (int ng = std::max(1, (ndirs + kFFDirs - 1) / kFFDirs); ng <= ndirs / 2; ++ng) {
+// such period with S <= most (S in *S; ndirs groups of one if none).
+int dir_groups(const float* dirs, int ndirs, int most, int* S) {
+    *S = 1;
+    if (!dirs || ndirs < 2) return std::max(ndirs, 0);
+    for (int ng = std::max(1, (ndirs + most - 1) / most); ng <= ndirs / 2; ++ng) {
         if (ndirs % ng) continue;
         bool ok = true;
         for (int dd = ng; dd < ndirs && ok; ++dd)
@@ -1213,7 +1248,7 @@ int dir_groups(const float* dirs, int ndirs, int* S) {
             return ng;
         }
     }
-    return 0;
+    return ndirs;
 }
 
 }  // namespace
@@ -1230,7 +1265,8 @@ int ddafft_set_directions(ddafft_ctx* c, int ndirs, const float* dirs) {
         c->dirs_cap = ndirs;
     }
     c->ndirs = ndirs;
-    c->ffg_n = dir_groups(dirs, ndirs, &c->ffg_S);
+    c->ffg_n = dir_groups(dirs, ndirs, kFFMembers, &c->ffg_S);
+    c->ffs_n = dir_groups(dirs, ndirs, kFFDirs, &c->ffs_S);
     if (ndirs) {
         HIPCHECK(hipMemcpy(c->dirs, dirs, (size_t)ndirs * 3 * sizeof(float), hipMemcpyHostToDevice));
     }
@@ -1407,7 +1443,10 @@ int iteration(Seq& q, int solver, int o, float tau, int part = 0) {
 // after the stream (or an event after the copies) has completed.
 struct Fin {
     int nrhs = 0, ndirs = 0, cb = 0, fchunk = 0, max_step = 0;
-    bool state = false, hist = false, grouped = false;
+    bool state = false, hist = false;
+    bool cols = false;   // far field by columns
+    bool grouped = false;   // by the S11 gradients' groups
+    int sets = 1;        // its phase tables at a time
     size_t o_st = 0, o_hist = 0, o_part = 0, o_esc = 0, total = 0;
 };
 
@@ -1424,23 +1463,45 @@ bool ff_mfma_on(const ddafft_ctx* c) {
     return mode == 1 && !c->sum_mode && c->d.ni + c->d.nj + c->d.nl <= 384;
 }
 
-// The far field by groups of directions sharing z (k_far_field_grp): when a
-// set of ndirs directions splits into ng groups of S = 2..16 (dir_groups)
-// and the lattice's phase rows fit the kernel's LDS (n_i + n_j <= 512,
-// n_l <= 256).
-bool ff_group_ok(const ddafft_ctx* c, int ndirs, int ng, int S) {
+// The far field by columns (k_far_field_cols), the default in the FP64-summed
+// mode for every lattice and direction set: ng groups of S directions sharing
+// z (dir_groups; one group per direction where none do).  Measured against
+// the forms kept behind ddafft_set_tuning on the sets and lattices in its
+// comment; it was ahead on all of them.
+bool ff_cols_on(const ddafft_ctx* c, int ndirs, int ng, int S) {
     const int mode = c->ff_group >= 0 ? c->ff_group : 1;
-    return mode == 1 && !c->sum_mode && !ff_mfma_on(c) && ndirs > 0 && ng > 0 && S >= 2 && S <= kFFDirs &&
-           ng * S == ndirs && c->nseg > 0 && c->d.ni + c->d.nj <= 512 && c->d.nl <= 256;
-}
-// ... for the resident set
-bool ff_group_on(const ddafft_ctx* c, int ndirs) {
-    return !c->ffg_off_call && ndirs == c->ndirs && ff_group_ok(c, ndirs, c->ffg_n, c->ffg_S);
+    return mode == 1 && !c->sum_mode && !c->ff_s11 && !ff_mfma_on(c) && ndirs > 0 && ng * S == ndirs &&
+           c->nffpiece > 0;
 }
 
-void obs_blocks(const ddafft_ctx* c, int ndirs, bool grouped, int* cb, int* fchunk) {
+// The S11 gradients' far field by groups (k_far_field_grp): where the set
+// splits and the lattice's phase rows fit the kernel's LDS (n_i + n_j <= 512,
+// n_l <= 256).
+bool ff_group_on(const ddafft_ctx* c, int ndirs) {
+    return c->ff_s11 && c->ff_group != 0 && !c->sum_mode && !ff_mfma_on(c) && ndirs > 0 && c->ffs_S >= 2 &&
+           c->ffs_n * c->ffs_S == ndirs && c->nseg > 0 && c->d.ni + c->d.nj <= 512 && c->d.nl <= 256;
+}
+
+// Chunks of the pieces: enough blocks of nrhs right-hand sides and ng / 16
+// group tiles for four per CU, at most one per four pieces and 256 (the
+// partial sums grow with them: at most 64 beyond 4096 directions); a multiple
+// of the XCDs from 8 up, so that an XCD's blocks share columns.
+int ff_col_chunks(const ddafft_ctx* c, int ndirs, int ng, int nrhs) {
+    const int tiles = (ng + kFFGroups - 1) / kFFGroups * std::max(nrhs, 1);
+    int n = std::min({std::max(64, std::min(256, (1 << 18) / std::max(ndirs, 1))),
+                      (c->nffpiece + kFFWaves - 1) / kFFWaves, (1024 + tiles - 1) / tiles});
+    if (n > kXcds) n -= n % kXcds;
+    if (c->ff_chunk_max > 0) n = std::min(n, c->ff_chunk_max);
+    return std::max(n, 1);
+}
+
+void obs_blocks(const ddafft_ctx* c, int nrhs, int ndirs, int ng, int S, int* cb, int* fchunk) {
     *cb = c->sum_mode ? 1 : (int)std::min<long long>((c->d.n + kBlock - 1) / kBlock, 512);
-    if (grouped) {   // one chunk per 256 segments, at most 64
+    if (ff_cols_on(c, ndirs, ng, S)) {
+        *fchunk = ff_col_chunks(c, ndirs, ng, nrhs);
+        return;
+    }
+    if (ff_group_on(c, ndirs)) {   // one chunk per 256 segments, at most 64
         *fchunk = (int)std::max(1, std::min(64, (c->nseg + kBlock - 1) / kBlock));
         return;
     }
@@ -1455,15 +1516,16 @@ void obs_blocks(const ddafft_ctx* c, int ndirs, bool grouped, int* cb, int* fchu
 
 // Sizes the downloads and reserves the pinned buffer (before anything of this
 // solve is queued to it).
-int fin_layout(ddafft_ctx* c, int nrhs, bool state, bool hist, int max_step, int ndirs, Fin& f) {
+int fin_layout(ddafft_ctx* c, int nrhs, bool state, bool hist, int max_step, int ndirs, long long dir_stride, Fin& f) {
     f = Fin{};
     f.nrhs = nrhs;
     f.ndirs = ndirs;
     f.state = state;
     f.hist = state && hist;
     f.max_step = max_step;
+    f.cols = ff_cols_on(c, ndirs, c->ffg_n, c->ffg_S);
     f.grouped = ff_group_on(c, ndirs);
-    obs_blocks(c, ndirs, f.grouped, &f.cb, &f.fchunk);
+    obs_blocks(c, nrhs, ndirs, c->ffg_n, c->ffg_S, &f.cb, &f.fchunk);
     size_t off = 0;
     auto take = [&](size_t b) {
         const size_t o = off;
@@ -1492,7 +1554,12 @@ int fin_layout(ddafft_ctx* c, int nrhs, bool state, bool hist, int max_step, int
         TRY(dev_alloc(&c->ffpc, (size_t)c->ncells * 6));
         c->ffpc_cap = (size_t)c->ncells * 6;
     }
-    const size_t ntab = (size_t)ndirs * (c->d.ni + c->d.nj + c->d.nl);
+    // phase tables: one, or as many of the per-right-hand-side sets at once as 64 MB hold
+    size_t ntab = (size_t)ndirs * (c->d.ni + c->d.nj + c->d.nl);
+    if (f.cols && dir_stride != 0) {
+        f.sets = (int)std::max<size_t>(1, std::min<size_t>(nrhs, ((size_t)64 << 20) / (ntab * sizeof(float2))));
+        ntab *= f.sets;
+    }
     if (ndirs > 0 && ntab > c->fftab_cap) {
         HIPCHECK(hipStreamSynchronize(c->stream));
         if (c->fftab) hipFree(c->fftab);
@@ -1510,12 +1577,36 @@ int fin_layout(ddafft_ctx* c, int nrhs, bool state, bool hist, int max_step, int
 // their results into the pinned buffer.
 int obs_enqueue_seq(ddafft_ctx* c, const Fin& f, const float* ddirs, long long dir_stride);
 
+// The far field by columns of the field P (zero off the dipoles): the phase
+// tables, then every right-hand side that they serve in one launch.
+int ff_cols_enqueue(ddafft_ctx* c, const Fin& f, const float* ddirs, long long dir_stride, const float2* P) {
+    Dims d = c->d;
+    const int S = c->ffg_S, ng = c->ffg_n, ndirs = f.ndirs;
+    const int ngt = (ng + kFFGroups - 1) / kFFGroups;
+    const long long per = (long long)ndirs * (d.ni + d.nj + d.nl);
+    if (!c->ffcol || !c->ffpiece || S < 1 || S > kFFMembers || (size_t)(per * f.sets) > c->fftab_cap)
+        return fail(DDAFFT_ESTATE, "internal: far-field columns or phase tables missing");
+    const Geometry g = make_geometry(c, nullptr);
+    const int step = dir_stride ? f.sets : f.nrhs;
+    for (int r0 = 0; r0 < f.nrhs; r0 += step) {
+        const int nr = std::min(step, f.nrhs - r0);
+        const dim3 gt((int)std::min<long long>((per + kBlock - 1) / kBlock, 1024), dir_stride ? nr : 1);
+        hipLaunchKernelGGL(k_ff_table, gt, kBlock, 0, c->stream, d, g, ddirs + r0 * dir_stride, dir_stride, ng, S,
+                           c->fftab);
+        HIPCHECK(hipGetLastError());
+        hipLaunchKernelGGL(k_far_field_cols, dim3(f.fchunk * ngt, nr), kBlock, 0, c->stream, d, c->fftab,
+                           dir_stride ? 1 : nr, c->ffcol, c->ffpiece, c->nffpiece, ng, S, f.fchunk, r0, P, c->partials);
+        HIPCHECK(hipGetLastError());
+    }
+    return DDAFFT_OK;
+}
+
 // The grouped far field of right-hand sides r0 .. r0 + R - 1 (R = 1, 2):
 // their dipole moments gathered in list order, then k_far_field_grp with as
 // many groups per block as fit 16 directions and 24 T values per thread.
 int ff_grouped_enqueue(ddafft_ctx* c, const Fin& f, int r0, int R, int ndirs) {
     Dims d = c->d;
-    const int S = c->ffg_S, ng = c->ffg_n;
+    const int S = c->ffs_S, ng = c->ffs_n;
     if (!c->ffpc || !c->ffseg || (size_t)c->ncells * 3 * R > c->ffpc_cap)
         return fail(DDAFFT_ESTATE, "internal: grouped far-field buffers not allocated");
     const int gb = std::min((c->ncells + kBlock - 1) / kBlock, 2048);
@@ -1552,7 +1643,9 @@ int ff_grouped_enqueue(ddafft_ctx* c, const Fin& f, int r0, int R, int ndirs) {
     return DDAFFT_OK;
 }
 
-int obs_enqueue(ddafft_ctx* c, const Fin& f, const float* ddirs, long long dir_stride) {
+// P: the field whose far field is summed (c->P, or a copy of it that is zero
+// off the dipoles where c->P need not be).
+int obs_enqueue(ddafft_ctx* c, const Fin& f, const float* ddirs, long long dir_stride, const float2* P) {
     if (c->sum_mode) return obs_enqueue_seq(c, f, ddirs, dir_stride);
     const int nrhs = f.nrhs, ndirs = f.ndirs;
     Dims d = c->d;
@@ -1573,7 +1666,8 @@ int obs_enqueue(ddafft_ctx* c, const Fin& f, const float* ddirs, long long dir_s
             return fail(DDAFFT_ESTATE, "internal: far-field phase table not allocated");
         const int ntab = ndirs * (d.ni + d.nj + d.nl);
         const float* tab_dirs = nullptr;
-        for (int r0 = 0; r0 < nrhs;) {
+        if (f.cols) TRY(ff_cols_enqueue(c, f, ddirs, dir_stride, P));
+        for (int r0 = 0; !f.cols && r0 < nrhs;) {
             const bool pair = r0 + 1 < nrhs && (dir_stride == 0 || c->dir_pairs[r0 / 2]);
             dim3 gf(f.fchunk, (ndirs + kFD - 1) / kFD);
             const float* dd = ddirs + r0 * dir_stride;
@@ -1614,8 +1708,8 @@ int obs_enqueue(ddafft_ctx* c, const Fin& f, const float* ddirs, long long dir_s
             HIPCHECK(hipGetLastError());
             r0 += pair ? 2 : 1;
         }
-        // one thread per (right-hand side, direction), in blocks of 64 to spread over the CUs
-        hipLaunchKernelGGL(k_far_field_sum, (nrhs * ndirs + 63) / 64, 64, 0, c->stream, c->partials,
+        hipLaunchKernelGGL(k_far_field_sum, (nrhs * ndirs + kFFSumDirs - 1) / kFFSumDirs,
+                           6 * kFFSumDirs * kFFSumParts, 0, c->stream, c->partials,
                            f.fchunk, ndirs, nrhs, ddirs, dir_stride, reinterpret_cast<float2*>(c->dn_dev + f.o_esc));
         HIPCHECK(hipGetLastError());
     }
@@ -1697,10 +1791,10 @@ void obs_complete(ddafft_ctx* c, const Fin& f, const float* einc, float* esc, fl
 
 // Standalone cross sections / far fields (one synchronization).
 int observables(ddafft_ctx* c, int nrhs, const float* einc, int ndirs, const float* ddirs, long long dir_stride,
-                float* esc, float* cabs, float* cext) {
+                float* esc, float* cabs, float* cext, const float2* P) {
     Fin f;
-    TRY(fin_layout(c, nrhs, false, false, 0, ndirs, f));
-    TRY(obs_enqueue(c, f, ddirs, dir_stride));
+    TRY(fin_layout(c, nrhs, false, false, 0, ndirs, dir_stride, f));
+    TRY(obs_enqueue(c, f, ddirs, dir_stride, P));
     HIPCHECK(hipStreamSynchronize(c->stream));
     obs_complete(c, f, einc, esc, cabs, cext);
     return DDAFFT_OK;
@@ -1948,7 +2042,7 @@ int fin_state_complete(Run& r, const Fin& f, double* err_hist, int* info, std::v
 
 int run_finish(Run& r, double* err_hist, int* info, std::vector<SolveState>& sf) {
     Fin f;
-    TRY(fin_layout(r.c, r.nrhs, true, err_hist != nullptr, r.max_step, 0, f));
+    TRY(fin_layout(r.c, r.nrhs, true, err_hist != nullptr, r.max_step, 0, 0, f));
     TRY(fin_state_enqueue(r, f));
     HIPCHECK(hipStreamSynchronize(r.c->stream));
     return fin_state_complete(r, f, err_hist, info, sf);
@@ -2005,7 +2099,9 @@ int job_prepare(ddafft_ctx* c, const ddafft_job* j, int solver, int max_step, co
             }
             TRY(upload(c, c->dirs, j->dirs, per * sets * sizeof(float)));
             c->ndirs = j->dirs_per_rhs ? 0 : ndirs;   // per-RHS sets are not resident for later calls
-            c->ffg_n = j->dirs_per_rhs ? 0 : dir_groups(j->dirs, ndirs, &c->ffg_S);
+            const float* gd = j->dirs_per_rhs ? nullptr : j->dirs;   // rotated sets: no groups
+            c->ffg_n = dir_groups(gd, ndirs, kFFMembers, &c->ffg_S);
+            c->ffs_n = dir_groups(gd, ndirs, kFFDirs, &c->ffs_S);
             if (j->dirs_per_rhs) {
                 *dir_stride = (long long)per;
                 c->dir_pairs.assign((size_t)(nrhs + 1) / 2, 0);
@@ -2046,9 +2142,9 @@ int ddafft_solve_ex(ddafft_ctx* c, const ddafft_job* job, int solver, float tau,
     TRY(run_begin(r));
     while (run_more(r)) TRY(run_step(r));
     Fin f;
-    TRY(fin_layout(c, job->nrhs, true, err_hist != nullptr, max_step, job->ndirs, f));
+    TRY(fin_layout(c, job->nrhs, true, err_hist != nullptr, max_step, job->ndirs, stride, f));
     TRY(fin_state_enqueue(r, f));
-    TRY(obs_enqueue(c, f, ddirs, stride));
+    TRY(obs_enqueue(c, f, ddirs, stride, c->P));
     HIPCHECK(hipStreamSynchronize(c->stream));
     if (t_noalloc)   // the results sit in the device scratch: one copy to the context's host buffer
         HIPCHECK(hipMemcpy(c->dn, c->dn_dev, f.total, hipMemcpyDeviceToHost));
@@ -2093,34 +2189,29 @@ int ddafft_solve_noalloc(ddafft_ctx* c, int nrhs, int solver, float tau, int max
     if (c->prof) return fail(DDAFFT_ESTATE, "profiling records events: disable it for the allocation-free solve");
     const Dims& d = c->d;
     // this call's pieces of the scratch
-    // the far field's form, as the solve will choose it for these directions;
-    // the grouped form needs the dipole moments gathered in the scratch
-    bool grouped = false;
-    {
-        int S = c->ffg_S;
-        const int ng = dirs ? dir_groups(dirs, ndirs, &S) : c->ffg_n;
-        grouped = ff_group_ok(c, ndirs, ng, S);
-    }
+    // the direction groups as the solve will find them
+    int ffS = c->ffg_S;
+    const int ffn = dirs ? dir_groups(dirs, ndirs, kFFMembers, &ffS) : c->ffg_n;
     int cb = 0, fchunk = 0;
-    size_t off = 0, res = 0, n_part = 0, n_hist = 0, n_esc = 0, n_tab = 0, n_dirs = 0, n_pc = 0;
-    size_t o_part = 0, o_hist = 0, o_esc = 0, o_tab = 0, o_dirs = 0, o_res = 0, o_pc = 0;
+    size_t off = 0, res = 0, n_part = 0, n_hist = 0, n_esc = 0, n_tab = 0, n_dirs = 0;
+    size_t o_part = 0, o_hist = 0, o_esc = 0, o_tab = 0, o_dirs = 0, o_res = 0;
     auto take = [&](size_t b) {
         const size_t o = off;
         off += (b + 255) & ~(size_t)255;
         return o;
     };
-    // the plan of the scratch; the grouped far field only where its pieces fit
+    // the plan of the scratch; the far field's columns in fewer chunks where its partial sums do not fit
+    c->ff_chunk_max = 0;
     for (;;) {
         off = 0;
         res = 0;   // results, laid out as fin_layout lays them out
-        obs_blocks(c, ndirs, grouped, &cb, &fchunk);
+        obs_blocks(c, nrhs, ndirs, ffn, ffS, &cb, &fchunk);
         n_part = std::max({(size_t)nrhs * std::max(zi_blocks(d), update_blocks(d)) * kSlots, (size_t)nrhs * cb * 2,
                            (size_t)nrhs * fchunk * std::max(ndirs, 1) * 6});
         n_hist = (size_t)c->nrhs_max * (max_step + 1);
         n_esc = (size_t)nrhs * ndirs * 3;
         n_tab = (size_t)ndirs * (d.ni + d.nj + d.nl);
         n_dirs = dirs ? (size_t)ndirs * 3 : 0;
-        n_pc = grouped ? (size_t)c->ncells * 6 : 0;
         {
             auto t = [&](size_t b) { res += (b + 255) & ~(size_t)255; };
             t((size_t)nrhs * sizeof(SolveState));
@@ -2134,10 +2225,13 @@ int ddafft_solve_noalloc(ddafft_ctx* c, int nrhs, int solver, float tau, int max
         o_tab = take(n_tab * sizeof(float2));
         o_dirs = take(n_dirs * sizeof(float));
         o_res = take(res);
-        o_pc = take(n_pc * sizeof(float2));
-        if (!grouped || off <= kScratchBytes) break;
-        grouped = false;
+        if (off <= kScratchBytes || fchunk <= 1 || !ff_cols_on(c, ndirs, ffn, ffS)) break;
+        c->ff_chunk_max = fchunk / 2;
     }
+    struct Unlimit {   // the cap holds for this call only
+        ddafft_ctx* c;
+        ~Unlimit() { c->ff_chunk_max = 0; }
+    } unlimit{c};
     size_t o_seq = 0, n_seq = 0;
     if (c->sum_mode) {   // the sequential-sum terms get the rest
         o_seq = take(0);
@@ -2158,11 +2252,10 @@ int ddafft_solve_noalloc(ddafft_ctx* c, int nrhs, int solver, float tau, int max
         float2* esc; int esc_cap;
         float2* fftab; size_t fftab_cap;
         float* dirs; int dirs_cap, ndirs, ffg_n, ffg_S;
-        float2* ffpc; size_t ffpc_cap;
         float* seqbuf; size_t seqbuf_cap;
         char *dn, *dn_dev; size_t dn_cap;
     } sv{c->partials, c->partials_cap, c->hist, c->hist_cap, c->esc, c->esc_cap, c->fftab, c->fftab_cap, c->dirs,
-         c->dirs_cap, c->ndirs, c->ffg_n, c->ffg_S, c->ffpc, c->ffpc_cap, c->seqbuf, c->seqbuf_cap, c->dn, c->dn_dev,
+         c->dirs_cap, c->ndirs, c->ffg_n, c->ffg_S, c->seqbuf, c->seqbuf_cap, c->dn, c->dn_dev,
          c->dn_cap};
     HIPCHECK(hipStreamSynchronize(c->stream));   // nothing of an earlier call still uses the old buffers
     char* sc = c->scratch;
@@ -2178,11 +2271,6 @@ int ddafft_solve_noalloc(ddafft_ctx* c, int nrhs, int solver, float tau, int max
         c->dirs = reinterpret_cast<float*>(sc + o_dirs);
         c->dirs_cap = ndirs;
     }
-    if (grouped) {
-        c->ffpc = reinterpret_cast<float2*>(sc + o_pc);
-        c->ffpc_cap = n_pc;
-    }
-    c->ffg_off_call = !grouped;   // the solve's own choice then agrees with this plan
     if (c->sum_mode) {
         c->seqbuf = reinterpret_cast<float*>(sc + o_seq);
         c->seqbuf_cap = n_seq;
@@ -2194,7 +2282,6 @@ int ddafft_solve_noalloc(ddafft_ctx* c, int nrhs, int solver, float tau, int max
     const int rc = ddafft_solve(c, nrhs, solver, tau, max_step, err_max, alpha, kinc, einc, ndirs, dirs, esc, cabs,
                                 cext, err_hist, info);
     t_noalloc = false;
-    c->ffg_off_call = false;
     if (rc) hipStreamSynchronize(c->stream);   // a failed call may have left work queued on the scratch
     c->partials = sv.partials;
     c->partials_cap = sv.partials_cap;
@@ -2209,8 +2296,6 @@ int ddafft_solve_noalloc(ddafft_ctx* c, int nrhs, int solver, float tau, int max
     c->ndirs = sv.ndirs;
     c->ffg_n = sv.ffg_n;
     c->ffg_S = sv.ffg_S;
-    c->ffpc = sv.ffpc;
-    c->ffpc_cap = sv.ffpc_cap;
     c->seqbuf = sv.seqbuf;
     c->seqbuf_cap = sv.seqbuf_cap;
     c->dn = sv.dn;
@@ -2294,9 +2379,9 @@ int ddafft_solve_batch(int n, ddafft_ctx* const* ctxs, const ddafft_job* jobs, i
             if (s.finishing || run_more(s.r)) continue;
             progress = true;
             const ddafft_job& j = jobs[s.job];
-            TRY(fin_layout(s.r.c, j.nrhs, true, false, max_step, j.ndirs, s.f));
+            TRY(fin_layout(s.r.c, j.nrhs, true, false, max_step, j.ndirs, s.stride, s.f));
             TRY(fin_state_enqueue(s.r, s.f));
-            TRY(obs_enqueue(s.r.c, s.f, s.ddirs, s.stride));
+            TRY(obs_enqueue(s.r.c, s.f, s.ddirs, s.stride, s.r.c->P));
             HIPCHECK(hipEventRecord(s.r.c->fin_ev, s.r.c->stream));
             s.finishing = true;
         }
@@ -2339,6 +2424,34 @@ int ddafft_solve_batch(int n, ddafft_ctx* const* ctxs, const ddafft_job* jobs, i
 
 namespace {
 
+// The far-field segments of the target for S11 gradients: each run of dipoles
+// in one (i, j) column, cut into near-equal pieces of at most kFFSeg.
+int ff_segments(ddafft_ctx* c) {
+    if (c->nseg > 0) return DDAFFT_OK;
+    std::vector<int> ij;
+    ij.reserve((size_t)c->ncells);
+    const int lnl = __builtin_ctz(c->d.nl);
+    for (size_t k = 0; k < c->dipf_h.size(); ++k)
+        if (c->dipf_h[k]) ij.push_back((int)(k >> lnl));
+    std::vector<int2> segs;
+    for (size_t e = 0; e < ij.size();) {
+        size_t e1 = e + 1;
+        while (e1 < ij.size() && ij[e1] == ij[e]) ++e1;
+        const int len = (int)(e1 - e), np = (len + kFFSeg - 1) / kFFSeg;
+        for (int q = 0, at = 0; q < np; ++q) {
+            const int cnt = (len - at) / (np - q);
+            segs.push_back(make_int2((int)e + at, (ij[e] << 6) | cnt));
+            at += cnt;
+        }
+        e = e1;
+    }
+    TRY(dev_alloc(&c->ffseg, segs.size()));
+    HIPCHECK(hipMemcpyAsync(c->ffseg, segs.data(), segs.size() * sizeof(int2), hipMemcpyHostToDevice, c->stream));
+    HIPCHECK(hipStreamSynchronize(c->stream));
+    c->nseg = (int)segs.size();
+    return DDAFFT_OK;
+}
+
 template <class T>
 int ensure_buf(ddafft_ctx* c, T** p, size_t& cap, size_t count) {
     if (count <= cap && *p) return DDAFFT_OK;
@@ -2378,6 +2491,12 @@ int ddafft_gradient(ddafft_ctx* c, int npol, int nobj, int solver, float tau, in
     const long long n = d.n;
 
     // forward solve of the npol polarizations; its dipoles are kept
+    if (any_s11) TRY(ff_segments(c));
+    struct S11Call {   // its far field feeds the adjoint source
+        ddafft_ctx* c;
+        S11Call(ddafft_ctx* x, bool on) : c(x) { c->ff_s11 = on; }
+        ~S11Call() { c->ff_s11 = false; }
+    } s11_call{c, any_s11};
     std::vector<float> esc_h((size_t)npol * std::max(ndirs, 1) * 6), cabs_h(npol), cext_h(npol);
     std::vector<int> info_f(4 * npol);
     TRY(ddafft_solve(c, npol, solver, tau, max_step, err_max, alpha, kinc, einc, ndirs, dirs,
@@ -2536,7 +2655,7 @@ int ddafft_gradient(ddafft_ctx* c, int npol, int nobj, int solver, float tau, in
     TRY(run_begin(ra));
     while (run_more(ra)) TRY(run_step(ra));
     Fin fa;
-    TRY(fin_layout(c, nadj, true, false, max_step, 0, fa));
+    TRY(fin_layout(c, nadj, true, false, max_step, 0, 0, fa));
     TRY(fin_state_enqueue(ra, fa));
 
     // df/dalpha per dipole, the chi map, and the per-material sums
@@ -2610,7 +2729,7 @@ int ddafft_cabs_cext(ddafft_ctx* c, const float* alpha, const float* kinc, const
     TRY(upload(c, c->einc, einc, 3 * sizeof(float2)));
     TRY(upload_incidence(c, 1, kinc));
     TRY(field_in(c, p, c->P, c->Y));
-    return observables(c, 1, einc, 0, nullptr, 0, nullptr, cabs, cext);
+    return observables(c, 1, einc, 0, nullptr, 0, nullptr, cabs, cext, c->P);
 }
 
 int ddafft_far_field(ddafft_ctx* c, const float* p, int ndirs, const float* dirs, float* esc) {
@@ -2625,7 +2744,10 @@ int ddafft_far_field(ddafft_ctx* c, const float* p, int ndirs, const float* dirs
     const float e[6] = {1.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     TRY(upload(c, c->einc, e, sizeof(e)));
     TRY(upload_incidence(c, 1, kz));
-    return observables(c, 1, e, ndirs, c->dirs, 0, esc, nullptr, nullptr);
+    // the columns' sums run over every cell they span: a copy that is zero off the dipoles
+    hipLaunchKernelGGL(k_mask_field, update_blocks(c->d), kBlock, 0, c->stream, c->d, c->dipf, c->P, c->X);
+    HIPCHECK(hipGetLastError());
+    return observables(c, 1, e, ndirs, c->dirs, 0, esc, nullptr, nullptr, c->X);
 }
 
 int ddafft_profile(ddafft_ctx* c, int enable, double* pass_ms, long long* matvecs) {

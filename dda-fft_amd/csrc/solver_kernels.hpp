@@ -483,13 +483,250 @@ __global__ __launch_bounds__(kBlock) void k_far_field_mfma(Dims d, const float2*
     }
 }
 
-// Far field of a direction set made of groups that share their z component
-// (the scattering planes of a fixed orientation are rotations of one plane
-// about z, so every polar angle gives one group with one direction per
-// plane).  With X, Y, Z the per-axis phase factors,
+// Far field by columns, the default form.  With X, Y, Z the per-axis phase
+// factors of a direction,
 //   S(n) = sum_(i,j) X_n[i] Y_n[j] T_g(i,j),   T_g(i,j) = sum_l Z_g[l] P(i,j,l),
-// so the l-sums are formed once per group instead of once per direction.
-// Group g holds the directions g, g + ngroups, ..., g + (S - 1) ngroups.
+// and directions that share their z component bit for bit (a group; the
+// scattering planes of a fixed orientation are rotations about z, so every
+// polar angle is one group with one direction per plane) share T.  A set of
+// ng * S directions whose z repeats with period ng has ng groups of S members
+// (group g: g, g + ng, ...); any other set is ndirs groups of one.
+//
+// Stage 1, on the matrix cores: a wave forms T of 16 groups for one piece, 8
+// columns over a range of l.  One v_mfma_f32_16x16x4f32 takes 16 groups (rows)
+// x 4 l x 8 complex columns as 16 real ones (lane n < 8: real part of column
+// n, else the imaginary part of column n - 8):
+//   D += Re(Z) [Pr | Pi]  and  D += Im(Z) [-Pi | Pr]
+// (lane layout: A[l % 16][l / 16], B[l / 16][l % 16], D[4 (l / 16) + v][l % 16]).
+// Lane group k of a wave takes the four l's 16 u + 4 k + s, s = 0 .. 3, of a
+// 16-point chunk u in four such products.  The chunk's moments are loaded as
+// whole 128-byte lines and change lanes through LDS (loaded straight into the
+// operand's lanes, each quarter-wave would touch 8 lines).  P is zero off the
+// dipoles, so a piece is whole chunks of the range that its columns' dipoles
+// span.  The next chunk's loads are in flight during the products of this one.
+// Stage 2: the T of the block's four pieces go through LDS to one thread per
+// direction and share of the columns, which adds Y T over a piece (its columns
+// lie in one plane i), then X times that: FP32 over 8 columns, then FP64.
+//
+// The column sums cost 8 FP32 operations per (dipole, component, group) on the
+// matrix cores (2 x the VALU's rate without packed FP32), and the phases one
+// product per (piece, direction) instead of two per (dipole, direction).
+// Against the per-direction sums and the z-groups summed per 16-dipole segment
+// on the VALU (with their gather of the moments), MI355X, us per solve:
+//   256^3 sphere, 8 planes x 361 angles, 2 RHS   25088 -> 2962
+//   64^3 spheroid, 4 x 181, 2 RHS                   46 -> 32
+//   16x32x128 ellipsoid, 3 x 37, 2 RHS              22 -> 8
+//   128^3 sphere, 1 x 19, 2 RHS                     67 -> 38
+//   32x32x64 agglomerate, 8 sets of 19, 16 RHS     173 -> 21 (one launch)
+// At 256^3 the products alone are 1.1 ms of matrix-core time; the rest is the
+// VALU work of stage 2 and LDS and L1 accesses that the four waves of a SIMD
+// do not hide.  Error against 64-bit sums: no larger than before (FP64 from 8
+// columns up).
+// tab: [set][ni + nj + nl][S][ng] phases; cols: (i nj + j) of the columns that
+// hold dipoles, padded to 8 with -1; piece: {first column / 8, 16-point chunks
+// [lo, hi) as lo | hi << 16}, padded to 4 with {0, 0}.  Grid: x over chunks of
+// the pieces and tiles of 16 groups (neighbouring blocks of one XCD: the same
+// pieces, other groups, so that the moments come from its L2), y over
+// right-hand sides, set_rhs of which share a phase table.
+// partials: [rhs][nchunk][ndirs][6].
+// ---------------------------------------------------------------------------
+
+constexpr int kFFGroups = 16;   // groups per block (rows of the matrix product)
+constexpr int kFFMembers = 8;   // directions per group at most (16 x 8 of a block's 256 threads in stage 2)
+constexpr int kFFCols = 8;      // columns per piece
+constexpr int kFFWaves = kBlock / 64;
+
+// The lanes of one wave exchange data through LDS that no other wave touches:
+// LDS operations of a wave execute in order, so only the compiler has to keep it.
+#ifndef DDA_WAVE_SYNC   // the CPU emulation of the kernels (tests/emul) defines its own
+#define DDA_WAVE_SYNC()                                          \
+    do {                                                         \
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   \
+        __builtin_amdgcn_wave_barrier();                         \
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");   \
+    } while (0)
+#endif
+
+// tab[u][a][s][g] for set u's directions dirs + u * dir_stride
+__global__ __launch_bounds__(kBlock) void k_ff_table(Dims d, Geometry g, const float* __restrict__ dirs,
+                                                     long long dir_stride, int ng, int S, float2* __restrict__ tab) {
+    const int ndirs = ng * S, total = ndirs * (d.ni + d.nj + d.nl);
+    dirs += blockIdx.y * dir_stride;
+    tab += (long long)blockIdx.y * total;
+    for (int f = blockIdx.x * blockDim.x + threadIdx.x; f < total; f += gridDim.x * blockDim.x) {
+        const int a = f / ndirs, dd = f - a * ndirs;   // dd = s * ng + g: the direction's index
+        float arg;
+        if (a < d.ni)
+            arg = dirs[3 * dd] * ((float)a * g.d0 - g.cx);
+        else if (a < d.ni + d.nj)
+            arg = dirs[3 * dd + 1] * ((float)(a - d.ni) * g.d0 - g.cy);
+        else
+            arg = dirs[3 * dd + 2] * ((float)(a - d.ni - d.nj) * g.d0 - g.cz);
+        tab[f] = exp_i(arg);
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_far_field_cols(Dims d, const float2* __restrict__ tab, int set_rhs,
+                                                           const int* __restrict__ cols,
+                                                           const int2* __restrict__ piece, int npiece, int ng, int S,
+                                                           int nchunk, int rhs_first, const float2* __restrict__ P,
+                                                           double* __restrict__ partials) {
+    typedef DDA_FLOAT4_MFMA f4;
+    constexpr int NC = kFFWaves * kFFCols;    // columns of a batch: one piece per wave
+    constexpr int CS = 3 * kFFGroups + 17;    // T's column stride: a wave's 8 columns start in different banks
+    constexpr int LP = 17;                    // stride of a (component, column)'s 16 moments
+    __shared__ float2 sT[NC * CS];
+    __shared__ float2 sP[kFFWaves * 3 * kFFCols * LP];
+    __shared__ unsigned sy[NC], sx[kFFWaves];
+    const int ndirs = ng * S, ngt = (ng + kFFGroups - 1) / kFFGroups;
+    // (chunk, group tile) of this block
+    int chunk, gt;
+    if (nchunk % kXcds == 0) {
+        const int q = blockIdx.x / kXcds;
+        gt = q % ngt;
+        chunk = (q / ngt) * kXcds + blockIdx.x % kXcds;
+    } else {
+        gt = blockIdx.x % ngt;
+        chunk = blockIdx.x / ngt;
+    }
+    const int rhs = rhs_first + blockIdx.y, g0 = gt * kFFGroups;
+    tab += (long long)(blockIdx.y / set_rhs) * ndirs * (d.ni + d.nj + d.nl);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int m = lane & 15, k = lane >> 4, c = lane & 7;
+    const bool imag = (lane & 8) != 0;
+    // 32-bit offsets from uniform bases: a phase table holds less than 2^29
+    // entries, the three component planes of P 3 * 2^24 at most
+    const unsigned zo = (unsigned)(d.ni + d.nj) * ndirs + min(g0 + m, ng - 1), pn = (unsigned)d.n;
+    const float2* Pr = P + (long long)rhs * 3 * d.n;
+    float2* wp = sP + wave * 3 * kFFCols * LP;
+    // stage-2 role: (member s2, group q2), and a share of the columns: every
+    // subs-th of the batch's 4, 8 or 16 runs of 8, 4 or 2 columns
+    const int items = kFFGroups * S, subs = kBlock / items;
+    const int item = tid % items, sub = tid / items;
+    const int s2 = item / kFFGroups, q2 = item % kFFGroups;
+    const bool adds = sub < subs;
+    const unsigned xo = s2 * ng + min(g0 + q2, ng - 1);
+    const int lrun = subs >= 16 ? 1 : subs >= 8 ? 2 : 3;   // columns per run: 1 << lrun
+    const int lnj = __builtin_ctz(d.nj);
+    double dacc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    const int nbatch = (npiece + kFFWaves - 1) / kFFWaves;
+    const int lo = (int)((long long)nbatch * chunk / nchunk), hi = (int)((long long)nbatch * (chunk + 1) / nchunk);
+    for (int b = lo; b < hi; ++b) {
+        const int2 pe = piece[b * kFFWaves + wave];
+        const int u0 = pe.y & 0xffff, u1 = pe.y >> 16;
+        // lane (k, m) loads point m of the chunk for columns k and k + 4
+        const int ca = cols[pe.x * kFFCols + k], cb = cols[pe.x * kFFCols + k + 4];
+        const unsigned pa = (unsigned)max(ca, 0) * d.nl + m, pb = (unsigned)max(cb, 0) * d.nl + m;
+        float2 pv[6], zv[4];   // pv: component q / 2, columns k (even q) and k + 4
+        auto fetch = [&](int u) {
+            const bool in = 16 * u + m < d.nl;
+#pragma unroll
+            for (int q = 0; q < 6; ++q) {
+                pv[q] = make_float2(0.f, 0.f);
+                if (in && (q & 1 ? cb : ca) >= 0) pv[q] = Pr[(q & 1 ? pb : pa) + 16 * u + (q / 2) * pn];
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) zv[s] = tab[zo + (unsigned)min(16 * u + 4 * k + s, d.nl - 1) * ndirs];
+        };
+        f4 acc[3];
+#pragma unroll
+        for (int v = 0; v < 3; ++v) acc[v] = f4{0.f, 0.f, 0.f, 0.f};
+        if (u0 < u1) fetch(u0);
+        for (int u = u0; u < u1; ++u) {
+            float2 z[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) z[s] = zv[s];
+            DDA_WAVE_SYNC();   // the previous chunk's moments have been read
+#pragma unroll
+            for (int q = 0; q < 6; ++q) wp[((q / 2) * kFFCols + k + 4 * (q & 1)) * LP + m] = pv[q];
+            DDA_WAVE_SYNC();
+            if (u + 1 < u1) fetch(u + 1);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                float b2[3];
+#pragma unroll
+                for (int v = 0; v < 3; ++v) {
+                    const float2 p = wp[(v * kFFCols + c) * LP + 4 * k + s];
+                    acc[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(z[s].x, imag ? p.y : p.x, acc[v], 0, 0, 0);
+                    b2[v] = imag ? p.x : -p.y;
+                }
+#pragma unroll
+                for (int v = 0; v < 3; ++v) acc[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(z[s].y, b2[v], acc[v], 0, 0, 0);
+            }
+        }
+        // T[column][component][group], and the phase table's rows of the columns
+        float* t = reinterpret_cast<float*>(sT + (wave * kFFCols + c) * CS + 4 * k) + (imag ? 1 : 0);
+#pragma unroll
+        for (int v = 0; v < 3; ++v)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) t[(v * kFFGroups + e) * 2] = acc[v][e];
+        if (m == 0) {   // T is zero where there is no column
+            sy[wave * kFFCols + k] = (unsigned)(d.ni + (max(ca, 0) & (d.nj - 1))) * ndirs;
+            sy[wave * kFFCols + k + 4] = (unsigned)(d.ni + (max(cb, 0) & (d.nj - 1))) * ndirs;
+            if (k == 0) sx[wave] = (unsigned)(max(ca, 0) >> lnj) * ndirs;
+        }
+        __syncthreads();
+        if (adds)
+            for (int run = sub; run < NC >> lrun; run += subs) {
+                const int e0 = run << lrun;
+                const float2 x = tab[xo + sx[e0 / kFFCols]];
+                float2 sum[3];
+#pragma unroll
+                for (int v = 0; v < 3; ++v) sum[v] = make_float2(0.f, 0.f);
+#pragma unroll 2
+                for (int e = e0; e < e0 + (1 << lrun); e += 2) {
+                    const float2 y0 = tab[xo + sy[e]], y1 = tab[xo + sy[e + 1]];
+                    const float2* te = sT + e * CS + q2;
+#pragma unroll
+                    for (int v = 0; v < 3; ++v) {
+                        cmac_fma(sum[v], y0, te[v * kFFGroups]);
+                        cmac_fma(sum[v], y1, te[CS + v * kFFGroups]);
+                    }
+                }
+#pragma unroll
+                for (int v = 0; v < 3; ++v) {
+                    const float2 w = cmul_fma(x, sum[v]);
+                    dacc[2 * v] += (double)w.x;
+                    dacc[2 * v + 1] += (double)w.y;
+                }
+            }
+        __syncthreads();   // sT, sy and sx are refilled by the next batch
+    }
+    // the subsets' sums, in a fixed order: [sub][6][item]
+    double* red = reinterpret_cast<double*>(sT);
+    static_assert(6 * kBlock * sizeof(double) <= sizeof(sT), "the FP64 sums fit T's rows");
+    if (adds)
+#pragma unroll
+        for (int e = 0; e < 6; ++e) red[(sub * 6 + e) * items + item] = dacc[e];
+    __syncthreads();
+    if (tid < items && g0 + q2 < ng) {
+        double* out = partials + (((long long)rhs * nchunk + chunk) * ndirs + s2 * ng + g0 + q2) * 6;
+#pragma unroll
+        for (int e = 0; e < 6; ++e) {
+            double v = 0.0;
+            for (int u = 0; u < subs; ++u) v += red[(u * 6 + e) * items + item];
+            out[e] = v;
+        }
+    }
+}
+
+// P on the dipole cells and zero elsewhere (a field from outside the solver).
+__global__ __launch_bounds__(kBlock) void k_mask_field(Dims d, const int8_t* __restrict__ dipf,
+                                                       const float2* __restrict__ P, float2* __restrict__ out) {
+    for (long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x; k < d.n; k += (long long)gridDim.x * blockDim.x) {
+        const bool dip = dipf[k] != 0;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) out[q * d.n + k] = dip ? P[q * d.n + k] : make_float2(0.f, 0.f);
+    }
+}
+
+// The far field that an adjoint source is built from (gradients of S11), for
+// direction sets of groups that share z: BiCGStab multiplies the last bits of
+// its source by up to 1e4 within a few steps near a breakdown, so those calls
+// keep these float sums, whose bits their gradients have had, rather than the
+// faster column form's (which is as exact, but rounds otherwise).  The l-sums
+// are formed once per group, as there; group g holds the directions g,
+// g + ngroups, ..., g + (S - 1) ngroups.
 // The dipole list is cut into segments of at most kFFSeg consecutive dipoles
 // of one (i, j) column (seg: {first dipole, (i nj + j) << 6 | count}).
 // Stage 1: one thread per segment sums its T for the block's G groups, from
@@ -635,38 +872,50 @@ __global__ __launch_bounds__(kBlock) void k_far_field_grp(Dims d, const float2* 
 // Sums the chunks and applies the transverse projection:
 // out[nrhs][ndirs][3] complex float.  Right-hand side r uses the directions
 // dirs + r * dir_stride (dir_stride 0: one set shared by all).
-__global__ __launch_bounds__(kBlock) void k_far_field_sum(const double* __restrict__ partials, int nchunk, int ndirs,
-                                                          int nrhs, const float* __restrict__ dirs,
-                                                          long long dir_stride, float2* __restrict__ out) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= nrhs * ndirs) return;
-    const int dd = idx % ndirs, rhs = idx / ndirs;
-    double s[6] = {0, 0, 0, 0, 0, 0};
-    const double* p0 = partials + ((long long)rhs * nchunk * ndirs + dd) * 6;
-    const long long cs = (long long)ndirs * 6;   // chunk stride
-    // chunks in order, the loads of four in flight together
-    int c = 0;
-    for (; c + 4 <= nchunk; c += 4) {
-        double t[4][6];
+// Four threads add each of the six values of a (right-hand side, direction),
+// a quarter of the chunks each, so that a chunk's loads are contiguous over
+// the block's 8 directions and the chain of loads is short.
+constexpr int kFFSumDirs = 8, kFFSumParts = 4;
+__global__ __launch_bounds__(6 * kFFSumDirs * kFFSumParts) void k_far_field_sum(
+    const double* __restrict__ partials, int nchunk, int ndirs, int nrhs, const float* __restrict__ dirs,
+    long long dir_stride, float2* __restrict__ out) {
+    constexpr int NT = 6 * kFFSumDirs;
+    __shared__ double sv[kFFSumParts * NT];
+    const int t = threadIdx.x % NT, part = threadIdx.x / NT, e = t % 6;
+    const int idx = blockIdx.x * kFFSumDirs + t / 6;
+    const bool on = idx < nrhs * ndirs;
+    const int rhs = on ? idx / ndirs : 0, dd = on ? idx - rhs * ndirs : 0;
+    double s = 0.0;
+    if (on) {
+        const double* p = partials + ((long long)rhs * nchunk * ndirs + dd) * 6 + e;
+        const long long cs = (long long)ndirs * 6;   // chunk stride
+        const int c1 = nchunk * (part + 1) / kFFSumParts;
+        // chunks in order, the loads of eight in flight together
+        int c = nchunk * part / kFFSumParts;
+        for (; c + 8 <= c1; c += 8) {
+            double v[8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+            for (int u = 0; u < 8; ++u) v[u] = p[(c + u) * cs];
 #pragma unroll
-            for (int e = 0; e < 6; ++e) t[u][e] = p0[(c + u) * cs + e];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int e = 0; e < 6; ++e) s[e] += t[u][e];
+            for (int u = 0; u < 8; ++u) s += v[u];
+        }
+        for (; c < c1; ++c) s += p[c * cs];
     }
-    for (; c < nchunk; ++c)
+    sv[part * NT + t] = s;
+    __syncthreads();
+    if (threadIdx.x < NT) {
 #pragma unroll
-        for (int e = 0; e < 6; ++e) s[e] += p0[c * cs + e];
+        for (int u = 1; u < kFFSumParts; ++u) s += sv[u * NT + t];
+        sv[t] = s;
+    }
+    __syncthreads();
+    if (!on || part > 0 || e >= 3) return;
+    const double* v = sv + (t - e);
     const float* dv = dirs + rhs * dir_stride + 3 * dd;
     const double n[3] = {dv[0], dv[1], dv[2]};
-    const double dr = n[0] * s[0] + n[1] * s[2] + n[2] * s[4];
-    const double di = n[0] * s[1] + n[1] * s[3] + n[2] * s[5];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-        out[(long long)idx * 3 + c] = make_float2((float)(s[2 * c] - n[c] * dr), (float)(s[2 * c + 1] - n[c] * di));
+    const double dr = n[0] * v[0] + n[1] * v[2] + n[2] * v[4];
+    const double di = n[0] * v[1] + n[1] * v[3] + n[2] * v[5];
+    out[(long long)idx * 3 + e] = make_float2((float)(v[2 * e] - n[e] * dr), (float)(v[2 * e + 1] - n[e] * di));
 }
 
 // ---------------------------------------------------------------------------

@@ -178,8 +178,8 @@ class Context:
         y-forward transforms of an i-plane in one kernel where it fits (True /
         False, or -1: tuned); ff_mfma: the far field on the matrix cores
         (True / False, or -1: the library's choice); ff_group: the far field
-        by groups of directions sharing their z component where the set
-        splits so (True / False, or -1: the default, on)."""
+        by columns, once per group of directions sharing their z component
+        (True / False, or -1: the default, on)."""
         if x_blocks is not None:
             _check(_lib.ddafft_set_tuning(self._h, 0, int(x_blocks)))
         if x_rb is not None:

@@ -104,13 +104,12 @@ int ddafft_solve(ddafft_ctx* ctx, int nrhs, int solver, float tau, int max_step,
  * is for callers that cannot allocate memory during a solve (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Same arguments and results as ddafft_solve, bit for bit (except the far
- * field of a direction set of scattering planes when the grouped far field's
- * gathered dipole moments, 48 B per dipole for two right-hand sides, do not
- * fit the scratch: then the per-direction kernel, within about 1e-7).  Its
+ * field where its partial sums do not fit the scratch: then fewer of them,
+ * within about 1e-7).  Its
  * scratch (block partials, discrepancy history, far-field partials and phase
  * tables, per-call directions, results on their way back, reference-order
- * sum terms, gathered moments) lives in a fixed 32 MiB device array, one per GPU, that every such call on
- * that GPU shares: calls that overlap on one GPU race.  A solve whose
+ * sum terms) lives in a fixed 32 MiB device array, one per GPU, that every such call on that GPU
+ * shares: calls that overlap on one GPU race.  A solve whose
  * scratch would exceed it fails with DDAFFT_EINVAL and a message giving the
  * size needed; results are limited to 1 MiB per call.  Inputs are copied from
  * the caller's memory (no page-locked staging is allocated). */
@@ -179,10 +178,10 @@ int ddafft_set_ahat_mode(ddafft_ctx* ctx, int mode);
  * bit. */
 #define DDAFFT_TUNE_FF_MFMA 4
 /* DDAFFT_TUNE_FF_GROUP: 1 (default, -1) sums the far field (FP64-summed mode)
- * of a direction set whose z components repeat with a period ng, i.e. ng
- * groups of 2..16 directions sharing z (the scattering planes of a fixed
- * orientation), by groups: the sum over l once per group, then per direction
- * over the (i, j) columns; lattices with n_i + n_j <= 512 and n_l <= 256.
+ * by columns on the matrix cores: the sum over l of each (i, j) column once
+ * per group of directions that share their z component (direction sets whose
+ * z repeats with a period ng, groups of at most 8: the scattering planes of a
+ * fixed orientation; otherwise once per direction), then over the columns.
  * 0 always uses the per-direction kernel.  The two agree to about 1e-7
  * relative, not bit for bit. */
 #define DDAFFT_TUNE_FF_GROUP 5

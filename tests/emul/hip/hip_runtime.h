@@ -51,6 +51,7 @@ struct float4 {
     float x, y, z, w;
 };
 inline float2 make_float2(float a, float b) { return float2{a, b}; }
+inline float4 make_float4(float a, float b, float c, float d) { return float4{a, b, c, d}; }
 struct int2 {
     int x, y;
 };
@@ -85,7 +86,7 @@ struct Fiber {
     ucontext_t ctx;     // used once, to enter the fiber
     jmp_buf jb;         // later switches: _setjmp/_longjmp (no signal-mask syscall)
     char* stack = nullptr;
-    int state = 0;      // 0 runnable, 1 waiting at the barrier, 2 returned
+    int state = 0;      // 0 runnable, 1 waiting at the block's barrier, 2 returned, 3 waiting for its wave
     bool started = false;
 };
 
@@ -191,6 +192,16 @@ void launch_now(F f, dim3 g, dim3 b, A... args) {
                                                (unsigned)(t / (b.x * b.y))};
                             resume(t);
                         }
+                    // waves whose 64 threads have all arrived go on
+                    bool released = false;
+                    for (int w = 0; w < nt; w += 64) {
+                        int at = 0;
+                        for (int t = w; t < w + 64 && t < nt; ++t) at += g_fib[t].state == 3;
+                        if (at != 64) continue;
+                        for (int t = w; t < w + 64; ++t) g_fib[t].state = 0;
+                        released = true;
+                    }
+                    if (released) continue;
                     int waiting = 0, done = 0;
                     for (int t = 0; t < nt; ++t) {
                         waiting += g_fib[t].state == 1;
@@ -215,6 +226,12 @@ inline void __syncthreads() {
     emul::to_main();
 }
 
+// All 64 threads of the wave meet.
+inline void emul_wave_sync() {
+    emul::g_fib[emul::g_cur].state = 3;
+    emul::to_main();
+}
+
 inline double __shfl_xor(double v, int off, int width = 64) {
     (void)width;
     emul::g_shfl[threadIdx.x] = v;
@@ -227,20 +244,21 @@ inline double __shfl_xor(double v, int off, int width = 64) {
 // 16x16x4 FP32 matrix product of one wave (v_mfma_f32_16x16x4f32): lane l
 // gives A[l % 16][l / 16] and B[l / 16][l % 16] and gets back
 // D[4 (l / 16) + v][l % 16] (+ its accumulator), the layout the GPU has.  The
-// block's threads meet at a barrier to exchange their operands, so every
-// thread of the block must call it the same number of times.
+// wave's threads meet to exchange their operands, so every thread of a wave
+// must call it the same number of times.
 struct emul_f4 {
     float v[4];
     float& operator[](int i) { return v[i]; }
     float operator[](int i) const { return v[i]; }
 };
 #define DDA_FLOAT4_MFMA emul_f4
+#define DDA_WAVE_SYNC() emul_wave_sync()
 inline emul_f4 __builtin_amdgcn_mfma_f32_16x16x4f32(float a, float b, emul_f4 c, int, int, int) {
     static float A[emul::kMaxThreads], B[emul::kMaxThreads];
     const int t = (int)threadIdx.x;
     A[t] = a;
     B[t] = b;
-    __syncthreads();
+    emul_wave_sync();
     const int w = t / 64, l = t % 64;
     emul_f4 d = c;
     for (int v = 0; v < 4; ++v) {
@@ -249,7 +267,7 @@ inline emul_f4 __builtin_amdgcn_mfma_f32_16x16x4f32(float a, float b, emul_f4 c,
         for (int k = 0; k < 4; ++k) acc += A[w * 64 + 16 * k + row] * B[w * 64 + 16 * k + col];
         d.v[v] = acc;
     }
-    __syncthreads();
+    emul_wave_sync();
     return d;
 }
 
