@@ -187,6 +187,7 @@ struct ddafft_ctx {
     // target
     int8_t* occ = nullptr;
     int8_t* dipf = nullptr;            // [n] 1 where the cell holds a dipole (mv[occ] != 0)
+    int2* rows = nullptr;              // [ni] the rows j of plane i that its dipoles span, [x, y) (0, 0: none)
     int* mv = nullptr;
     int nmat = 0;
     int* cells = nullptr;   // dipole cell indices (far field)
@@ -508,7 +509,7 @@ int launch_matvec(ddafft_ctx* c, int nrhs, const ProArgs& pa, SolveState* st, in
     {
         const int rc = check_args(pa, ea, st != nullptr);
         if (rc) return rc;
-        if (!c->occ || !c->mv || !c->b1 || !c->b2 || !c->b3 || !c->ahat || !c->tables)
+        if (!c->occ || !c->mv || !c->rows || !c->b1 || !c->b2 || !c->b3 || !c->ahat || !c->tables)
             return fail(DDAFFT_ESTATE, "internal: context buffers missing");
     }
     TRY(flush_small(c));
@@ -526,14 +527,14 @@ int launch_matvec(ddafft_ctx* c, int nrhs, const ProArgs& pa, SolveState* st, in
     {
         const int tj = std::min(tile_zf(d.nl), d.nj);
         dim3 grid(d.ni * (d.nj / tj), C);
-        DDA_SWITCH_SMALL(d.nl, hipLaunchKernelGGL((k_zf<NN>), grid, kBlock, 0, s, d, pa, st, c->dipf, c->b1, c->wpre_l,
+        DDA_SWITCH_SMALL(d.nl, hipLaunchKernelGGL((k_zf<NN>), grid, kBlock, 0, s, d, pa, st, c->dipf, c->rows, c->b1, c->wpre_l,
                                                                   c->tw_l));
     }
     if (ev) HIPCHECK(hipEventRecord(ev[1], s));
     {
         const int tl = std::min(tile_zf(d.nj), 2 * d.nl);   // L' lines per block
         dim3 grid(d.ni * (2 * d.nl / tl), C);
-        DDA_SWITCH_SMALL(d.nj, hipLaunchKernelGGL((k_yf<NN>), grid, kBlock, 0, s, d, st, c->b1, c->b2, c->wpre_j, c->tw_j));
+        DDA_SWITCH_SMALL(d.nj, hipLaunchKernelGGL((k_yf<NN>), grid, kBlock, 0, s, d, st, c->rows, c->b1, c->b2, c->wpre_j, c->tw_j));
     }
     }
     if (ev) HIPCHECK(hipEventRecord(ev[2], s));
@@ -574,12 +575,12 @@ int launch_matvec(ddafft_ctx* c, int nrhs, const ProArgs& pa, SolveState* st, in
     {
         const int tl = std::min(tile_yi(2 * d.nj), 2 * d.nl);
         dim3 grid(d.ni * (2 * d.nl / tl), C);
-        DDA_SWITCH_LARGE(2 * d.nj, hipLaunchKernelGGL((k_yi<NN>), grid, kBlock, 0, s, d, st, b3, c->b1, c->tw_2j));
+        DDA_SWITCH_LARGE(2 * d.nj, hipLaunchKernelGGL((k_yi<NN>), grid, kBlock, 0, s, d, st, c->rows, b3, c->b1, c->tw_2j));
     }
     if (ev) HIPCHECK(hipEventRecord(ev[4], s));
     {
         dim3 grid(zi_blocks(d), nrhs);
-        DDA_SWITCH_LARGE(2 * d.nl, hipLaunchKernelGGL((k_zi<NN>), grid, kBlock, 0, s, d, st, c->b1, ea, c->occ, c->dipf,
+        DDA_SWITCH_LARGE(2 * d.nl, hipLaunchKernelGGL((k_zi<NN>), grid, kBlock, 0, s, d, st, c->b1, ea, c->occ, c->dipf, c->rows,
                                                                       c->tw_2l));
     }
     if (ev) HIPCHECK(hipEventRecord(ev[5], s));
@@ -948,7 +949,7 @@ int ddafft_host_free(void* p) {
 int ddafft_destroy(ddafft_ctx* c) {
     if (!c) return DDAFFT_OK;
     if (c->stream) hipStreamSynchronize(c->stream);
-    void* bufs[] = {c->ahat, c->tables, c->occ, c->dipf, c->mv, c->cells, c->b1, c->b2, c->b3, c->P, c->Pmin, c->R,
+    void* bufs[] = {c->ahat, c->tables, c->occ, c->dipf, c->rows, c->mv, c->cells, c->b1, c->b2, c->b3, c->P, c->Pmin, c->R,
                     c->S, c->G, c->H, c->W, c->X, c->Y, c->small, c->hist, c->partials,
                     c->dirs, c->esc, c->fftab, c->Pf, c->phase, c->gaux, c->inc_cell, c->seqbuf,
                     c->ffcol, c->ffpiece, c->ffseg, c->ffpc};
@@ -1015,6 +1016,7 @@ int ddafft_create(int ni, int nj, int nl, float kd, int nrhs_max, ddafft_ctx** o
     if (!rc) rc = small_layout(c);
     if (!rc) rc = dev_alloc(&c->occ, (size_t)n);
     if (!rc) rc = dev_alloc(&c->dipf, (size_t)n);
+    if (!rc) rc = dev_alloc(&c->rows, (size_t)ni);
     if (!rc && hipHostMalloc((void**)&c->state_ring, (size_t)4 * nrhs_max * sizeof(SolveState),
                              hipHostMallocDefault) != hipSuccess)
         rc = fail(DDAFFT_ENOMEM, "hipHostMalloc");
@@ -1109,6 +1111,14 @@ int ddafft_set_target(ddafft_ctx* c, const signed char* occ, int nmat, const int
         if (mv[m]) cells.push_back((int)k);
     }
     if (cells.empty()) return fail(DDAFFT_EINVAL, "target has no dipoles");
+    // the rows that each plane's dipoles span
+    std::vector<int2> rows((size_t)c->d.ni, make_int2(0, 0));
+    for (const int k : cells) {   // ascending along j within a plane
+        const int ij = k / c->d.nl, j = ij & (c->d.nj - 1);
+        int2& r = rows[ij / c->d.nj];
+        if (r.x == r.y) r.x = j;
+        r.y = j + 1;
+    }
     // far-field columns: the (i, j) that hold dipoles, and 8 of them at a time
     // the 16-point chunks of l that their dipoles span, cut into pieces
     std::vector<int> fcol;
@@ -1168,6 +1178,7 @@ int ddafft_set_target(ddafft_ctx* c, const signed char* occ, int nmat, const int
     c->dipf_h.assign((size_t)n, 0);
     for (long long k = 0; k < n; ++k) c->dipf_h[k] = mv[occ[k]] ? 1 : 0;
     if ((rc = upload(c, c->dipf, c->dipf_h.data(), (size_t)n))) return rc;
+    if ((rc = upload(c, c->rows, rows.data(), rows.size() * sizeof(int2)))) return rc;
     if ((rc = upload(c, c->mv, mv, (size_t)nmat * sizeof(int)))) return rc;
     if ((rc = upload(c, c->cells, cells.data(), cells.size() * sizeof(int)))) return rc;
     if ((rc = upload(c, c->ffcol, fcol.data(), fcol.size() * sizeof(int)))) return rc;
@@ -1993,8 +2004,8 @@ int fin_state_enqueue(Run& r, const Fin& f) {
     Dims d = c->d;
     d.nrhs = r.nrhs;
     {
-        dim3 grid((int)std::min<long long>((3 * d.n + kBlock - 1) / kBlock, 2048), r.nrhs);
-        hipLaunchKernelGGL(k_restore, grid, kBlock, 0, c->stream, d, c->st, c->P, c->Pmin,
+        dim3 grid((int)std::min<long long>((d.n + kBlock - 1) / kBlock, 2048), r.nrhs);
+        hipLaunchKernelGGL(k_restore, grid, kBlock, 0, c->stream, d, c->st, c->dipf, c->P, c->Pmin,
                            reinterpret_cast<SolveState*>(c->dn_dev + f.o_st));
         HIPCHECK(hipGetLastError());
     }

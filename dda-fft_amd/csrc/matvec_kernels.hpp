@@ -134,13 +134,65 @@ struct ProArgs {
     float2* Pmin;       // snapshot destination (P_min, dda_func.cpp:1305-1313)
 };
 
+// In a solve (st given) every matvec's input is zero off the dipoles and its
+// output is needed on them only, so the passes leave the rest out: the
+// prologue and the epilogue read and write the solver's vectors on dipole
+// cells, and the rows j of a plane i outside [rows[i].x, rows[i].y), which
+// hold no dipole, are skipped in B1 and B4 (ZF and YI do not write them, YF
+// takes zeros for them, ZI does not read them).  What is left out are zeros,
+// so the results keep their bits.  ddafft_convolution, ddafft_matvec and
+// ddafft_time_matvec (no st) take fields of any values and run dense.
+//
+// Small launches wait for latency, not for bytes: up to 2^18 cells x
+// right-hand sides they keep every row and load the prologue's operands of
+// every cell beside the flags instead of behind them (32^3, 2 RHS: YF 4.8
+// against 5.6 us with the row range, ZF 5.4 against 6.0; 32x32x64, 16 RHS =
+// 2^20: ZYF 29.4 -> 26.2, ZI 21.0 -> 18.4, YI 14.6 -> 12.7 us by leaving them
+// out; 64^3, 2 RHS = 2^19: ZI 18.7 -> 17.4, the others even).
+__device__ __forceinline__ bool small_launch(const Dims& d) { return d.n * d.nrhs <= (1 << 18); }
+
+// The range is requested together with the right-hand side's stopping state (its
+// use in stopped() keeps the load there): one wait for both.
+__device__ __forceinline__ int2 row_range(const Dims& d, const SolveState* st, const int2* __restrict__ rows, int i) {
+    return st && !small_launch(d) ? rows[i] : make_int2(0, d.nj);
+}
+__device__ __forceinline__ bool stopped(const SolveState* st, int rhs, int2 jr) {
+    return st && ((st[rhs].it >= st[rhs].stop_at) | (jr.y < 0));   // jr.y is never negative
+}
+
+// The matvec's input at cell `at` from the loaded operands, zero off the
+// dipoles; the linear combinations go back to the vector they update.
+__device__ __forceinline__ float2 prologue(int mode, bool dip, float2 c1, float2 c2, float2 a, float2 b, float2 d,
+                                           const ProArgs& pa, long long at) {
+    if (!dip) return make_float2(0.f, 0.f);
+    float2 v = a;
+    switch (mode) {
+        case PRO_LC1:   // dda_func.cpp:884-905
+            v = cadd(a, cmul(c1, b));
+            pa.A[at] = v;
+            break;
+        case PRO_LC4:   // :843-882
+            v = cadd(cmul(c2, d), cadd(a, cmul(c1, b)));
+            pa.B[at] = v;
+            break;
+        case PRO_LC2:   // :906-924
+            v = cadd(a, cmul(c1, b));
+            pa.B[at] = v;
+            break;
+        default:
+            break;
+    }
+    return v;
+}
+
 // ---------------------------------------------------------------------------
 // ZF: lines (c, i, j) along l; n_l inputs -> 2 n_l outputs.
 // ---------------------------------------------------------------------------
 
 template <int NL>
 __global__ __launch_bounds__(kBlock) void k_zf(Dims d, ProArgs pa, const SolveState* __restrict__ st,
-                                               const int8_t* __restrict__ dipf, float2* __restrict__ b1,
+                                               const int8_t* __restrict__ dipf, const int2* __restrict__ rows,
+                                               float2* __restrict__ b1,
                                                const float2* __restrict__ wpre, const float2* __restrict__ tw) {
     constexpr int TJ = TileZF<NL>::T;
     constexpr int LS = NL + kLpad;
@@ -151,8 +203,10 @@ __global__ __launch_bounds__(kBlock) void k_zf(Dims d, ProArgs pa, const SolveSt
     const int c = blockIdx.y, rhs = c / 3;
     float2 c1 = make_float2(0.f, 0.f), c2 = c1;
     int snap = 0;
+    const int i = blockIdx.x >> __builtin_ctz(max(d.nj / TJ, 1));   // tiles per plane: a power of two
+    const int2 jr = row_range(d, st, rows, i);
+    if (stopped(st, rhs, jr)) return;
     if (st) {
-        if (st[rhs].it >= st[rhs].stop_at) return;
         c1 = st[rhs].pro_c1;
         c2 = st[rhs].pro_c2;
         // only the first matvec of an iteration carries the P -> P_min copy
@@ -162,56 +216,43 @@ __global__ __launch_bounds__(kBlock) void k_zf(Dims d, ProArgs pa, const SolveSt
     // tiles and a run-time one otherwise
     auto tile = [&](auto tile_arg) {
         const int tj = tile_arg, ntile = d.nj / tj;
-        const int i = blockIdx.x / ntile, j0 = (blockIdx.x - i * ntile) * tj;
+        const int j0 = (blockIdx.x - i * ntile) * tj;
+        if (j0 + tj <= jr.x || j0 >= jr.y) return;   // no dipole in these rows: YF does not read them
         const long long cell0 = ((long long)i * d.nj + j0) * NL;
         const long long cb = (long long)c * d.n + cell0;   // this block's cells of component c
         const int nld = tj * NL;
-        // every load of the thread is issued before the first is used: flags and
-        // the prologue's operands (the prologue writes only cells it has read)
+        // the flags of all of the thread's cells, then the prologue's operands on
+        // the dipoles (the prologue writes only cells it has read)
         bool dip[NLD];
         float2 va[NLD], vb[NLD], vd[NLD], vp[NLD];
         const int mode = pa.mode;
-#pragma unroll
-        for (int q = 0; q < NLD; ++q) {
-            const int f = threadIdx.x + q * kBlock;
-            dip[q] = false;
+        auto operands = [&](int q, int f, bool on) {
             va[q] = vb[q] = vd[q] = vp[q] = make_float2(0.f, 0.f);
-            if (f < nld) {
-                dip[q] = dipf[cell0 + f] != 0;
+            if (f < nld && on) {
                 va[q] = pa.A[cb + f];
                 if (mode != PRO_COPY) vb[q] = pa.B[cb + f];
                 if (mode == PRO_LC4) vd[q] = pa.D[cb + f];
                 if (snap) vp[q] = pa.P[cb + f];   // P is never a prologue output
             }
+        };
+#pragma unroll
+        for (int q = 0; q < NLD; ++q) {
+            const int f = threadIdx.x + q * kBlock;
+            dip[q] = !st || (f < nld && dipf[cell0 + f] != 0);
+        }
+        if (small_launch(d)) {
+#pragma unroll
+            for (int q = 0; q < NLD; ++q) operands(q, threadIdx.x + q * kBlock, true);
+        } else {
+#pragma unroll
+            for (int q = 0; q < NLD; ++q) operands(q, threadIdx.x + q * kBlock, dip[q]);
         }
 #pragma unroll
         for (int q = 0; q < NLD; ++q) {
             const int f = threadIdx.x + q * kBlock;
             if (f < nld) {
-                float2 v;
-                switch (mode) {
-                    case PRO_LC1:   // dda_func.cpp:884-905
-                        v = va[q];
-                        if (dip[q]) {
-                            v = cadd(va[q], cmul(c1, vb[q]));
-                            pa.A[cb + f] = v;
-                        }
-                        break;
-                    case PRO_LC4:   // :843-882
-                        v = dip[q] ? cadd(cmul(c2, vd[q]), cadd(va[q], cmul(c1, vb[q]))) : make_float2(0.f, 0.f);
-                        pa.B[cb + f] = v;
-                        break;
-                    case PRO_LC2:   // :906-924
-                        v = vb[q];
-                        if (dip[q]) {
-                            v = cadd(va[q], cmul(c1, vb[q]));
-                            pa.B[cb + f] = v;
-                        }
-                        break;
-                    default:
-                        v = va[q];
-                }
-                if (snap) pa.Pmin[cb + f] = vp[q];
+                const float2 v = prologue(mode, dip[q], c1, c2, va[q], vb[q], vd[q], pa, cb + f);
+                if (snap && dip[q]) pa.Pmin[cb + f] = vp[q];
                 const int t = f >> LNL, l = f & (NL - 1);
                 s[t * LS + l] = v;
                 s[(tj + t) * LS + l] = cmul(wpre[l], v);
@@ -229,7 +270,8 @@ __global__ __launch_bounds__(kBlock) void k_zf(Dims d, ProArgs pa, const SolveSt
             fft_lds_fixed<NL, 2 * TJ, LS, kBlock, Plan<NL>::NST - 1>(s, stw);
             fft_last_stage_out<NL, 2 * TJ, LS, NL>(s, stw, [&](int line, int k, float2 v) {
                 const bool odd = line >= TJ;
-                dst[((odd ? NL + k : k) << lnj) + (odd ? line - TJ : line)] = v;
+                const int t = odd ? line - TJ : line;
+                if (j0 + t >= jr.x && j0 + t < jr.y) dst[((odd ? NL + k : k) << lnj) + t] = v;
             });
         } else {
             fft_lds<NL, 2 * TJ, LS>(s, 2 * tj, stw);
@@ -241,7 +283,7 @@ __global__ __launch_bounds__(kBlock) void k_zf(Dims d, ProArgs pa, const SolveSt
                 if (f < 2 * NL * tj) {   // row L' of B1: the even transform's outputs, then the odd one's
                     const int Lp = f >> ltj, t = f - (Lp << ltj);
                     const float2 v = Lp >= NL ? s[(tj + t) * LS + (Lp - NL)] : s[t * LS + Lp];
-                    dst[(Lp << lnj) + t] = v;
+                    if (j0 + t >= jr.x && j0 + t < jr.y) dst[(Lp << lnj) + t] = v;
                 }
             }
         }
@@ -311,51 +353,35 @@ __global__ __launch_bounds__((ZyfShape<NJ, NL>::BT)) void k_zyf(Dims d, ProArgs 
     for (int q0 = 0; q0 < E; q0 += KC) {
         bool dip[KC];
         float2 va[KC], vb[KC], vd[KC], vp[KC];
-#pragma unroll
-        for (int k = 0; k < KC; ++k) {
-            const int f = threadIdx.x + (q0 + k) * BT;
-            dip[k] = false;
+        auto operands = [&](int k, int f, bool on) {
             va[k] = vb[k] = vd[k] = vp[k] = make_float2(0.f, 0.f);
-            if (NP % BT == 0 || f < NP) {
-                dip[k] = dipf[cell0 + f] != 0;
+            if ((NP % BT == 0 || f < NP) && on) {
                 va[k] = pa.A[cb + f];
                 if (mode != PRO_COPY) vb[k] = pa.B[cb + f];
                 if (mode == PRO_LC4) vd[k] = pa.D[cb + f];
                 if (snap) vp[k] = pa.P[cb + f];
             }
+        };
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            const int f = threadIdx.x + (q0 + k) * BT;
+            dip[k] = !st || ((NP % BT == 0 || f < NP) && dipf[cell0 + f] != 0);
+        }
+        if (small_launch(d)) {
+#pragma unroll
+            for (int k = 0; k < KC; ++k) operands(k, threadIdx.x + (q0 + k) * BT, true);
+        } else {
+#pragma unroll
+            for (int k = 0; k < KC; ++k) operands(k, threadIdx.x + (q0 + k) * BT, dip[k]);
         }
 #pragma unroll
         for (int k = 0; k < KC; ++k) {
             const int q = q0 + k;
             const int f = threadIdx.x + q * BT;
+            v[q] = make_float2(0.f, 0.f);
             if (NP % BT == 0 || f < NP) {
-                float2 x;
-                switch (mode) {
-                    case PRO_LC1:
-                        x = va[k];
-                        if (dip[k]) {
-                            x = cadd(va[k], cmul(c1, vb[k]));
-                            pa.A[cb + f] = x;
-                        }
-                        break;
-                    case PRO_LC4:
-                        x = dip[k] ? cadd(cmul(c2, vd[k]), cadd(va[k], cmul(c1, vb[k]))) : make_float2(0.f, 0.f);
-                        pa.B[cb + f] = x;
-                        break;
-                    case PRO_LC2:
-                        x = vb[k];
-                        if (dip[k]) {
-                            x = cadd(va[k], cmul(c1, vb[k]));
-                            pa.B[cb + f] = x;
-                        }
-                        break;
-                    default:
-                        x = va[k];
-                }
-                if (snap) pa.Pmin[cb + f] = vp[k];
-                v[q] = x;
-            } else {
-                v[q] = make_float2(0.f, 0.f);
+                v[q] = prologue(mode, dip[k], c1, c2, va[k], vb[k], vd[k], pa, cb + f);
+                if (snap && dip[k]) pa.Pmin[cb + f] = vp[k];
             }
         }
         __builtin_amdgcn_sched_barrier(0);   // keep the next chunk's loads behind this chunk's use
@@ -419,21 +445,23 @@ __global__ __launch_bounds__((ZyfShape<NJ, NL>::BT)) void k_zyf(Dims d, ProArgs 
 
 template <int NJ>
 __global__ __launch_bounds__(kBlock) void k_yf(Dims d, const SolveState* __restrict__ st,
-                                               const float2* __restrict__ b1, float2* __restrict__ b2,
+                                               const int2* __restrict__ rows, const float2* __restrict__ b1, float2* __restrict__ b2,
                                                const float2* __restrict__ wpre, const float2* __restrict__ tw) {
     constexpr int TI = TileZF<NJ>::T;
     constexpr int LS = NJ + kLpad;
     __shared__ float2 s[2 * TI * LS];
     __shared__ float2 stw[NJ];
-    const int c = blockIdx.y, rhs = c / 3;
-    if (st && st[rhs].it >= st[rhs].stop_at) return;
+    const int c = blockIdx.y;
     constexpr int LNJ = ilog2c(NJ);
     const int NL2 = 2 * d.nl;
+    const int i = blockIdx.x >> __builtin_ctz(max(NL2 / TI, 1));
+    const int2 jr = row_range(d, st, rows, i);
+    if (stopped(st, c / 3, jr)) return;
     // the tile body, with the tile width a compile-time constant for full
     // tiles and a run-time one otherwise
     auto tile = [&](auto tile_arg) {
         const int ti = tile_arg, nlt = NL2 / ti;
-        const int i = blockIdx.x / nlt, L0 = (blockIdx.x - i * nlt) * ti;
+        const int L0 = (blockIdx.x - i * nlt) * ti;
         const int lnl2 = __builtin_ctz(NL2), lti = __builtin_ctz(ti);
         {
             constexpr int NLD = (TI * NJ + kBlock - 1) / kBlock;
@@ -441,8 +469,9 @@ __global__ __launch_bounds__(kBlock) void k_yf(Dims d, const SolveState* __restr
             float2 v[NLD];
 #pragma unroll
             for (int q = 0; q < NLD; ++q) {
-                const int f = threadIdx.x + q * kBlock;
-                if (f < ti * NJ) v[q] = src[f];
+                const int f = threadIdx.x + q * kBlock, jj = f & (NJ - 1);
+                v[q] = make_float2(0.f, 0.f);
+                if (f < ti * NJ && jj >= jr.x && jj < jr.y) v[q] = src[f];
             }
 #pragma unroll
             for (int q = 0; q < NLD; ++q) {
@@ -819,20 +848,22 @@ __global__ __launch_bounds__(kBlock) DDA_WAVES_PER_EU(XWaves<NI, RB, RUN, COMPAC
 
 template <int NJ2>
 __global__ __launch_bounds__(kBlock) void k_yi(Dims d, const SolveState* __restrict__ st,
-                                               const float2* __restrict__ b3, float2* __restrict__ b4,
+                                               const int2* __restrict__ rows, const float2* __restrict__ b3, float2* __restrict__ b4,
                                                const float2* __restrict__ tw) {
     constexpr int TL = TileYI<NJ2>::T;
     constexpr int LS = NJ2 + kLpad;
     __shared__ float2 s[TL * LS];
     __shared__ float2 stw[NJ2];
-    const int c = blockIdx.y, rhs = c / 3;
-    if (st && st[rhs].it >= st[rhs].stop_at) return;
+    const int c = blockIdx.y;
     const int NL2 = 2 * d.nl;
+    const int i = blockIdx.x >> __builtin_ctz(max(NL2 / TL, 1));
+    const int2 jr = row_range(d, st, rows, i);
+    if (stopped(st, c / 3, jr) || jr.x >= jr.y) return;   // a plane without dipoles: nothing to keep
     // the tile body, with the tile width a compile-time constant for full
     // tiles and a run-time one otherwise
     auto tile = [&](auto tile_arg) {
         const int tl = tile_arg, nlt = NL2 / tl;
-        const int i = blockIdx.x / nlt, L0 = (blockIdx.x - i * nlt) * tl;
+        const int L0 = (blockIdx.x - i * nlt) * tl;
         const int ltl0 = __builtin_ctz(tl), lnl20 = __builtin_ctz(NL2);
         // columns L0 .. L0 + tl - 1 of plane (c, i) of B3 [C][J][i][L']: runs of
         // tl in every row J
@@ -876,7 +907,9 @@ __global__ __launch_bounds__(kBlock) void k_yi(Dims d, const SolveState* __restr
             constexpr int NJ = NJ2 / 2;
             const int lnl2 = __builtin_ctz(NL2);
             float2* dst = b4 + (((long long)c * d.ni + i) * NJ) * NL2 + L0;
-            fft_last_stage_out<NJ2, TL, LS, NJ>(s, stw, [&](int t, int j, float2 v) { dst[(j << lnl2) + t] = v; });
+            fft_last_stage_out<NJ2, TL, LS, NJ>(s, stw, [&](int t, int j, float2 v) {
+                if (j >= jr.x && j < jr.y) dst[(j << lnl2) + t] = v;
+            });
         } else {
             {
                 constexpr int NLD = (TL * NJ2 + kBlock - 1) / kBlock;
@@ -904,7 +937,7 @@ __global__ __launch_bounds__(kBlock) void k_yi(Dims d, const SolveState* __restr
                 const int f = threadIdx.x + q * kBlock;
                 if (f < tl * NJ) {
                     const int j = f >> ltl, t = f - (j << ltl);
-                    dst[(j << lnl2) + t] = s[t * LS + j];
+                    if (j >= jr.x && j < jr.y) dst[(j << lnl2) + t] = s[t * LS + j];
                 }
             }
         }
@@ -963,7 +996,7 @@ template <int NL2>
 __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ st,
                                                const float2* __restrict__ b4, EpiArgs ea,
                                                const int8_t* __restrict__ occ, const int8_t* __restrict__ dipf,
-                                               const float2* __restrict__ tw) {
+                                               const int2* __restrict__ rows, const float2* __restrict__ tw) {
     constexpr int TJ = TileZI<NL2>::T;
     constexpr int LS = ZStride<NL2, TJ>::S;
     constexpr int NLH = NL2 / 2;
@@ -974,17 +1007,21 @@ __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ 
     __shared__ float2 stw[NL2];
     __shared__ double red[kSlots * 16];
     const int rhs = blockIdx.y;
-    float rB = 0.f;
-    if (st) {
-        if (st[rhs].it >= st[rhs].stop_at) return;
-        rB = st[rhs].rB;
-    }
+    const int i = blockIdx.x >> __builtin_ctz(max(d.nj / TJ, 1));
+    const int2 jr = row_range(d, st, rows, i);
+    if (stopped(st, rhs, jr)) return;
+    const float rB = st ? st[rhs].rB : 0.f;
     // the tile body, with the row count a compile-time constant for full tiles
     // (nj >= TJ) and a run-time one otherwise
     auto tile = [&](auto tj_arg) {
         const int tj = tj_arg, njt = d.nj / tj;
-        const int i = blockIdx.x / njt, j0 = (blockIdx.x - i * njt) * tj;
+        const int j0 = (blockIdx.x - i * njt) * tj;
         const int ltj = __builtin_ctz(tj), lnj = __builtin_ctz(d.nj), lni = __builtin_ctz(d.ni);
+        if (j0 + tj <= jr.x || j0 >= jr.y) {   // no dipole in these rows
+            if (ea.partials && threadIdx.x < kSlots)
+                ea.partials[((long long)rhs * gridDim.x + blockIdx.x) * kSlots + threadIdx.x] = 0.0;
+            return;
+        }
         {
             const float2* src = b4 + (((long long)rhs * 3 * d.ni + i) * d.nj + j0) * NL2;
             const int lcs = lni + lnj + LNL2;   // one component plane of B4
@@ -993,9 +1030,10 @@ __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ 
 #pragma unroll
             for (int q = 0; q < NLD; ++q) {
                 const int f = threadIdx.x + q * kBlock;
+                v[q] = make_float2(0.f, 0.f);
                 if (f < nld) {
                     const int LL = f & (NL2 - 1), r = f >> LNL2, t = r & (tj - 1), comp = r >> ltj;
-                    v[q] = src[(comp << lcs) + (t << LNL2) + LL];
+                    if (j0 + t >= jr.x && j0 + t < jr.y) v[q] = src[(comp << lcs) + (t << LNL2) + LL];
                 }
             }
 #pragma unroll
@@ -1021,10 +1059,9 @@ __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ 
         const long long rb = (long long)rhs * 3 * d.n;
         const long long k0 = ((long long)i * d.nj + j0) * NLH;   // first cell of the block
         const int nep = tj * NLH;
-        // off the dipoles only the Simple solver's first step reads x (every
-        // other epilogue writes zeros there or leaves the cell): the operand
-        // loads wait on the flags as the polarizability waits on occ
-        const bool x_everywhere = kind == EK_SIM_R0;
+        // a solve's epilogue works on dipole cells; the operand loads wait on the
+        // flags as the polarizability waits on occ
+        const bool dense = !st;
         int kq[NEP];
         bool dip[NEP];
         float2 a[NEP], xr[NEP][3], yr[NEP][3], o2[NEP][3];
@@ -1040,37 +1077,40 @@ __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ 
                 const int m = occ[k0 + f];
                 dip[q] = dipf[k0 + f] != 0;
                 a[q] = al[m];
-                const bool ldx = need_x && (dip[q] || x_everywhere);
-                const bool ldd = dip[q];
+                if (dip[q])
 #pragma unroll
-                for (int c3 = 0; c3 < 3; ++c3) {
-                    const long long ck = rb + c3 * d.n + k0 + f;
-                    if (ldx) xr[q][c3] = ea.x[ck];
-                    if (need_y && ldd) yr[q][c3] = ea.y[ck];
-                    if (need_o2 && ldd) o2[q][c3] = ea.out2[ck];
-                }
+                    for (int c3 = 0; c3 < 3; ++c3) {
+                        const long long ck = rb + c3 * d.n + k0 + f;
+                        if (need_x) xr[q][c3] = ea.x[ck];
+                        if (need_y) yr[q][c3] = ea.y[ck];
+                        if (need_o2) o2[q][c3] = ea.out2[ck];
+                    }
             }
         }
         double acc[kSlots] = {0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int q = 0; q < NEP; ++q) {
             const int f = kq[q];
-            if (f >= nep) continue;
+            if (f >= nep || !(dip[q] || dense)) continue;
             const int t = f >> LNLH, l = f & (NLH - 1);
             const long long k = k0 + f;
-            const bool dp = dip[q];
             float2 av = a[q];
             if (ea.conj) av.y = -av.y;
             float2 cv[3], o[3];
 #pragma unroll
             for (int comp = 0; comp < 3; ++comp) cv[comp] = cconj(s[(comp * tj + t) * LS + l]);
             double nrm = 0;
+            // every kind but the two dense ones comes here on dipole cells only
             switch (kind) {
                 case EK_CONV:
 #pragma unroll
                     for (int c3 = 0; c3 < 3; ++c3) ea.out[rb + c3 * d.n + k] = cv[c3];
                     break;
                 case EK_MV:
+#pragma unroll
+                    for (int c3 = 0; c3 < 3; ++c3)
+                        ea.out[rb + c3 * d.n + k] = dip[q] ? csub(xr[q][c3], cmul(av, cv[c3])) : make_float2(0.f, 0.f);
+                    break;
                 case EK_BICG_H:
                 case EK_BICG_W:
                 case EK_CG_W:
@@ -1078,11 +1118,9 @@ __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ 
                 case EK_AA_W:
 #pragma unroll
                     for (int c3 = 0; c3 < 3; ++c3) {
-                        const long long ck = rb + c3 * d.n + k;
                         const float2 x = xr[q][c3];
-                        o[c3] = dp ? csub(x, cmul(av, cv[c3])) : make_float2(0.f, 0.f);
-                        ea.out[ck] = o[c3];
-                        if (!dp) continue;
+                        o[c3] = csub(x, cmul(av, cv[c3]));
+                        ea.out[rb + c3 * d.n + k] = o[c3];
                         if (kind == EK_BICG_H) dot_acc(yr[q][c3], o[c3], acc[0], acc[1]);
                         if (kind == EK_BICG_W) {
                             dot_acc(o[c3], x, acc[0], acc[1]);
@@ -1095,7 +1133,7 @@ __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ 
                         if (kind == EK_AA_S0) nrm += norm_term(x);
                         if (kind == EK_AA_W) acc[4] += norm_term(x);
                     }
-                    if (kind == EK_AA_S0 && dp) acc[5] += sqrt(nrm);
+                    if (kind == EK_AA_S0) acc[5] += sqrt(nrm);
                     break;
                 case EK_BICG_R0:
                 case EK_CG_R0:
@@ -1104,51 +1142,43 @@ __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ 
 #pragma unroll
                     for (int c3 = 0; c3 < 3; ++c3) {
                         const long long ck = rb + c3 * d.n + k;
-                        o[c3] = dp ? cneg(cmul(av, cv[c3])) : make_float2(0.f, 0.f);
+                        o[c3] = cneg(cmul(av, cv[c3]));
                         ea.out[ck] = o[c3];
                         if (kind == EK_BICG_R0) {
                             ea.out2[ck] = o[c3];
                             ea.out3[ck] = o[c3];
-                            if (dp) dot_acc(o[c3], o[c3], acc[0], acc[1]);
+                            dot_acc(o[c3], o[c3], acc[0], acc[1]);
                         }
                         if (kind == EK_CG_R0) ea.out2[ck] = o[c3];
-                        if (kind == EK_AA_R0 && dp) acc[4] += norm_term(o[c3]);
+                        if (kind == EK_AA_R0) acc[4] += norm_term(o[c3]);
                         if (kind == EK_SIM_R0) {
                             const float2 x = xr[q][c3];
                             ea.out2[ck] = x;                       // S = P0 (Copying)
-                            ea.out3[ck] = csub(x, o[c3]);          // P = S - R (all cells)
+                            ea.out3[ck] = csub(x, o[c3]);          // P = S - R
                         }
-                        if (dp) nrm += norm_term(o[c3]);
+                        nrm += norm_term(o[c3]);
                     }
-                    if ((kind == EK_CG_R0 || kind == EK_SIM_R0) && dp) acc[5] += sqrt(nrm);
+                    if (kind == EK_CG_R0 || kind == EK_SIM_R0) acc[5] += sqrt(nrm);
                     break;
                 case EK_AA_SUPD:
 #pragma unroll
                     for (int c3 = 0; c3 < 3; ++c3) {
-                        const long long ck = rb + c3 * d.n + k;
-                        if (dp) {
-                            const float2 w = csub(xr[q][c3], cmul(av, cv[c3]));
-                            ea.out2[ck] = cadd(w, rmul(rB, o2[q][c3]));
-                        }
+                        const float2 w = csub(xr[q][c3], cmul(av, cv[c3]));
+                        ea.out2[rb + c3 * d.n + k] = cadd(w, rmul(rB, o2[q][c3]));
                     }
                     break;
                 case EK_SIM:
 #pragma unroll
                     for (int c3 = 0; c3 < 3; ++c3) {
                         const long long ck = rb + c3 * d.n + k;
-                        if (dp) {
-                            const float2 x = xr[q][c3];
-                            const float2 w = csub(x, cmul(av, cv[c3]));
-                            const float2 rr = csub(w, yr[q][c3]);
-                            ea.out[ck] = rr;
-                            ea.out2[ck] = csub(x, rmul(ea.tau, rr));
-                            nrm += norm_term(rr);
-                        } else {
-                            ea.out[ck] = make_float2(0.f, 0.f);
-                            ea.out2[ck] = make_float2(0.f, 0.f);
-                        }
+                        const float2 x = xr[q][c3];
+                        const float2 w = csub(x, cmul(av, cv[c3]));
+                        const float2 rr = csub(w, yr[q][c3]);
+                        ea.out[ck] = rr;
+                        ea.out2[ck] = csub(x, rmul(ea.tau, rr));
+                        nrm += norm_term(rr);
                     }
-                    if (dp) acc[5] += sqrt(nrm);
+                    acc[5] += sqrt(nrm);
                     break;
                 default:
                     break;

@@ -117,15 +117,9 @@ __global__ __launch_bounds__(kBlock) void k_update(Dims d, SolveState* __restric
     double acc[kSlots] = {0, 0, 0, 0, 0, 0};
     for (long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x; k < d.n;
          k += (long long)gridDim.x * blockDim.x) {
-        if (dipf[k] == 0) {
-            // off the dipoles R keeps its value, and so does P except in
-            // BiCGStab, which sets it to zero: nothing is read there
-            if (ua.kind == UK_BICG) {
-#pragma unroll
-                for (int q = 0; q < 3; ++q) ua.P[rb + q * d.n + k] = make_float2(0.f, 0.f);
-            }
-            continue;
-        }
+        // off the dipoles P is zero from the first approximation (or the
+        // adjoint source) on and nothing reads the other vectors
+        if (dipf[k] == 0) continue;
         double nrm = 0;
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
@@ -178,7 +172,8 @@ __global__ __launch_bounds__(kBlock) void k_finalize(SolveState* __restrict__ st
 
 // Best-iterate fallback (dda_func.cpp:1537-1548); block 0 also writes the
 // final states to `out` (host-visible, may be nullptr).
-__global__ __launch_bounds__(kBlock) void k_restore(Dims d, SolveState* __restrict__ st, float2* __restrict__ P,
+__global__ __launch_bounds__(kBlock) void k_restore(Dims d, SolveState* __restrict__ st,
+                                                    const int8_t* __restrict__ dipf, float2* __restrict__ P,
                                                     const float2* __restrict__ Pmin, SolveState* __restrict__ out) {
     const int rhs = blockIdx.y;
     SolveState s = st[rhs];
@@ -192,9 +187,11 @@ __global__ __launch_bounds__(kBlock) void k_restore(Dims d, SolveState* __restri
     }
     if (!restore) return;
     const long long rb = (long long)rhs * 3 * d.n;
-    for (long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x; k < 3 * d.n;
-         k += (long long)gridDim.x * blockDim.x)
-        P[rb + k] = Pmin[rb + k];
+    for (long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x; k < d.n; k += (long long)gridDim.x * blockDim.x) {
+        if (dipf[k] == 0) continue;   // P is zero there, and Pmin was not written
+#pragma unroll
+        for (int q = 0; q < 3; ++q) P[rb + q * d.n + k] = Pmin[rb + q * d.n + k];
+    }
 }
 
 // ---------------------------------------------------------------------------
