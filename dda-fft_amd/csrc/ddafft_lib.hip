@@ -299,6 +299,15 @@ namespace {
 int flush_small(ddafft_ctx* c);
 int inc_tab_len(const ddafft_ctx* c);
 
+// Plane shapes (n_j, n_l) of the fused passes that hold a plane's lines in LDS
+// at once (k_zyf_wide, k_yzi): at most 2^11 cells, axes of 8 to 256 points.
+#define DDA_PLANES(X)                                                                            \
+    X(8, 8) X(8, 16) X(8, 32) X(8, 64) X(8, 128) X(8, 256)                                       \
+    X(16, 8) X(16, 16) X(16, 32) X(16, 64) X(16, 128) X(32, 8) X(32, 16) X(32, 32) X(32, 64)     \
+    X(64, 8) X(64, 16) X(64, 32) X(128, 8) X(128, 16) X(256, 8)
+
+bool small_plane(const Dims& d) { return d.nj >= 8 && d.nl >= 8 && d.nj * d.nl <= 2048; }
+
 // The launch schedule of one matvec / iteration: the tuned table's entry for
 // this lattice and right-hand-side count (tuned_table.hpp, written by
 // dda-fft_amd/tune.py on an MI355X), else the built-in rule; a value set
@@ -311,16 +320,17 @@ Schedule schedule(const ddafft_ctx* c, int nrhs) {
     // built-in rule: four right-hand sides per X tile when they come in fours
     // on lines of at most 32 points (32^3, 16 RHS: 41 us against 44.5 in
     // pairs; 64^3: 425 against 315), every group its own block, graphs on;
-    // z/y forward fused when its launch (one block per (component, i)-plane)
-    // has at least 192 blocks: below that the split passes' wider grids win
-    // (32^3, 1 RHS: 38.0 us a matvec split, 39.3 fused; 64^3, 16 RHS: 709
-    // against 675)
+    // z/y forward of 64 x 64 planes fused when its launch (one block per
+    // (component, i)-plane) has at least 192 blocks (64^3, 16 RHS: 709 us a
+    // matvec split, 675 fused)
     Schedule s{(nrhs % 4 == 0 && c->d.ni <= 32) ? 4 : 2, 1 << 30, 1, c->d.ni * 3 * nrhs >= 192 ? 1 : 0};
     for (const TunedEntry& e : kTuned)
         if (e.ni == c->d.ni && e.nj == c->d.nj && e.nl == c->d.nl && e.nrhs == nrhs) {
             s = Schedule{e.x_rb, e.x_blocks, e.graph, e.fuse};
             break;
         }
+    // planes whose lines fit a block's LDS at once always run fused (zyf_launch)
+    if (small_plane(c->d)) s.fuse = 1;
     if (c->x_rb > 0) s.x_rb = c->x_rb;
     if (c->x_blocks > 0) s.x_blocks = c->x_blocks;
     if (c->use_graph >= 0) s.graph = c->use_graph;
@@ -471,27 +481,79 @@ int check_args(const ProArgs& pa, const EpiArgs& ea, bool solver) {
     return DDAFFT_OK;
 }
 
-// The fused z/y-forward pass for the plane shapes it is built for (n_j, n_l
-// in {8, 16, 32, 64}); false when the plane needs ZF + YF.
+// The fused z/y-forward pass: planes of at most 2^11 cells, and 64 x 64 ones;
+// false when the plane needs ZF + YF.  Up to 2^18 cells x right-hand sides the
+// form with every line of the plane in LDS at once (k_zyf_wide: a shorter
+// chain), beyond that the one that takes the parities in turn (k_zyf: a
+// quarter of the LDS, more blocks per CU) where both are built.  CG step,
+// MI355X, turn by turn against at once: 32^3, 2 RHS 46.6 -> 44.5 us; 32x32x64,
+// 2 RHS 58.2 -> 55.4; 64x32x64, 1 RHS 68.1 -> 65.7; 128x32x32, 2 RHS (2^18)
+// 88.4 -> 87.8; 32x32x64, 6 RHS 101.6 -> 102.7; 64x64x32, 4 RHS 119.9 -> 123.2;
+// 32^3, 16 RHS 101.0 -> 103.5.
 bool zyf_launch(ddafft_ctx* c, const Dims& d, const ProArgs& pa, SolveState* st, int C, hipStream_t s) {
     const dim3 grid(d.ni, C);
-#define DDA_ZYF(NJ, NL)                                                                                        \
-    case NJ * 1024 + NL:                                                                                       \
-        hipLaunchKernelGGL((k_zyf<NJ, NL>), grid, (ZyfShape<NJ, NL>::BT), 0, s, d, pa, st, c->dipf, c->b2, c->wpre_l, c->tw_l, \
-                           c->wpre_j, c->tw_j);                                                                \
+#define DDA_ZYF(NJ, NL)                                                                                              \
+    case NJ * 1024 + NL:                                                                                             \
+        hipLaunchKernelGGL((k_zyf<NJ, NL>), grid, (ZyfShape<NJ, NL>::BT), 0, s, d, pa, st, c->dipf, c->b2, c->wpre_l, \
+                           c->tw_l, c->wpre_j, c->tw_j);                                                             \
         return true;
+#define DDA_ZYFW(NJ, NL)                                                                                             \
+    case NJ * 1024 + NL:                                                                                             \
+        hipLaunchKernelGGL((k_zyf_wide<NJ, NL>), grid, (ZyfwShape<NJ, NL>::BT), 0, s, d, pa, st, c->dipf, c->b2,     \
+                           c->wpre_l, c->tw_l, c->wpre_j, c->tw_j);                                                  \
+        return true;
+    if (d.n * d.nrhs > (1 << 18) || d.nj * d.nl > 2048) {
+        switch (d.nj * 1024 + d.nl) {
+            DDA_ZYF(8, 8) DDA_ZYF(8, 16) DDA_ZYF(8, 32) DDA_ZYF(8, 64)
+            DDA_ZYF(16, 8) DDA_ZYF(16, 16) DDA_ZYF(16, 32) DDA_ZYF(16, 64)
+            DDA_ZYF(32, 8) DDA_ZYF(32, 16) DDA_ZYF(32, 32) DDA_ZYF(32, 64)
+            DDA_ZYF(64, 8) DDA_ZYF(64, 16) DDA_ZYF(64, 32) DDA_ZYF(64, 64)
+            default:
+                break;
+        }
+    }
     switch (d.nj * 1024 + d.nl) {
-        DDA_ZYF(8, 8) DDA_ZYF(8, 16) DDA_ZYF(8, 32) DDA_ZYF(8, 64)
-        DDA_ZYF(16, 8) DDA_ZYF(16, 16) DDA_ZYF(16, 32) DDA_ZYF(16, 64)
-        DDA_ZYF(32, 8) DDA_ZYF(32, 16) DDA_ZYF(32, 32) DDA_ZYF(32, 64)
-        DDA_ZYF(64, 8) DDA_ZYF(64, 16) DDA_ZYF(64, 32) DDA_ZYF(64, 64)
+        DDA_PLANES(DDA_ZYFW)
         default:
             return false;
     }
 #undef DDA_ZYF
+#undef DDA_ZYFW
 }
 
-// One matvec of nrhs right-hand sides: ZF -> YF (or the fused ZYF) -> X -> YI -> ZI.
+// Whether a matvec's inverse y and z passes run fused (k_yzi): plane shapes it
+// is built for and an epilogue that one component at a time can finish.  One
+// block holds all of the plane's padded lines, so it is ahead as far as they
+// fit 66 KB of LDS, two blocks per CU (CG step, MI355X, YI + ZI against YZI:
+// 16^3, 2 RHS 39.9 -> 36.2 us; 32^3, 2 RHS 48.7 -> 46.6; 32^3, 16 RHS 114.4 ->
+// 101.0; 32x32x64, 16 RHS 189.5 -> 175.7; 64x128x8, 4 RHS 123 -> 95); planes of
+// twice that (132 KB, one block) lost where it counts: 64^3, 2 RHS 125 -> 129,
+// 64x32x128, 6 RHS 343 -> 353.
+bool yzi_on(const ddafft_ctx* c, int kind) {
+    return one_component(kind) && small_plane(c->d) && c->fuse_zy != 0;
+}
+
+bool yzi_launch(ddafft_ctx* c, const Dims& d, const float2* b3, SolveState* st, const EpiArgs& ea, int C, hipStream_t s) {
+    const dim3 grid(d.ni, C);
+#define DDA_YZI(NJ, NL)                                                                                              \
+    case NJ * 1024 + NL:                                                                                             \
+        hipLaunchKernelGGL((k_yzi<NJ, NL>), grid, (YziShape<NJ, NL>::BT), 0, s, d, st, c->rows, b3, ea, c->occ, c->dipf, \
+                           c->tw_2j, c->tw_2l);                                                                      \
+        return true;
+    switch (d.nj * 1024 + d.nl) {
+        DDA_PLANES(DDA_YZI)
+        default:
+            return false;
+    }
+#undef DDA_YZI
+}
+
+// Blocks of a matvec's epilogue per right-hand side (its partial sums).
+int epi_blocks(const ddafft_ctx* c, int kind) { return yzi_on(c, kind) ? 3 * c->d.ni : zi_blocks(c->d); }
+int max_epi_blocks(const Dims& d) { return std::max(zi_blocks(d), 3 * d.ni); }
+
+// One matvec of nrhs right-hand sides: ZF -> YF (or the fused ZYF) -> X ->
+// YI -> ZI (or the fused YZI).
 int launch_matvec(ddafft_ctx* c, int nrhs, const ProArgs& pa, SolveState* st, int iter, const EpiArgs& ea,
                   int conj, hipEvent_t* ev = nullptr) {
     if (!ev && c->prof) {
@@ -572,6 +634,13 @@ int launch_matvec(ddafft_ctx* c, int nrhs, const ProArgs& pa, SolveState* st, in
 #undef DDA_KX
     }
     if (ev) HIPCHECK(hipEventRecord(ev[3], s));
+    if (yzi_on(c, ea.kind)) {
+        if (ev) HIPCHECK(hipEventRecord(ev[4], s));
+        if (!yzi_launch(c, d, b3, st, ea, C, s)) return fail(DDAFFT_ESTATE, "internal: fused inverse pass not built");
+        if (ev) HIPCHECK(hipEventRecord(ev[5], s));
+        HIPCHECK(hipGetLastError());
+        return DDAFFT_OK;
+    }
     {
         const int tl = std::min(tile_yi(2 * d.nj), 2 * d.nl);
         dim3 grid(d.ni * (2 * d.nl / tl), C);
@@ -1022,7 +1091,7 @@ int ddafft_create(int ni, int nj, int nl, float kd, int nrhs_max, ddafft_ctx** o
         rc = fail(DDAFFT_ENOMEM, "hipHostMalloc");
     if (!rc && hipHostGetDevicePointer((void**)&c->ring_dev, c->state_ring, 0) != hipSuccess)
         rc = fail(DDAFFT_EHIP, "hipHostGetDevicePointer of the state ring");
-    if (!rc) rc = ensure_partials(c, (size_t)nrhs_max * std::max<long long>(zi_blocks(c->d), 1024) * kSlots);
+    if (!rc) rc = ensure_partials(c, (size_t)nrhs_max * std::max<long long>(max_epi_blocks(c->d), 1024) * kSlots);
     if (rc) {
         ddafft_destroy(c);
         return rc;
@@ -1352,7 +1421,7 @@ struct Seq {
         ea.partials = c->partials;
         ea.conj = conj;
         TRY(launch_matvec(c, nrhs, pa, c->st, iter, ea, conj));
-        return fin_kind >= 0 ? fin(fin_kind, iter, zi_blocks(c->d)) : DDAFFT_OK;
+        return fin_kind >= 0 ? fin(fin_kind, iter, epi_blocks(c, ea.kind)) : DDAFFT_OK;
     }
     // the solver update, then (fin_kind >= 0) the scalar step over its partials
     int upd(int iter, UpdArgs ua, int fin_kind = -1) {
@@ -1387,8 +1456,6 @@ EpiArgs epi(int kind, const float2* x, float2* out, float2* out2 = nullptr, floa
 
 int step0(Seq& q, int solver) {
     ddafft_ctx* c = q.c;
-    const int zb = zi_blocks(c->d);
-    const int ub = update_blocks(c->d);
     switch (solver) {
         case DDAFFT_SOLVER_CG:
             TRY(q.mv(0, pro(PRO_COPY, c->P), epi(EK_CG_R0, nullptr, c->R, c->S), 0, FK_CG_E0));
@@ -1414,8 +1481,6 @@ int step0(Seq& q, int solver) {
 // matvec and its scalar step) and 2 (the rest)
 int iteration(Seq& q, int solver, int o, float tau, int part = 0) {
     ddafft_ctx* c = q.c;
-    const int zb = zi_blocks(c->d);
-    const int ub = update_blocks(c->d);
     auto snap = [&](ProArgs p) {
         p.P = c->P;
         p.Pmin = c->Pmin;
@@ -1845,7 +1910,7 @@ int run_begin(Run& r) {
         s.stop_at = r.max_step + 1;
     }
     TRY(upload(c, c->st, s0.data(), r.nrhs * sizeof(SolveState)));
-    TRY(ensure_partials(c, (size_t)r.nrhs * std::max(zi_blocks(d), update_blocks(d)) * kSlots));
+    TRY(ensure_partials(c, (size_t)r.nrhs * std::max(max_epi_blocks(d), update_blocks(d)) * kSlots));
     TRY(flush_small(c));   // every staged input of the solve, in one copy
     if (c->pending_first_approx) {
         c->pending_first_approx = false;
@@ -2217,7 +2282,7 @@ int ddafft_solve_noalloc(ddafft_ctx* c, int nrhs, int solver, float tau, int max
         off = 0;
         res = 0;   // results, laid out as fin_layout lays them out
         obs_blocks(c, nrhs, ndirs, ffn, ffS, &cb, &fchunk);
-        n_part = std::max({(size_t)nrhs * std::max(zi_blocks(d), update_blocks(d)) * kSlots, (size_t)nrhs * cb * 2,
+        n_part = std::max({(size_t)nrhs * std::max(max_epi_blocks(d), update_blocks(d)) * kSlots, (size_t)nrhs * cb * 2,
                            (size_t)nrhs * fchunk * std::max(ndirs, 1) * 6});
         n_hist = (size_t)c->nrhs_max * (max_step + 1);
         n_esc = (size_t)nrhs * ndirs * 3;

@@ -369,17 +369,17 @@ __device__ __forceinline__ void fft_lds_fixed(float2* s, const float2* __restric
 // instead of back to LDS.  The butterflies, twiddles and order of the stage
 // in FixedStage: the same bits.  No barrier at the end (nothing is written to
 // LDS).
-template <int N, int NLINES, int LS, int KEEP, class Out>
+template <int N, int NLINES, int LS, int KEEP, int BT = kBlock, class Out>
 __device__ __forceinline__ void fft_last_stage_out(const float2* s, const float2* __restrict__ tw, Out out) {
     constexpr int NST = Plan<N>::NST;
     static_assert(NST >= 2, "a transform of at least two stages");
     constexpr int RL = plan_radix(Plan<N>::K, NST - 1), HL = N / RL;   // span N, step 1
-    constexpr int WL = NLINES * HL, ITL = (WL + kBlock - 1) / kBlock;
+    constexpr int WL = NLINES * HL, ITL = (WL + BT - 1) / BT;
     static_assert(KEEP % HL == 0 && KEEP <= N, "kept outputs: whole runs of the last stage");
 #pragma unroll
     for (int it = 0; it < ITL; ++it) {
-        const int f = threadIdx.x + it * kBlock;
-        if (WL % kBlock == 0 || f < WL) {
+        const int f = threadIdx.x + it * BT;
+        if (WL % BT == 0 || f < WL) {
             const int line = f % NLINES, bf = f / NLINES;   // consecutive lanes: consecutive lines
             const float2* v = s + line * LS + bf;
             float2 z[RL];
@@ -474,13 +474,13 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// Sums NV values over a block of kBlock threads; the result is valid in
+// Sums NV values over a block of BT threads; the result is valid in
 // thread 0.  The wave count is the compile-time block size: reading blockDim
 // would make the compiler wait for every memory operation in flight, the
 // caller's stores included, before the sum.
-template <int NV>
+template <int NV, int BT = kBlock>
 __device__ __forceinline__ void block_sum(double (&v)[NV], double* scratch /* >= NV*16 doubles */) {
-    constexpr int nw = kBlock >> 6;
+    constexpr int nw = BT >> 6;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
     for (int q = 0; q < NV; ++q) v[q] = wave_sum(v[q]);

@@ -438,6 +438,126 @@ __global__ __launch_bounds__((ZyfShape<NJ, NL>::BT)) void k_zyf(Dims d, ProArgs 
     }
 }
 
+// ZYF for planes of at most 2^11 cells: both parities of the z and of the y
+// frequencies at once, 2 n_j z lines and then 4 n_l y lines in LDS (66 KB at
+// most), where k_zyf runs them one after another.  The short chain is what
+// counts here: these planes give a block little work and a launch few blocks
+// (zyf_launch has the rule and the figures).
+template <int NJ, int NL>
+struct ZyfwShape {
+    static constexpr int NP = NJ * NL;
+    static constexpr int BT = NP / 4 < 256 ? 256 : NP / 4;
+    static constexpr int LSZ = NL + kLpad, LSY = NJ + kLpad;
+    static constexpr int WORDS = 2 * NJ * LSZ > 4 * NL * LSY ? 2 * NJ * LSZ : 4 * NL * LSY;
+    static constexpr int E = (NP + BT - 1) / BT;   // cells per thread
+    static_assert(BT <= 512, "planes of at most 2^11 cells");
+};
+
+template <int NJ, int NL>
+__global__ __launch_bounds__((ZyfwShape<NJ, NL>::BT)) void k_zyf_wide(
+    Dims d, ProArgs pa, const SolveState* __restrict__ st, const int8_t* __restrict__ dipf, float2* __restrict__ b2,
+    const float2* __restrict__ wpre_l, const float2* __restrict__ tw_l, const float2* __restrict__ wpre_j,
+    const float2* __restrict__ tw_j) {
+    using S = ZyfwShape<NJ, NL>;
+    constexpr int E = S::E, LSZ = S::LSZ, LSY = S::LSY, BT = S::BT, NP = S::NP;
+    constexpr int LNL = ilog2c(NL), LNJ = ilog2c(NJ), NL2 = 2 * NL;
+    __shared__ float2 s[S::WORDS];
+    __shared__ float2 stl[NL], stj[NJ];
+    const int i = blockIdx.x, c = blockIdx.y, rhs = c / 3;
+    float2 c1 = make_float2(0.f, 0.f), c2 = c1;
+    int snap = 0;
+    if (st) {
+        if (st[rhs].it >= st[rhs].stop_at) return;
+        c1 = st[rhs].pro_c1;
+        c2 = st[rhs].pro_c2;
+        snap = (pa.Pmin != nullptr && pa.P != nullptr) ? st[rhs].snapshot : 0;
+    }
+    const long long cell0 = (long long)i * NP, cb = (long long)c * d.n + cell0;
+    for (int f = threadIdx.x; f < NL; f += BT) stl[f] = tw_l[f];
+    for (int f = threadIdx.x; f < NJ; f += BT) stj[f] = tw_j[f];
+    {
+        const int mode = pa.mode;
+        bool dip[E];
+        float2 va[E], vb[E], vd[E], vp[E];
+        auto operands = [&](int k, int f, bool on) {
+            va[k] = vb[k] = vd[k] = vp[k] = make_float2(0.f, 0.f);
+            if ((NP % BT == 0 || f < NP) && on) {
+                va[k] = pa.A[cb + f];
+                if (mode != PRO_COPY) vb[k] = pa.B[cb + f];
+                if (mode == PRO_LC4) vd[k] = pa.D[cb + f];
+                if (snap) vp[k] = pa.P[cb + f];
+            }
+        };
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            const int f = threadIdx.x + k * BT;
+            dip[k] = !st || ((NP % BT == 0 || f < NP) && dipf[cell0 + f] != 0);
+        }
+        if (small_launch(d)) {
+#pragma unroll
+            for (int k = 0; k < E; ++k) operands(k, threadIdx.x + k * BT, true);
+        } else {
+#pragma unroll
+            for (int k = 0; k < E; ++k) operands(k, threadIdx.x + k * BT, dip[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            const int f = threadIdx.x + k * BT;
+            if (NP % BT == 0 || f < NP) {
+                const float2 v = prologue(mode, dip[k], c1, c2, va[k], vb[k], vd[k], pa, cb + f);
+                if (snap && dip[k]) pa.Pmin[cb + f] = vp[k];
+                const int j = f >> LNL, l = f & (NL - 1);
+                s[j * LSZ + l] = v;
+                s[(NJ + j) * LSZ + l] = cmul(wpre_l[l], v);
+            }
+        }
+    }
+    __syncthreads();
+    fft_lds_fixed<NL, 2 * NJ, LSZ, BT>(s, stl);
+    {
+        constexpr int U = (2 * NP + BT - 1) / BT;
+        float2 u[U];   // column L' = p n_l + lh at row j: element f = L' n_j + j
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+            const int f = threadIdx.x + q * BT;
+            if ((2 * NP) % BT == 0 || f < 2 * NP) {
+                const int Lp = f >> LNJ, j = f & (NJ - 1);
+                u[q] = s[((Lp >> LNL) * NJ + j) * LSZ + (Lp & (NL - 1))];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+            const int f = threadIdx.x + q * BT;
+            if ((2 * NP) % BT == 0 || f < 2 * NP) {
+                const int Lp = f >> LNJ, j = f & (NJ - 1);
+                s[Lp * LSY + j] = u[q];
+                s[(NL2 + Lp) * LSY + j] = cmul(wpre_j[j], u[q]);
+            }
+        }
+    }
+    __syncthreads();
+    // row J = 2 jh + q of plane (c, i) of B2 [C][J][i][L'], q = line / (2 n_l)
+    float2* dst = b2 + ((long long)c * (2 * NJ) * d.ni + i) * NL2;
+    const int rowj = d.ni * NL2;
+    if constexpr (Plan<NJ>::NST >= 2) {
+        fft_lds_fixed<NJ, 4 * NL, LSY, BT, Plan<NJ>::NST - 1>(s, stj);
+        fft_last_stage_out<NJ, 4 * NL, LSY, NJ, BT>(s, stj, [&](int line, int k, float2 v) {
+            dst[(2 * k + (line >= NL2 ? 1 : 0)) * rowj + (line & (NL2 - 1))] = v;
+        });
+    } else {
+        fft_lds_fixed<NJ, 4 * NL, LSY, BT>(s, stj);
+#pragma unroll
+        for (int q = 0; q < (4 * NP + BT - 1) / BT; ++q) {
+            const int f = threadIdx.x + q * BT;
+            if ((4 * NP) % BT == 0 || f < 4 * NP) {
+                const int Lp = f & (NL2 - 1), J = f / NL2;
+                dst[J * rowj + Lp] = s[((J & 1) * NL2 + Lp) * LSY + (J >> 1)];
+            }
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // YF: lines (c, i, L') along j; n_j -> 2 n_j.  A tile: consecutive L' of one
 // i-plane, written as runs of L' in each row J of B2.
@@ -1197,6 +1317,219 @@ __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ 
         tile(std::integral_constant<int, TJ>{});
     else
         tile(d.nj);
+}
+
+// ---------------------------------------------------------------------------
+// YZI: the y- and z-inverse passes of one (c, i) plane in one block, with the
+// epilogue, for planes of at most 2^13 padded cells (the counterpart of ZYF).
+// The lines along J are transformed in LDS as in YI (first stage from the
+// loads, last stage in registers), the kept rows j go back to LDS in natural
+// L order once every thread has read its last-stage inputs, and the lines
+// along L are transformed and finished there as in ZI: the same butterflies,
+// twiddles and order, the same bits.  B4 is not touched.  A block holds one
+// component, so the epilogues with sums over a cell's three components
+// (one_component() false) take YI + ZI.
+// ---------------------------------------------------------------------------
+
+__host__ __device__ constexpr bool one_component(int kind) {
+    return kind != EK_CG_R0 && kind != EK_AA_S0 && kind != EK_SIM_R0 && kind != EK_SIM;
+}
+
+template <int NJ, int NL>
+struct YziShape {
+    static constexpr int NJ2 = 2 * NJ, NL2 = 2 * NL;
+    static constexpr int BT = NJ2 * NL2 / 16 < 256 ? 256 : NJ2 * NL2 / 16;   // up to 16 points per thread
+    static constexpr int LSY = NJ2 + kLpad, LSZ = NL2 + kLpad;               // y / z line strides
+    static constexpr int WORDS = NL2 * LSY > NJ * LSZ ? NL2 * LSY : NJ * LSZ;
+    static_assert(BT <= 512, "planes of at most 2^13 padded cells");
+};
+
+template <int NJ, int NL>
+__global__ __launch_bounds__((YziShape<NJ, NL>::BT)) void k_yzi(Dims d, const SolveState* __restrict__ st,
+                                                                const int2* __restrict__ rows,
+                                                                const float2* __restrict__ b3, EpiArgs ea,
+                                                                const int8_t* __restrict__ occ,
+                                                                const int8_t* __restrict__ dipf,
+                                                                const float2* __restrict__ twj,
+                                                                const float2* __restrict__ twl) {
+    using S = YziShape<NJ, NL>;
+    constexpr int NJ2 = S::NJ2, NL2 = S::NL2, BT = S::BT, LSY = S::LSY, LSZ = S::LSZ;
+    constexpr int NP = NJ * NL, NEP = (NP + BT - 1) / BT, LNL = ilog2c(NL);
+    __shared__ float2 s[S::WORDS];
+    __shared__ float2 stj[NJ2], stl[NL2];
+    __shared__ double red[kSlots * 16];
+    const int i = blockIdx.x, c = blockIdx.y, rhs = c / 3, comp = c - 3 * rhs;
+    const int2 jr = row_range(d, st, rows, i);
+    if (stopped(st, rhs, jr)) return;
+    double* part = ea.partials ? ea.partials + ((long long)(rhs * 3 + comp) * d.ni + i) * kSlots : nullptr;
+    if (jr.x >= jr.y) {   // a plane without dipoles
+        if (part && threadIdx.x < kSlots) part[threadIdx.x] = 0.0;
+        return;
+    }
+    const float rB = st ? st[rhs].rB : 0.f;
+    const float2* src = b3 + ((long long)c * NJ2 * d.ni + i) * NL2;
+    const int rowj = d.ni * NL2;
+    constexpr int NSTJ = Plan<NJ2>::NST, R0 = plan_radix(Plan<NJ2>::K, 0), NB0 = NJ2 / R0;
+    constexpr int NITEM = NL2 * NB0, IPT = (NITEM + BT - 1) / BT;
+    static_assert(NSTJ >= 2, "J lines of at least two stages");
+    float2 xv[IPT][R0];
+#pragma unroll
+    for (int it = 0; it < IPT; ++it) {
+        const int f = threadIdx.x + it * BT;
+        if (NITEM % BT == 0 || f < NITEM) {
+            const int t = f % NL2, j0 = rest_natural<NJ2>(f / NL2);
+#pragma unroll
+            for (int q = 0; q < R0; ++q) xv[it][q] = src[(q * NB0 + j0) * rowj + t];
+        }
+    }
+    // the epilogue's operands: before the transforms where the launch waits for
+    // latency, else behind them, on dipole cells
+    const int kind = ea.kind;
+    const bool need_x = kind != EK_CONV && kind != EK_BICG_R0 && kind != EK_AA_R0;
+    const bool need_y = kind == EK_BICG_H || kind == EK_CG_W, need_o2 = kind == EK_AA_SUPD;
+    const float2* al = ea.alpha + (long long)rhs * ea.nmat;
+    const long long k0 = (long long)i * NP, ck0 = (long long)c * d.n + k0;
+    bool dip[NEP];
+    float2 a[NEP], xr[NEP], yr[NEP], o2[NEP];
+    auto operands = [&](bool everywhere) {
+#pragma unroll
+        for (int q = 0; q < NEP; ++q) {
+            const int f = threadIdx.x + q * BT;
+            dip[q] = false;
+            a[q] = xr[q] = yr[q] = o2[q] = make_float2(0.f, 0.f);
+            if (NP % BT == 0 || f < NP) {
+                dip[q] = dipf[k0 + f] != 0;
+                a[q] = al[occ[k0 + f]];
+                if (everywhere || dip[q]) {
+                    if (need_x) xr[q] = ea.x[ck0 + f];
+                    if (need_y) yr[q] = ea.y[ck0 + f];
+                    if (need_o2) o2[q] = ea.out2[ck0 + f];
+                }
+            }
+        }
+    };
+    const bool early = small_launch(d);
+    if (early) operands(true);
+    for (int f = threadIdx.x; f < NJ2; f += BT) stj[f] = twj[f];
+    for (int f = threadIdx.x; f < NL2; f += BT) stl[f] = twl[f];
+#pragma unroll
+    for (int it = 0; it < IPT; ++it) {
+        const int f = threadIdx.x + it * BT;
+        if (NITEM % BT == 0 || f < NITEM) {
+            butterfly<R0>(xv[it]);
+            float2* v = s + (f % NL2) * LSY + (f / NL2) * R0;
+#pragma unroll
+            for (int q = 0; q < R0; ++q) v[q] = xv[it][q];
+        }
+    }
+    __syncthreads();
+    FixedStage<NJ2, NL2, LSY, 1, BT, NSTJ - 1>::run(s, stj);
+    {
+        constexpr int RL = plan_radix(Plan<NJ2>::K, NSTJ - 1), HL = NJ2 / RL;   // span NJ2, step 1
+        constexpr int WL = NL2 * HL, ITL = (WL + BT - 1) / BT;
+        float2 keep[ITL][RL / 2];   // outputs bf + q HL < n_j: the first half
+#pragma unroll
+        for (int it = 0; it < ITL; ++it) {
+            const int f = threadIdx.x + it * BT;
+            if (WL % BT == 0 || f < WL) {
+                const int bf = f / NL2;
+                const float2* v = s + (f % NL2) * LSY + bf;
+                float2 z[RL];
+#pragma unroll
+                for (int q = 0; q < RL; ++q) z[q] = v[q * HL];
+                if (RL > 2 && bf > 0) {
+                    int tq = 0;
+#pragma unroll
+                    for (int q = 1; q < RL; ++q) {
+                        tq += bf;
+                        const float2 tv = stj[tq];
+                        const float tr = z[q].x * tv.x - z[q].y * tv.y;
+                        z[q].y = z[q].x * tv.y + z[q].y * tv.x;
+                        z[q].x = tr;
+                    }
+                }
+                butterfly<RL>(z);
+#pragma unroll
+                for (int q = 0; q < RL / 2; ++q) keep[it][q] = z[q];
+            }
+        }
+        __syncthreads();   // every last-stage input has been read: the rows j take their place
+#pragma unroll
+        for (int it = 0; it < ITL; ++it) {
+            const int f = threadIdx.x + it * BT;
+            if (WL % BT == 0 || f < WL) {
+                const int Lp = f % NL2, bf = f / NL2;
+                float2* v = s + bf * LSZ + (Lp < NL ? 2 * Lp : 2 * (Lp - NL) + 1);
+#pragma unroll
+                for (int q = 0; q < RL / 2; ++q) v[q * HL * LSZ] = keep[it][q];
+            }
+        }
+    }
+    __syncthreads();
+    fft_lds_fixed<NL2, NJ, LSZ, BT>(s, stl);
+    if (!early) operands(!st);
+    double acc[kSlots] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < NEP; ++q) {
+        const int f = threadIdx.x + q * BT;
+        if ((NP % BT != 0 && f >= NP) || !(dip[q] || !st)) continue;
+        float2 av = a[q];
+        if (ea.conj) av.y = -av.y;
+        const float2 cv = cconj(s[(f >> LNL) * LSZ + (f & (NL - 1))]);
+        const float2 x = xr[q];
+        const long long ck = ck0 + f;
+        switch (kind) {   // as in k_zi
+            case EK_CONV:
+                ea.out[ck] = cv;
+                break;
+            case EK_MV:
+                ea.out[ck] = dip[q] ? csub(x, cmul(av, cv)) : make_float2(0.f, 0.f);
+                break;
+            case EK_BICG_H:
+            case EK_BICG_W:
+            case EK_CG_W:
+            case EK_AA_W: {
+                const float2 o = csub(x, cmul(av, cv));
+                ea.out[ck] = o;
+                if (kind == EK_BICG_H) dot_acc(yr[q], o, acc[0], acc[1]);
+                if (kind == EK_BICG_W) {
+                    dot_acc(o, x, acc[0], acc[1]);
+                    dot_acc(o, o, acc[2], acc[3]);
+                }
+                if (kind == EK_CG_W) {
+                    dot_acc(x, o, acc[0], acc[1]);
+                    dot_acc(yr[q], x, acc[2], acc[3]);
+                }
+                if (kind == EK_AA_W) acc[4] += norm_term(x);
+                break;
+            }
+            case EK_BICG_R0:
+            case EK_AA_R0: {
+                const float2 o = cneg(cmul(av, cv));
+                ea.out[ck] = o;
+                if (kind == EK_BICG_R0) {
+                    ea.out2[ck] = o;
+                    ea.out3[ck] = o;
+                    dot_acc(o, o, acc[0], acc[1]);
+                } else {
+                    acc[4] += norm_term(o);
+                }
+                break;
+            }
+            case EK_AA_SUPD:
+                ea.out2[ck] = cadd(csub(x, cmul(av, cv)), rmul(rB, o2[q]));
+                break;
+            default:
+                break;
+        }
+    }
+    if (part) {
+        block_sum<kSlots, BT>(acc, red);
+        if (threadIdx.x == 0) {
+#pragma unroll
+            for (int q = 0; q < kSlots; ++q) part[q] = acc[q];
+        }
+    }
 }
 
 }  // namespace ddafft

@@ -168,8 +168,10 @@ int ddafft_set_ahat_mode(ddafft_ctx* ctx, int mode);
 #define DDAFFT_TUNE_X_RB 1
 #define DDAFFT_TUNE_GRAPH 2
 /* DDAFFT_TUNE_FUSE_ZY: 1 runs the z- and y-forward transforms of one
- * i-plane in one kernel where n_j, n_l <= 64, 0 always as two passes, -1
- * (default) as the table says. */
+ * i-plane in one kernel where n_j n_l <= 2048 (axes of 8 to 256) or n_j = n_l
+ * = 64, and the y- and z-inverse ones with the epilogue where n_j n_l <= 2048;
+ * 0 always as two passes each, -1 (default) as the table says, and fused where
+ * n_j n_l <= 2048. */
 #define DDAFFT_TUNE_FUSE_ZY 3
 /* DDAFFT_TUNE_FF_MFMA: 1 sums the far field (FP64-summed mode) on the matrix
  * cores, 16 directions per block, where the phase rows fit (ni + nj + nl <=
