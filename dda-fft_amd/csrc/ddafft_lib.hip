@@ -184,7 +184,9 @@ struct ddafft_ctx {
     const float2 *tw_i = nullptr, *tw_j = nullptr, *tw_l = nullptr;      // n-point plans
     const float2 *tw_2i = nullptr, *tw_2j = nullptr, *tw_2l = nullptr;   // 2n-point plans
 
-    // target
+    // target: one device block that the pointers below point into
+    char* target = nullptr;
+    size_t target_cap = 0;
     int8_t* occ = nullptr;
     int8_t* dipf = nullptr;            // [n] 1 where the cell holds a dipole (mv[occ] != 0)
     int2* rows = nullptr;              // [ni] the rows j of plane i that its dipoles span, [x, y) (0, 0: none)
@@ -1018,10 +1020,10 @@ int ddafft_host_free(void* p) {
 int ddafft_destroy(ddafft_ctx* c) {
     if (!c) return DDAFFT_OK;
     if (c->stream) hipStreamSynchronize(c->stream);
-    void* bufs[] = {c->ahat, c->tables, c->occ, c->dipf, c->rows, c->mv, c->cells, c->b1, c->b2, c->b3, c->P, c->Pmin, c->R,
+    void* bufs[] = {c->ahat, c->tables, c->target, c->b1, c->b2, c->b3, c->P, c->Pmin, c->R,
                     c->S, c->G, c->H, c->W, c->X, c->Y, c->small, c->hist, c->partials,
                     c->dirs, c->esc, c->fftab, c->Pf, c->phase, c->gaux, c->inc_cell, c->seqbuf,
-                    c->ffcol, c->ffpiece, c->ffseg, c->ffpc};
+                    c->ffseg, c->ffpc};
     for (void* b : bufs)
         if (b) hipFree(b);
     if (c->state_ring) hipHostFree(c->state_ring);
@@ -1083,15 +1085,16 @@ int ddafft_create(int ni, int nj, int nl, float kd, int nrhs_max, ddafft_ctx** o
     for (float2** f : fields)
         if (!rc) rc = dev_alloc(f, (size_t)(n * C));
     if (!rc) rc = small_layout(c);
-    if (!rc) rc = dev_alloc(&c->occ, (size_t)n);
-    if (!rc) rc = dev_alloc(&c->dipf, (size_t)n);
-    if (!rc) rc = dev_alloc(&c->rows, (size_t)ni);
     if (!rc && hipHostMalloc((void**)&c->state_ring, (size_t)4 * nrhs_max * sizeof(SolveState),
                              hipHostMallocDefault) != hipSuccess)
         rc = fail(DDAFFT_ENOMEM, "hipHostMalloc");
     if (!rc && hipHostGetDevicePointer((void**)&c->ring_dev, c->state_ring, 0) != hipSuccess)
         rc = fail(DDAFFT_EHIP, "hipHostGetDevicePointer of the state ring");
-    if (!rc) rc = ensure_partials(c, (size_t)nrhs_max * std::max<long long>(max_epi_blocks(c->d), 1024) * kSlots);
+    // at least 512 KB: room for the far field's partial sums of most direction
+    // sets, which would otherwise be allocated by the first solve
+    if (!rc)
+        rc = ensure_partials(c, std::max<size_t>((size_t)nrhs_max * std::max<long long>(max_epi_blocks(c->d), 1024) * kSlots,
+                                                 (size_t)1 << 16));
     if (rc) {
         ddafft_destroy(c);
         return rc;
@@ -1221,39 +1224,53 @@ int ddafft_set_target(ddafft_ctx* c, const signed char* occ, int nmat, const int
     }
     const int npiece = (int)fpiece.size();
     while (fpiece.size() % kFFWaves) fpiece.push_back(make_int2(0, 0));
+    c->dipf_h.assign((size_t)n, 0);
+    for (const int k : cells) c->dipf_h[(size_t)k] = 1;
+    // one device block and one copy for all of it; the pieces that a captured
+    // iteration reads lie at offsets that depend on the lattice only
+    std::vector<char> blk;
+    auto put = [&](const void* src, size_t bytes, size_t room) {
+        const size_t at = blk.size();
+        blk.resize((at + room + 255) & ~(size_t)255);
+        std::memcpy(blk.data() + at, src, bytes);
+        return at;
+    };
+    const size_t o_occ = put(occ, (size_t)n, (size_t)n);
+    const size_t o_dip = put(c->dipf_h.data(), (size_t)n, (size_t)n);
+    const size_t o_row = put(rows.data(), rows.size() * sizeof(int2), rows.size() * sizeof(int2));
+    const size_t o_mv = put(mv, (size_t)nmat * sizeof(int), 128 * sizeof(int));
+    const size_t o_cell = put(cells.data(), cells.size() * sizeof(int), cells.size() * sizeof(int));
+    const size_t o_col = put(fcol.data(), fcol.size() * sizeof(int), fcol.size() * sizeof(int));
+    const size_t o_pc = put(fpiece.data(), fpiece.size() * sizeof(int2), fpiece.size() * sizeof(int2));
     HIPCHECK(hipStreamSynchronize(c->stream));
-    if (c->mv) hipFree(c->mv);
-    if (c->cells) hipFree(c->cells);
-    if (c->ffcol) hipFree(c->ffcol);
-    if (c->ffpiece) hipFree(c->ffpiece);
     if (c->ffseg) hipFree(c->ffseg);
-    c->mv = nullptr;
-    c->cells = nullptr;
-    c->ffcol = nullptr;
-    c->ffpiece = nullptr;
     c->ffseg = nullptr;
     c->nffpiece = c->nseg = 0;
-    int rc = dev_alloc(&c->mv, (size_t)nmat);
-    if (!rc) rc = dev_alloc(&c->cells, cells.size());
-    if (!rc) rc = dev_alloc(&c->ffcol, fcol.size());
-    if (!rc) rc = dev_alloc(&c->ffpiece, fpiece.size());
-    if (rc) return rc;
+    if (blk.size() > c->target_cap) {
+        if (c->target) hipFree(c->target);
+        c->target = nullptr;
+        c->target_cap = 0;
+        c->occ = c->dipf = nullptr;
+        c->rows = nullptr;
+        c->mv = nullptr;
+        TRY(dev_alloc(&c->target, blk.size()));
+        c->target_cap = blk.size();
+    }
+    HIPCHECK(hipMemcpyAsync(c->target, blk.data(), blk.size(), hipMemcpyHostToDevice, c->stream));
+    HIPCHECK(hipStreamSynchronize(c->stream));
+    c->occ = reinterpret_cast<int8_t*>(c->target + o_occ);
+    c->dipf = reinterpret_cast<int8_t*>(c->target + o_dip);
+    c->rows = reinterpret_cast<int2*>(c->target + o_row);
+    c->mv = reinterpret_cast<int*>(c->target + o_mv);
+    c->cells = reinterpret_cast<int*>(c->target + o_cell);
+    c->ffcol = reinterpret_cast<int*>(c->target + o_col);
+    c->ffpiece = reinterpret_cast<int2*>(c->target + o_pc);
     c->nmat = nmat;
     c->mat_count.assign(nmat, 0);
-    for (long long k = 0; k < n; ++k) c->mat_count[occ[k]] += mv[occ[k]] ? 1 : 0;
+    for (const int k : cells) c->mat_count[occ[k]]++;
     c->ncells = (int)cells.size();
     c->ndip = (long long)cells.size();
-    if ((rc = upload(c, c->occ, occ, (size_t)n))) return rc;
-    c->dipf_h.assign((size_t)n, 0);
-    for (long long k = 0; k < n; ++k) c->dipf_h[k] = mv[occ[k]] ? 1 : 0;
-    if ((rc = upload(c, c->dipf, c->dipf_h.data(), (size_t)n))) return rc;
-    if ((rc = upload(c, c->rows, rows.data(), rows.size() * sizeof(int2)))) return rc;
-    if ((rc = upload(c, c->mv, mv, (size_t)nmat * sizeof(int)))) return rc;
-    if ((rc = upload(c, c->cells, cells.data(), cells.size() * sizeof(int)))) return rc;
-    if ((rc = upload(c, c->ffcol, fcol.data(), fcol.size() * sizeof(int)))) return rc;
-    if ((rc = upload(c, c->ffpiece, fpiece.data(), fpiece.size() * sizeof(int2)))) return rc;
     c->nffpiece = npiece;
-    HIPCHECK(hipStreamSynchronize(c->stream));
     c->have_target = true;
     return DDAFFT_OK;
 }

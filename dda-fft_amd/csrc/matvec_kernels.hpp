@@ -446,7 +446,7 @@ __global__ __launch_bounds__((ZyfShape<NJ, NL>::BT)) void k_zyf(Dims d, ProArgs 
 template <int NJ, int NL>
 struct ZyfwShape {
     static constexpr int NP = NJ * NL;
-    static constexpr int BT = NP / 4 < 256 ? 256 : NP / 4;
+    static constexpr int BT = NP / 2 < 256 ? 256 : NP / 2 > 512 ? 512 : NP / 2;
     static constexpr int LSZ = NL + kLpad, LSY = NJ + kLpad;
     static constexpr int WORDS = 2 * NJ * LSZ > 4 * NL * LSY ? 2 * NJ * LSZ : 4 * NL * LSY;
     static constexpr int E = (NP + BT - 1) / BT;   // cells per thread
@@ -1335,10 +1335,13 @@ __host__ __device__ constexpr bool one_component(int kind) {
     return kind != EK_CG_R0 && kind != EK_AA_S0 && kind != EK_SIM_R0 && kind != EK_SIM;
 }
 
+// Threads: 8 padded points each, at least 256 and at most 512 (32 x 32 planes,
+// one or two RHS: CG step 44.4 -> 43.1 and 45.4 -> 41.8 us against 16 points;
+// 32 x 64 planes with 1024 threads lost, 177 -> 185 us at 16 RHS).
 template <int NJ, int NL>
 struct YziShape {
     static constexpr int NJ2 = 2 * NJ, NL2 = 2 * NL;
-    static constexpr int BT = NJ2 * NL2 / 16 < 256 ? 256 : NJ2 * NL2 / 16;   // up to 16 points per thread
+    static constexpr int BT = NJ2 * NL2 / 8 < 256 ? 256 : NJ2 * NL2 / 8 > 512 ? 512 : NJ2 * NL2 / 8;
     static constexpr int LSY = NJ2 + kLpad, LSZ = NL2 + kLpad;               // y / z line strides
     static constexpr int WORDS = NL2 * LSY > NJ * LSZ ? NL2 * LSY : NJ * LSZ;
     static_assert(BT <= 512, "planes of at most 2^13 padded cells");
