@@ -591,14 +591,14 @@ int launch_matvec(ddafft_ctx* c, int nrhs, const ProArgs& pa, SolveState* st, in
     {
         const int tj = std::min(tile_zf(d.nl), d.nj);
         dim3 grid(d.ni * (d.nj / tj), C);
-        DDA_SWITCH_SMALL(d.nl, hipLaunchKernelGGL((k_zf<NN>), grid, kBlock, 0, s, d, pa, st, c->dipf, c->rows, c->b1, c->wpre_l,
+        DDA_SWITCH_SMALL(d.nl, hipLaunchKernelGGL((k_zf<NN>), grid, LineBlock<NN>::BT, 0, s, d, pa, st, c->dipf, c->rows, c->b1, c->wpre_l,
                                                                   c->tw_l));
     }
     if (ev) HIPCHECK(hipEventRecord(ev[1], s));
     {
         const int tl = std::min(tile_zf(d.nj), 2 * d.nl);   // L' lines per block
         dim3 grid(d.ni * (2 * d.nl / tl), C);
-        DDA_SWITCH_SMALL(d.nj, hipLaunchKernelGGL((k_yf<NN>), grid, kBlock, 0, s, d, st, c->rows, c->b1, c->b2, c->wpre_j, c->tw_j));
+        DDA_SWITCH_SMALL(d.nj, hipLaunchKernelGGL((k_yf<NN>), grid, LineBlock<NN>::BT, 0, s, d, st, c->rows, c->b1, c->b2, c->wpre_j, c->tw_j));
     }
     }
     if (ev) HIPCHECK(hipEventRecord(ev[2], s));
@@ -646,7 +646,7 @@ int launch_matvec(ddafft_ctx* c, int nrhs, const ProArgs& pa, SolveState* st, in
     {
         const int tl = std::min(tile_yi(2 * d.nj), 2 * d.nl);
         dim3 grid(d.ni * (2 * d.nl / tl), C);
-        DDA_SWITCH_LARGE(2 * d.nj, hipLaunchKernelGGL((k_yi<NN>), grid, kBlock, 0, s, d, st, c->rows, b3, c->b1, c->tw_2j));
+        DDA_SWITCH_LARGE(2 * d.nj, hipLaunchKernelGGL((k_yi<NN>), grid, LineBlock<NN / 2>::BT, 0, s, d, st, c->rows, b3, c->b1, c->tw_2j));
     }
     if (ev) HIPCHECK(hipEventRecord(ev[4], s));
     {

@@ -170,9 +170,9 @@ __device__ __forceinline__ void butterfly<8>(float2* z) { bf8(z); }
 
 struct LineWalk {
     int nlines, dq, dr, b0, l0;
-    __device__ __forceinline__ explicit LineWalk(int nl) : nlines(nl) {
-        dq = kBlock / nl;
-        dr = kBlock - dq * nl;
+    __device__ __forceinline__ explicit LineWalk(int nl, int bt = kBlock) : nlines(nl) {
+        dq = bt / nl;
+        dr = bt - dq * nl;
         b0 = (int)threadIdx.x / nl;
         l0 = (int)threadIdx.x - b0 * nl;
     }
@@ -406,19 +406,19 @@ __device__ __forceinline__ void fft_last_stage_out(const float2* s, const float2
 
 // MAXL: the most lines any call of this instance passes (sizes the registers
 // that carry stage 0 across its barrier); LS: the line stride in float2.
-// TWS: twiddle stride.  Ends with a __syncthreads.
-template <int N, int MAXL, int LS, int TWS = 1>
+// TWS: twiddle stride; BT: threads per block.  Ends with a __syncthreads.
+template <int N, int MAXL, int LS, int TWS = 1, int BT = kBlock>
 __device__ __forceinline__ void fft_lds(float2* s, int nlines, const float2* __restrict__ tw) {
     constexpr int ls = LS;
     if (nlines == MAXL) {   // the usual case: full tiles
-        fft_lds_fixed<N, MAXL, LS, kBlock, Plan<N>::NST, TWS>(s, tw);
+        fft_lds_fixed<N, MAXL, LS, BT, Plan<N>::NST, TWS>(s, tw);
         return;
     }
     constexpr int K = Plan<N>::K;
     constexpr int R0 = plan_radix(K, 0);
     constexpr int NB0 = N / R0;
-    constexpr int ITEMS = (MAXL * NB0 + kBlock - 1) / kBlock;
-    const LineWalk w(nlines);
+    constexpr int ITEMS = (MAXL * NB0 + BT - 1) / BT;
+    const LineWalk w(nlines, BT);
     // stage 0: gather in digit-reversed order (no twiddles: i = 0 throughout)
     float2 z[ITEMS][R0];
     int bb[ITEMS], ll[ITEMS];

@@ -48,7 +48,16 @@ namespace ddafft {
 // 530 at 2); 32^3 keeps 4 (13.2 us, 13.8 at 8); 256-point lines keep two,
 // so that the 384 butterflies of a stage fill the block's threads evenly
 // (256^3, 2 RHS: 7.16 ms at one column, 6.66 at two).
-template <int N> struct TileZF { static constexpr int T = clamp16(pow2floor(6144 / (2 * (N + kLpad)))); };
+// The z and y passes of 256-point and longer lines (2 n = 512 for the inverse
+// ones) run 512 threads, and so keep whole 128-byte runs of 16 (512-point
+// lines: 64-byte runs of 8) with 16 waves per CU.  Against 256 threads and half
+// the lines, 256^3, 2 RHS: ZF 613 -> 442 us, YF 1297 -> 910, YI 1320 -> 924;
+// 64x256x64: YI 93 -> 61 us; 32x512x32, 1 RHS: YF 32.5 -> 21.6, YI 55 -> 33.
+// (128-point lines with 512 threads: the same times.)
+template <int N> struct LineBlock { static constexpr int BT = N >= 256 ? 512 : kBlock; };   // N-point input lines
+template <int N> struct TileZF {
+    static constexpr int T = clamp16(pow2floor(LineBlock<N>::BT / kBlock * 6144 / (2 * (N + kLpad))));
+};
 // Four right-hand sides per tile take half as many columns as two, so the
 // tile's LDS and its transforms stay those of the two-right-hand-side tile
 // while each Â value serves twice the right-hand sides.
@@ -104,7 +113,9 @@ template <> struct LaneGroup<128, 12, 131, 2> { static constexpr int G = 32; };
 // 22.7 us per launch (64^3, 2 RHS).
 template <int NL2, int T> struct ZStride { static constexpr int S = NL2 + kLpad; };
 template <> struct ZStride<128, 4> { static constexpr int S = 131; };
-template <int N> struct TileYI { static constexpr int T = clamp16(pow2floor(6144 / (N + kLpad))); };
+template <int N> struct TileYI {
+    static constexpr int T = clamp16(pow2floor(LineBlock<N / 2>::BT / kBlock * 6144 / (N + kLpad)));
+};
 // The Z-inverse pass runs the solver epilogue as well; at most four (i, j)
 // rows per block keeps more blocks in flight (64^3: 16.0 vs 17.1 us at 2 RHS,
 // 78.6 vs 87.1 us at 16; 32^3: 8.0 vs 9.9 us at 2 RHS).
@@ -190,14 +201,15 @@ __device__ __forceinline__ float2 prologue(int mode, bool dip, float2 c1, float2
 // ---------------------------------------------------------------------------
 
 template <int NL>
-__global__ __launch_bounds__(kBlock) void k_zf(Dims d, ProArgs pa, const SolveState* __restrict__ st,
+__global__ __launch_bounds__(LineBlock<NL>::BT) void k_zf(Dims d, ProArgs pa, const SolveState* __restrict__ st,
                                                const int8_t* __restrict__ dipf, const int2* __restrict__ rows,
                                                float2* __restrict__ b1,
                                                const float2* __restrict__ wpre, const float2* __restrict__ tw) {
+    constexpr int BT = LineBlock<NL>::BT;
     constexpr int TJ = TileZF<NL>::T;
     constexpr int LS = NL + kLpad;
     constexpr int LNL = ilog2c(NL);
-    constexpr int NLD = (TJ * NL + kBlock - 1) / kBlock;
+    constexpr int NLD = (TJ * NL + BT - 1) / BT;
     __shared__ float2 s[2 * TJ * LS];
     __shared__ float2 stw[NL];
     const int c = blockIdx.y, rhs = c / 3;
@@ -237,19 +249,19 @@ __global__ __launch_bounds__(kBlock) void k_zf(Dims d, ProArgs pa, const SolveSt
         };
 #pragma unroll
         for (int q = 0; q < NLD; ++q) {
-            const int f = threadIdx.x + q * kBlock;
+            const int f = threadIdx.x + q * BT;
             dip[q] = !st || (f < nld && dipf[cell0 + f] != 0);
         }
         if (small_launch(d)) {
 #pragma unroll
-            for (int q = 0; q < NLD; ++q) operands(q, threadIdx.x + q * kBlock, true);
+            for (int q = 0; q < NLD; ++q) operands(q, threadIdx.x + q * BT, true);
         } else {
 #pragma unroll
-            for (int q = 0; q < NLD; ++q) operands(q, threadIdx.x + q * kBlock, dip[q]);
+            for (int q = 0; q < NLD; ++q) operands(q, threadIdx.x + q * BT, dip[q]);
         }
 #pragma unroll
         for (int q = 0; q < NLD; ++q) {
-            const int f = threadIdx.x + q * kBlock;
+            const int f = threadIdx.x + q * BT;
             if (f < nld) {
                 const float2 v = prologue(mode, dip[q], c1, c2, va[q], vb[q], vd[q], pa, cb + f);
                 if (snap && dip[q]) pa.Pmin[cb + f] = vp[q];
@@ -258,28 +270,29 @@ __global__ __launch_bounds__(kBlock) void k_zf(Dims d, ProArgs pa, const SolveSt
                 s[(tj + t) * LS + l] = cmul(wpre[l], v);
             }
         }
-        for (int f = threadIdx.x; f < NL; f += kBlock) stw[f] = tw[f];
+        for (int f = threadIdx.x; f < NL; f += BT) stw[f] = tw[f];
         __syncthreads();
         float2* dst = b1 + ((long long)c * d.ni + i) * (2 * NL) * d.nj + j0;
         const int lnj = __builtin_ctz(d.nj);
         constexpr bool FULL = !std::is_same_v<decltype(tile_arg), int>;
-        if constexpr (FULL && Plan<NL>::NST >= 2 && NL <= 128) {
+        if constexpr (FULL && Plan<NL>::NST >= 2 && NL <= 256) {
             // the last stage in registers, stored straight to B1: row L' = k
             // of the line's output k (n_l + k for the pre-twiddled line)
-            // (64^3, 2 RHS: 14.6 -> 14.2 us; 128^3: 75.6 -> 72 us)
-            fft_lds_fixed<NL, 2 * TJ, LS, kBlock, Plan<NL>::NST - 1>(s, stw);
-            fft_last_stage_out<NL, 2 * TJ, LS, NL>(s, stw, [&](int line, int k, float2 v) {
+            // (64^3, 2 RHS: 14.6 -> 14.2 us; 128^3: 75.6 -> 72 us; 256^3: 442
+            // -> 422 us)
+            fft_lds_fixed<NL, 2 * TJ, LS, BT, Plan<NL>::NST - 1>(s, stw);
+            fft_last_stage_out<NL, 2 * TJ, LS, NL, BT>(s, stw, [&](int line, int k, float2 v) {
                 const bool odd = line >= TJ;
                 const int t = odd ? line - TJ : line;
                 if (j0 + t >= jr.x && j0 + t < jr.y) dst[((odd ? NL + k : k) << lnj) + t] = v;
             });
         } else {
-            fft_lds<NL, 2 * TJ, LS>(s, 2 * tj, stw);
+            fft_lds<NL, 2 * TJ, LS, 1, BT>(s, 2 * tj, stw);
             const int ltj = __builtin_ctz(tj);
-            constexpr int NST = (2 * NL * TJ + kBlock - 1) / kBlock;
+            constexpr int NST = (2 * NL * TJ + BT - 1) / BT;
 #pragma unroll
             for (int q = 0; q < NST; ++q) {
-                const int f = threadIdx.x + q * kBlock;
+                const int f = threadIdx.x + q * BT;
                 if (f < 2 * NL * tj) {   // row L' of B1: the even transform's outputs, then the odd one's
                     const int Lp = f >> ltj, t = f - (Lp << ltj);
                     const float2 v = Lp >= NL ? s[(tj + t) * LS + (Lp - NL)] : s[t * LS + Lp];
@@ -564,9 +577,10 @@ __global__ __launch_bounds__((ZyfwShape<NJ, NL>::BT)) void k_zyf_wide(
 // ---------------------------------------------------------------------------
 
 template <int NJ>
-__global__ __launch_bounds__(kBlock) void k_yf(Dims d, const SolveState* __restrict__ st,
+__global__ __launch_bounds__(LineBlock<NJ>::BT) void k_yf(Dims d, const SolveState* __restrict__ st,
                                                const int2* __restrict__ rows, const float2* __restrict__ b1, float2* __restrict__ b2,
                                                const float2* __restrict__ wpre, const float2* __restrict__ tw) {
+    constexpr int BT = LineBlock<NJ>::BT;
     constexpr int TI = TileZF<NJ>::T;
     constexpr int LS = NJ + kLpad;
     __shared__ float2 s[2 * TI * LS];
@@ -584,18 +598,18 @@ __global__ __launch_bounds__(kBlock) void k_yf(Dims d, const SolveState* __restr
         const int L0 = (blockIdx.x - i * nlt) * ti;
         const int lnl2 = __builtin_ctz(NL2), lti = __builtin_ctz(ti);
         {
-            constexpr int NLD = (TI * NJ + kBlock - 1) / kBlock;
+            constexpr int NLD = (TI * NJ + BT - 1) / BT;
             const float2* src = b1 + (((long long)c * d.ni + i) * NL2 + L0) * NJ;   // ti contiguous lines
             float2 v[NLD];
 #pragma unroll
             for (int q = 0; q < NLD; ++q) {
-                const int f = threadIdx.x + q * kBlock, jj = f & (NJ - 1);
+                const int f = threadIdx.x + q * BT, jj = f & (NJ - 1);
                 v[q] = make_float2(0.f, 0.f);
                 if (f < ti * NJ && jj >= jr.x && jj < jr.y) v[q] = src[f];
             }
 #pragma unroll
             for (int q = 0; q < NLD; ++q) {
-                const int f = threadIdx.x + q * kBlock;
+                const int f = threadIdx.x + q * BT;
                 if (f < ti * NJ) {
                     const int t = f >> LNJ, jj = f & (NJ - 1);
                     s[t * LS + jj] = v[q];
@@ -603,7 +617,7 @@ __global__ __launch_bounds__(kBlock) void k_yf(Dims d, const SolveState* __restr
                 }
             }
         }
-        for (int f = threadIdx.x; f < NJ; f += kBlock) stw[f] = tw[f];
+        for (int f = threadIdx.x; f < NJ; f += BT) stw[f] = tw[f];
         __syncthreads();
         // row J of plane (c, i) of B2 [C][J][i][L'], from L0
         float2* dst = b2 + ((long long)c * (2 * NJ) * d.ni + i) * NL2 + L0;
@@ -613,17 +627,17 @@ __global__ __launch_bounds__(kBlock) void k_yf(Dims d, const SolveState* __restr
             // the last stage in registers, stored straight to B2: row
             // J = 2 k (+1 for the pre-twiddled line) of output k (64^3, 2 RHS:
             // 16.3 -> 15.9 us; 256-point lines stay in LDS: 1270 -> 1315 us)
-            fft_lds_fixed<NJ, 2 * TI, LS, kBlock, Plan<NJ>::NST - 1>(s, stw);
-            fft_last_stage_out<NJ, 2 * TI, LS, NJ>(s, stw, [&](int line, int k, float2 v) {
+            fft_lds_fixed<NJ, 2 * TI, LS, BT, Plan<NJ>::NST - 1>(s, stw);
+            fft_last_stage_out<NJ, 2 * TI, LS, NJ, BT>(s, stw, [&](int line, int k, float2 v) {
                 const bool odd = line >= TI;
                 dst[(2 * k + (odd ? 1 : 0)) * rowj + (odd ? line - TI : line)] = v;
             });
         } else {
-            fft_lds<NJ, 2 * TI, LS>(s, 2 * ti, stw);
-            constexpr int NST = (2 * NJ * TI + kBlock - 1) / kBlock;
+            fft_lds<NJ, 2 * TI, LS, 1, BT>(s, 2 * ti, stw);
+            constexpr int NST = (2 * NJ * TI + BT - 1) / BT;
 #pragma unroll
             for (int q = 0; q < NST; ++q) {
-                const int f = threadIdx.x + q * kBlock;
+                const int f = threadIdx.x + q * BT;
                 if (f < 2 * NJ * ti) {
                     const int J = f >> lti, t = f - (J << lti);
                     const float2 v = (J & 1) ? s[(ti + t) * LS + (J >> 1)] : s[t * LS + (J >> 1)];
@@ -967,9 +981,10 @@ __global__ __launch_bounds__(kBlock) DDA_WAVES_PER_EU(XWaves<NI, RB, RUN, COMPAC
 // ---------------------------------------------------------------------------
 
 template <int NJ2>
-__global__ __launch_bounds__(kBlock) void k_yi(Dims d, const SolveState* __restrict__ st,
+__global__ __launch_bounds__(LineBlock<NJ2 / 2>::BT) void k_yi(Dims d, const SolveState* __restrict__ st,
                                                const int2* __restrict__ rows, const float2* __restrict__ b3, float2* __restrict__ b4,
                                                const float2* __restrict__ tw) {
+    constexpr int BT = LineBlock<NJ2 / 2>::BT;
     constexpr int TL = TileYI<NJ2>::T;
     constexpr int LS = NJ2 + kLpad;
     __shared__ float2 s[TL * LS];
@@ -999,22 +1014,22 @@ __global__ __launch_bounds__(kBlock) void k_yi(Dims d, const SolveState* __restr
             // butterflies and twiddles as the transform in LDS, with two LDS
             // round trips and a barrier fewer
             constexpr int R0 = plan_radix(Plan<NJ2>::K, 0), NB0 = NJ2 / R0;
-            constexpr int NITEM = TL * NB0, IPT = (NITEM + kBlock - 1) / kBlock;
+            constexpr int NITEM = TL * NB0, IPT = (NITEM + BT - 1) / BT;
             float2 xv[IPT][R0];
 #pragma unroll
             for (int it = 0; it < IPT; ++it) {
-                const int f = threadIdx.x + it * kBlock;
-                if (NITEM % kBlock == 0 || f < NITEM) {
+                const int f = threadIdx.x + it * BT;
+                if (NITEM % BT == 0 || f < NITEM) {
                     const int t = f % TL, bf = f / TL, j0 = rest_natural<NJ2>(bf);
 #pragma unroll
                     for (int q = 0; q < R0; ++q) xv[it][q] = src[(q * NB0 + j0) * rowj + t];
                 }
             }
-            for (int f = threadIdx.x; f < NJ2; f += kBlock) stw[f] = tw[f];
+            for (int f = threadIdx.x; f < NJ2; f += BT) stw[f] = tw[f];
 #pragma unroll
             for (int it = 0; it < IPT; ++it) {
-                const int f = threadIdx.x + it * kBlock;
-                if (NITEM % kBlock == 0 || f < NITEM) {
+                const int f = threadIdx.x + it * BT;
+                if (NITEM % BT == 0 || f < NITEM) {
                     const int t = f % TL, bf = f / TL;
                     butterfly<R0>(xv[it]);
                     float2* v = s + t * LS + bf * R0;
@@ -1023,38 +1038,38 @@ __global__ __launch_bounds__(kBlock) void k_yi(Dims d, const SolveState* __restr
                 }
             }
             __syncthreads();
-            FixedStage<NJ2, TL, LS, 1, kBlock, NSTJ - 1>::run(s, stw);
+            FixedStage<NJ2, TL, LS, 1, BT, NSTJ - 1>::run(s, stw);
             constexpr int NJ = NJ2 / 2;
             const int lnl2 = __builtin_ctz(NL2);
             float2* dst = b4 + (((long long)c * d.ni + i) * NJ) * NL2 + L0;
-            fft_last_stage_out<NJ2, TL, LS, NJ>(s, stw, [&](int t, int j, float2 v) {
+            fft_last_stage_out<NJ2, TL, LS, NJ, BT>(s, stw, [&](int t, int j, float2 v) {
                 if (j >= jr.x && j < jr.y) dst[(j << lnl2) + t] = v;
             });
         } else {
             {
-                constexpr int NLD = (TL * NJ2 + kBlock - 1) / kBlock;
+                constexpr int NLD = (TL * NJ2 + BT - 1) / BT;
                 float2 v[NLD];
 #pragma unroll
                 for (int q = 0; q < NLD; ++q) {
-                    const int f = threadIdx.x + q * kBlock;
+                    const int f = threadIdx.x + q * BT;
                     if (f < tl * NJ2) v[q] = src[(f >> ltl0) * rowj + (f & (tl - 1))];
                 }
 #pragma unroll
                 for (int q = 0; q < NLD; ++q) {
-                    const int f = threadIdx.x + q * kBlock;
+                    const int f = threadIdx.x + q * BT;
                     if (f < tl * NJ2) s[(f & (tl - 1)) * LS + (f >> ltl0)] = v[q];   // line t, point J
                 }
             }
-            for (int f = threadIdx.x; f < NJ2; f += kBlock) stw[f] = tw[f];
+            for (int f = threadIdx.x; f < NJ2; f += BT) stw[f] = tw[f];
             __syncthreads();
-            fft_lds<NJ2, TL, LS>(s, tl, stw);
+            fft_lds<NJ2, TL, LS, 1, BT>(s, tl, stw);
             constexpr int NJ = NJ2 / 2;
             const int ltl = __builtin_ctz(tl), lnl2 = __builtin_ctz(NL2);
             float2* dst = b4 + (((long long)c * d.ni + i) * NJ) * NL2 + L0;
-            constexpr int NST = (TL * NJ + kBlock - 1) / kBlock;
+            constexpr int NST = (TL * NJ + BT - 1) / BT;
 #pragma unroll
             for (int q = 0; q < NST; ++q) {
-                const int f = threadIdx.x + q * kBlock;
+                const int f = threadIdx.x + q * BT;
                 if (f < tl * NJ) {
                     const int j = f >> ltl, t = f - (j << ltl);
                     if (j >= jr.x && j < jr.y) dst[(j << lnl2) + t] = s[t * LS + j];
