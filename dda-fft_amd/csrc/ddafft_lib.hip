@@ -1175,41 +1175,46 @@ static constexpr long long kFFPieces = 2048;
 int ddafft_set_target(ddafft_ctx* c, const signed char* occ, int nmat, const int* mv) {
     if (!c || !occ || !mv || nmat < 1 || nmat > 128) return fail(DDAFFT_EINVAL, "bad target arguments");
     const long long n = c->d.n;
+    // one pass over the rows (i, j): the dipole cells, the rows that each
+    // plane's dipoles span, and the far-field columns: the (i, j) that hold
+    // dipoles and, for 8 of them at a time, the 16-point chunks of l that their
+    // dipoles span, cut into pieces
     std::vector<int> cells;
     cells.reserve((size_t)n);
-    for (long long k = 0; k < n; ++k) {
-        const int m = occ[k];
-        if (m < 0 || m >= nmat) return fail(DDAFFT_EINVAL, "occupancy index outside the material table");
-        if (mv[m]) cells.push_back((int)k);
-    }
-    if (cells.empty()) return fail(DDAFFT_EINVAL, "target has no dipoles");
-    // the rows that each plane's dipoles span
+    std::vector<int8_t> flags((size_t)n, 0);
+    long long count[128] = {0};
     std::vector<int2> rows((size_t)c->d.ni, make_int2(0, 0));
-    for (const int k : cells) {   // ascending along j within a plane
-        const int ij = k / c->d.nl, j = ij & (c->d.nj - 1);
-        int2& r = rows[ij / c->d.nj];
-        if (r.x == r.y) r.x = j;
-        r.y = j + 1;
-    }
-    // far-field columns: the (i, j) that hold dipoles, and 8 of them at a time
-    // the 16-point chunks of l that their dipoles span, cut into pieces
     std::vector<int> fcol;
     std::vector<int2> fpiece;
     {
-        const int lnl = __builtin_ctz(c->d.nl);
-        const int lnj = __builtin_ctz(c->d.nj);
         std::vector<std::pair<int, int>> span;   // chunks [lo, hi) of 8 columns of one plane i
-        for (const int k : cells) {
-            const int ij = k >> lnl, u = (k & (c->d.nl - 1)) >> 4;
-            if (fcol.empty() || fcol.back() != ij) {
-                if (!fcol.empty() && (fcol.back() >> lnj) != (ij >> lnj))
-                    fcol.resize((fcol.size() + kFFCols - 1) / kFFCols * kFFCols, -1);
-                if (fcol.size() % kFFCols == 0) span.emplace_back(u, u + 1);
-                fcol.push_back(ij);
+        const int nj = c->d.nj, nl = c->d.nl;
+        for (int ij = 0; ij < c->d.ni * nj; ++ij) {
+            const int k0 = ij * nl;
+            int first = -1, last = -1;
+            for (int l = 0; l < nl; ++l) {
+                const int m = occ[k0 + l];
+                if (m < 0 || m >= nmat) return fail(DDAFFT_EINVAL, "occupancy index outside the material table");
+                ++count[m];
+                if (!mv[m]) continue;
+                cells.push_back(k0 + l);
+                flags[(size_t)k0 + l] = 1;
+                if (first < 0) first = l;
+                last = l;
             }
-            span.back().first = std::min(span.back().first, u);
-            span.back().second = std::max(span.back().second, u + 1);
+            if (first < 0) continue;
+            const int i = ij / nj, j = ij - i * nj;
+            if (rows[i].x == rows[i].y) {   // the plane's first row with dipoles
+                rows[i].x = j;
+                fcol.resize((fcol.size() + kFFCols - 1) / kFFCols * kFFCols, -1);
+            }
+            rows[i].y = j + 1;
+            if (fcol.size() % kFFCols == 0) span.emplace_back(first >> 4, (last >> 4) + 1);
+            fcol.push_back(ij);
+            span.back().first = std::min(span.back().first, first >> 4);
+            span.back().second = std::max(span.back().second, (last >> 4) + 1);
         }
+        if (cells.empty()) return fail(DDAFFT_EINVAL, "target has no dipoles");
         fcol.resize((fcol.size() + kFFCols - 1) / kFFCols * kFFCols, -1);
         // a piece is short where there are few of them (parallelism) and long
         // where there are many (fewer T for stage 2): see kFFPieces
@@ -1224,19 +1229,22 @@ int ddafft_set_target(ddafft_ctx* c, const signed char* occ, int nmat, const int
     }
     const int npiece = (int)fpiece.size();
     while (fpiece.size() % kFFWaves) fpiece.push_back(make_int2(0, 0));
-    c->dipf_h.assign((size_t)n, 0);
-    for (const int k : cells) c->dipf_h[(size_t)k] = 1;
-    // one device block and one copy for all of it; the pieces that a captured
-    // iteration reads lie at offsets that depend on the lattice only
-    std::vector<char> blk;
+    // one device block for all of it; the pieces that a captured iteration
+    // reads lie at offsets that depend on the lattice only
+    struct Piece {
+        const void* src;
+        size_t bytes, at;
+    };
+    std::vector<Piece> pieces;
+    size_t total = 0;
     auto put = [&](const void* src, size_t bytes, size_t room) {
-        const size_t at = blk.size();
-        blk.resize((at + room + 255) & ~(size_t)255);
-        std::memcpy(blk.data() + at, src, bytes);
+        const size_t at = total;
+        pieces.push_back(Piece{src, bytes, at});
+        total = (at + room + 255) & ~(size_t)255;
         return at;
     };
     const size_t o_occ = put(occ, (size_t)n, (size_t)n);
-    const size_t o_dip = put(c->dipf_h.data(), (size_t)n, (size_t)n);
+    const size_t o_dip = put(flags.data(), (size_t)n, (size_t)n);
     const size_t o_row = put(rows.data(), rows.size() * sizeof(int2), rows.size() * sizeof(int2));
     const size_t o_mv = put(mv, (size_t)nmat * sizeof(int), 128 * sizeof(int));
     const size_t o_cell = put(cells.data(), cells.size() * sizeof(int), cells.size() * sizeof(int));
@@ -1246,18 +1254,29 @@ int ddafft_set_target(ddafft_ctx* c, const signed char* occ, int nmat, const int
     if (c->ffseg) hipFree(c->ffseg);
     c->ffseg = nullptr;
     c->nffpiece = c->nseg = 0;
-    if (blk.size() > c->target_cap) {
+    if (total > c->target_cap) {
         if (c->target) hipFree(c->target);
         c->target = nullptr;
         c->target_cap = 0;
         c->occ = c->dipf = nullptr;
         c->rows = nullptr;
         c->mv = nullptr;
-        TRY(dev_alloc(&c->target, blk.size()));
-        c->target_cap = blk.size();
+        TRY(dev_alloc(&c->target, total));
+        c->target_cap = total;
     }
-    HIPCHECK(hipMemcpyAsync(c->target, blk.data(), blk.size(), hipMemcpyHostToDevice, c->stream));
-    HIPCHECK(hipStreamSynchronize(c->stream));
+    // small targets in one copy (each costs more than its bytes), large ones
+    // piece by piece, without another pass over them
+    if (total <= (size_t)1 << 18) {
+        std::vector<char> blk(total);
+        for (const Piece& p : pieces) std::memcpy(blk.data() + p.at, p.src, p.bytes);
+        HIPCHECK(hipMemcpyAsync(c->target, blk.data(), total, hipMemcpyHostToDevice, c->stream));
+        HIPCHECK(hipStreamSynchronize(c->stream));
+    } else {
+        for (const Piece& p : pieces)
+            HIPCHECK(hipMemcpyAsync(c->target + p.at, p.src, p.bytes, hipMemcpyHostToDevice, c->stream));
+        HIPCHECK(hipStreamSynchronize(c->stream));
+    }
+    c->dipf_h.swap(flags);
     c->occ = reinterpret_cast<int8_t*>(c->target + o_occ);
     c->dipf = reinterpret_cast<int8_t*>(c->target + o_dip);
     c->rows = reinterpret_cast<int2*>(c->target + o_row);
@@ -1267,7 +1286,7 @@ int ddafft_set_target(ddafft_ctx* c, const signed char* occ, int nmat, const int
     c->ffpiece = reinterpret_cast<int2*>(c->target + o_pc);
     c->nmat = nmat;
     c->mat_count.assign(nmat, 0);
-    for (const int k : cells) c->mat_count[occ[k]]++;
+    for (int m = 0; m < nmat; ++m) c->mat_count[m] = mv[m] ? count[m] : 0;
     c->ncells = (int)cells.size();
     c->ndip = (long long)cells.size();
     c->nffpiece = npiece;
