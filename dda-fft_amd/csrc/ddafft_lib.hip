@@ -591,7 +591,7 @@ int launch_matvec(ddafft_ctx* c, int nrhs, const ProArgs& pa, SolveState* st, in
     {
         const int tj = std::min(tile_zf(d.nl), d.nj);
         dim3 grid(d.ni * (d.nj / tj), C);
-        DDA_SWITCH_SMALL(d.nl, hipLaunchKernelGGL((k_zf<NN>), grid, LineBlock<NN>::BT, 0, s, d, pa, st, c->dipf, c->rows, c->b1, c->wpre_l,
+        DDA_SWITCH_SMALL(d.nl, hipLaunchKernelGGL((k_zf<NN>), grid, ZBlock<NN>::BT, 0, s, d, pa, st, c->dipf, c->rows, c->b1, c->wpre_l,
                                                                   c->tw_l));
     }
     if (ev) HIPCHECK(hipEventRecord(ev[1], s));
@@ -651,8 +651,15 @@ int launch_matvec(ddafft_ctx* c, int nrhs, const ProArgs& pa, SolveState* st, in
     if (ev) HIPCHECK(hipEventRecord(ev[4], s));
     {
         dim3 grid(zi_blocks(d), nrhs);
-        DDA_SWITCH_LARGE(2 * d.nl, hipLaunchKernelGGL((k_zi<NN>), grid, kBlock, 0, s, d, st, c->b1, ea, c->occ, c->dipf, c->rows,
-                                                                      c->tw_2l));
+#define DDA_ZI(BT)                                                                                                   \
+    DDA_SWITCH_LARGE(2 * d.nl, hipLaunchKernelGGL((k_zi<NN, BT>), grid, BT, 0, s, d, st, c->b1, ea, c->occ, c->dipf, \
+                                                  c->rows, c->tw_2l))
+        if (small_launch(d)) {
+            DDA_ZI(ZBlock<NN / 2>::BT);
+        } else {
+            DDA_ZI(kBlock);
+        }
+#undef DDA_ZI
     }
     if (ev) HIPCHECK(hipEventRecord(ev[5], s));
     HIPCHECK(hipGetLastError());

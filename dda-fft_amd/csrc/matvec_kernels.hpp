@@ -55,6 +55,14 @@ namespace ddafft {
 // 64x256x64: YI 93 -> 61 us; 32x512x32, 1 RHS: YF 32.5 -> 21.6, YI 55 -> 33.
 // (128-point lines with 512 threads: the same times.)
 template <int N> struct LineBlock { static constexpr int BT = N >= 256 ? 512 : kBlock; };   // N-point input lines
+// The z passes run 512 threads from 128 points up, on the same tiles: a
+// block's chain of load, stages and store is half as long (ZF: 16x32x128, 2
+// RHS, 192 blocks 12.9 -> 10.8 us in a solve; 64x64x128 22.4 -> 20.4; 128^3
+// 97 -> 90; 256^3 even).  The inverse one only in small launches (below):
+// 16x32x128, 256 blocks 10.3 -> 9.5 us, but its epilogue's operands then
+// leave fewer waves per CU, and 128^3 and 256^3 lose (101 -> 115, 730 -> 893
+// us).  64-point lines, 6 points a thread, lose throughout.
+template <int N> struct ZBlock { static constexpr int BT = N >= 128 ? 512 : kBlock; };
 template <int N> struct TileZF {
     static constexpr int T = clamp16(pow2floor(LineBlock<N>::BT / kBlock * 6144 / (2 * (N + kLpad))));
 };
@@ -160,7 +168,7 @@ struct ProArgs {
 // against 5.6 us with the row range, ZF 5.4 against 6.0; 32x32x64, 16 RHS =
 // 2^20: ZYF 29.4 -> 26.2, ZI 21.0 -> 18.4, YI 14.6 -> 12.7 us by leaving them
 // out; 64^3, 2 RHS = 2^19: ZI 18.7 -> 17.4, the others even).
-__device__ __forceinline__ bool small_launch(const Dims& d) { return d.n * d.nrhs <= (1 << 18); }
+__host__ __device__ __forceinline__ bool small_launch(const Dims& d) { return d.n * d.nrhs <= (1 << 18); }
 
 // The range is requested together with the right-hand side's stopping state (its
 // use in stopped() keeps the load there): one wait for both.
@@ -201,11 +209,11 @@ __device__ __forceinline__ float2 prologue(int mode, bool dip, float2 c1, float2
 // ---------------------------------------------------------------------------
 
 template <int NL>
-__global__ __launch_bounds__(LineBlock<NL>::BT) void k_zf(Dims d, ProArgs pa, const SolveState* __restrict__ st,
+__global__ __launch_bounds__(ZBlock<NL>::BT) void k_zf(Dims d, ProArgs pa, const SolveState* __restrict__ st,
                                                const int8_t* __restrict__ dipf, const int2* __restrict__ rows,
                                                float2* __restrict__ b1,
                                                const float2* __restrict__ wpre, const float2* __restrict__ tw) {
-    constexpr int BT = LineBlock<NL>::BT;
+    constexpr int BT = ZBlock<NL>::BT;
     constexpr int TJ = TileZF<NL>::T;
     constexpr int LS = NL + kLpad;
     constexpr int LNL = ilog2c(NL);
@@ -1127,8 +1135,8 @@ __device__ __forceinline__ void dot_acc(float2 a, float2 b, double& re, double& 
 // ldScalMulConj / ldError term (dda_func.cpp:767-775, 796-805)
 __device__ __forceinline__ double norm_term(float2 a) { return (double)(a.x * a.x + a.y * a.y); }
 
-template <int NL2>
-__global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ st,
+template <int NL2, int BT>
+__global__ __launch_bounds__(BT) void k_zi(Dims d, SolveState* __restrict__ st,
                                                const float2* __restrict__ b4, EpiArgs ea,
                                                const int8_t* __restrict__ occ, const int8_t* __restrict__ dipf,
                                                const int2* __restrict__ rows, const float2* __restrict__ tw) {
@@ -1136,8 +1144,8 @@ __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ 
     constexpr int LS = ZStride<NL2, TJ>::S;
     constexpr int NLH = NL2 / 2;
     constexpr int LNL2 = ilog2c(NL2), LNLH = LNL2 - 1;
-    constexpr int NLD = (3 * TJ * NL2 + kBlock - 1) / kBlock;
-    constexpr int NEP = (TJ * NLH + kBlock - 1) / kBlock;
+    constexpr int NLD = (3 * TJ * NL2 + BT - 1) / BT;
+    constexpr int NEP = (TJ * NLH + BT - 1) / BT;
     __shared__ float2 s[3 * TJ * LS];
     __shared__ float2 stw[NL2];
     __shared__ double red[kSlots * 16];
@@ -1164,7 +1172,7 @@ __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ 
             float2 v[NLD];
 #pragma unroll
             for (int q = 0; q < NLD; ++q) {
-                const int f = threadIdx.x + q * kBlock;
+                const int f = threadIdx.x + q * BT;
                 v[q] = make_float2(0.f, 0.f);
                 if (f < nld) {
                     const int LL = f & (NL2 - 1), r = f >> LNL2, t = r & (tj - 1), comp = r >> ltj;
@@ -1173,16 +1181,16 @@ __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ 
             }
 #pragma unroll
             for (int q = 0; q < NLD; ++q) {
-                const int f = threadIdx.x + q * kBlock;
+                const int f = threadIdx.x + q * BT;
                 if (f < nld) {   // line comp * tj + t; L' back to natural order
                     const int Lp = f & (NL2 - 1);
                     s[(f >> LNL2) * LS + (Lp < NLH ? 2 * Lp : 2 * (Lp - NLH) + 1)] = v[q];
                 }
             }
         }
-        for (int f = threadIdx.x; f < NL2; f += kBlock) stw[f] = tw[f];
+        for (int f = threadIdx.x; f < NL2; f += BT) stw[f] = tw[f];
         __syncthreads();
-        fft_lds<NL2, 3 * TJ, LS>(s, 3 * tj, stw);
+        fft_lds<NL2, 3 * TJ, LS, 1, BT>(s, 3 * tj, stw);
 
         // epilogue operands of every cell of this thread are loaded before the
         // first is used (each cell's outputs overwrite only its own operands)
@@ -1202,7 +1210,7 @@ __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ 
         float2 a[NEP], xr[NEP][3], yr[NEP][3], o2[NEP][3];
 #pragma unroll
         for (int q = 0; q < NEP; ++q) {
-            const int f = threadIdx.x + q * kBlock;
+            const int f = threadIdx.x + q * BT;
             kq[q] = f;   // cell k0 + f: row t = f / nl, l = f % nl
             dip[q] = false;
             a[q] = make_float2(0.f, 0.f);
@@ -1320,7 +1328,7 @@ __global__ __launch_bounds__(kBlock) void k_zi(Dims d, SolveState* __restrict__ 
             }
         }
         if (ea.partials) {
-            block_sum<kSlots>(acc, red);
+            block_sum<kSlots, BT>(acc, red);
             if (threadIdx.x == 0) {
                 double* p = ea.partials + ((long long)rhs * gridDim.x + blockIdx.x) * kSlots;
 #pragma unroll
