@@ -997,6 +997,24 @@ float cabs_prefactor(const float* e) {
 
 int update_blocks(const Dims& d) { return (int)std::min<long long>((d.n + kBlock - 1) / kBlock, 1024); }
 
+// Whether the update runs the scalar step that precedes it (k_update): up to
+// 256 epilogue partials per right-hand side, one per thread, and 512 update
+// blocks, two per CU.  CG step, MI355X, in a launch of its own against within:
+// 16^3, 2 RHS 35.5 -> 34.0 us; 32^3, 2 RHS 42.3 -> 40.6; 16x32x128, 2 RHS (128
+// partials, 512 blocks) 69.3 -> 67.3; 32x32x64, 2 RHS 55.3 -> 53.5; with more
+// blocks that each repeat it, it loses: 32x32x64, 4 RHS (1024 blocks) 82.9 ->
+// 85.7, 16 RHS 175 -> 187.
+constexpr int kMidBlocks = 256;
+bool mid_within(const Dims& d, int nblk) {
+    return nblk <= kMidBlocks && (long long)update_blocks(d) * d.nrhs <= 512;
+}
+
+// Partial sums of a solve per right-hand side, in doubles: an epilogue's, or
+// an update's behind those of the epilogue that its scalar step reads.
+size_t step_partials(const Dims& d) {
+    return (size_t)std::max(max_epi_blocks(d), update_blocks(d) + std::min(max_epi_blocks(d), kMidBlocks)) * kSlots;
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -1100,8 +1118,7 @@ int ddafft_create(int ni, int nj, int nl, float kd, int nrhs_max, ddafft_ctx** o
     // at least 512 KB: room for the far field's partial sums of most direction
     // sets, which would otherwise be allocated by the first solve
     if (!rc)
-        rc = ensure_partials(c, std::max<size_t>((size_t)nrhs_max * std::max<long long>(max_epi_blocks(c->d), 1024) * kSlots,
-                                                 (size_t)1 << 16));
+        rc = ensure_partials(c, std::max<size_t>((size_t)nrhs_max * std::max<size_t>(step_partials(c->d), 1024 * kSlots), (size_t)1 << 16));
     if (rc) {
         ddafft_destroy(c);
         return rc;
@@ -1441,11 +1458,11 @@ struct Seq {
     FinArgs fa;
 
     // the scalar step `kind` over nblk block partials per right-hand side
-    int fin(int kind, int iter, int nblk) {
-        FinArgs f = fa;
+    int fin_args(int kind, int nblk, const double* partials, FinArgs& f) {
+        f = fa;
         f.kind = kind;
         f.nblk = nblk;
-        f.partials = c->partials;
+        f.partials = partials;
         f.hist = c->hist;
         // the step that closes an iteration publishes the states to the ring
         // (slot: the iteration & 3, read on the device)
@@ -1453,6 +1470,11 @@ struct Seq {
         f.ring_stride = c->nrhs_max;
         if (!f.partials || !f.hist || (ends_step(kind) && !c->ring_dev))
             return fail(DDAFFT_ESTATE, "solver scratch not allocated");
+        return DDAFFT_OK;
+    }
+    int fin(int kind, int nblk, const double* partials) {
+        FinArgs f;
+        TRY(fin_args(kind, nblk, partials, f));
         hipLaunchKernelGGL(k_finalize, nrhs, kBlock, 0, c->stream, c->st, f);
         HIPCHECK(hipGetLastError());
         return DDAFFT_OK;
@@ -1464,19 +1486,32 @@ struct Seq {
         ea.partials = c->partials;
         ea.conj = conj;
         TRY(launch_matvec(c, nrhs, pa, c->st, iter, ea, conj));
-        return fin_kind >= 0 ? fin(fin_kind, iter, epi_blocks(c, ea.kind)) : DDAFFT_OK;
+        return fin_kind >= 0 ? fin(fin_kind, epi_blocks(c, ea.kind), c->partials) : DDAFFT_OK;
     }
-    // the solver update, then (fin_kind >= 0) the scalar step over its partials
-    int upd(int iter, UpdArgs ua, int fin_kind = -1) {
+    // the scalar step `mid` over the partials of the epilogue `epi_kind`, the
+    // solver update, then the scalar step `fin_kind` over the update's partials
+    int upd(int mid, int epi_kind, UpdArgs ua, int fin_kind) {
         Dims d = c->d;
         d.nrhs = nrhs;
+        FinArgs f{};
+        const int nblk = epi_blocks(c, epi_kind);
         ua.partials = c->partials;
+        const bool within = mid_within(d, nblk);
+        if (within) {
+            TRY(fin_args(mid, nblk, c->partials, f));
+            ua.partials += (size_t)nrhs * nblk * kSlots;
+        } else {
+            TRY(fin(mid, nblk, c->partials));
+        }
         if (!ua.P || !ua.R || !ua.S || !ua.W || !ua.partials || (ua.kind == UK_BICG && !ua.G))
             return fail(DDAFFT_ESTATE, "internal: update launched with a missing buffer");
         dim3 g(update_blocks(d), nrhs);
-        hipLaunchKernelGGL(k_update, g, kBlock, 0, c->stream, d, c->st, ua, c->dipf);
+        if (within)
+            hipLaunchKernelGGL(k_update<true>, g, kBlock, 0, c->stream, d, c->st, ua, c->dipf, f);
+        else
+            hipLaunchKernelGGL(k_update<false>, g, kBlock, 0, c->stream, d, c->st, ua, c->dipf, f);
         HIPCHECK(hipGetLastError());
-        return fin_kind >= 0 ? fin(fin_kind, iter, update_blocks(d)) : DDAFFT_OK;
+        return fin(fin_kind, update_blocks(d), ua.partials);
     }
 };
 
@@ -1510,8 +1545,8 @@ int step0(Seq& q, int solver) {
         case DDAFFT_SOLVER_BICGSTAB:
             TRY(q.mv(0, pro(PRO_COPY, c->P), epi(EK_BICG_R0, nullptr, c->R, c->S, c->G), 0, FK_BICG_0));
             TRY(q.mv(0, pro(PRO_COPY, c->S), epi(EK_BICG_H, c->S, c->H, nullptr, nullptr, c->G), 0, FK_BICG_A));
-            TRY(q.mv(0, pro(PRO_LC1, c->R, c->H), epi(EK_BICG_W, c->R, c->W), 0, FK_BICG_W));
-            TRY(q.upd(0, UpdArgs{UK_BICG, c->P, c->R, c->S, c->W, c->G, nullptr}, FK_BICG_E));
+            TRY(q.mv(0, pro(PRO_LC1, c->R, c->H), epi(EK_BICG_W, c->R, c->W), 0));
+            TRY(q.upd(FK_BICG_W, EK_BICG_W, UpdArgs{UK_BICG, c->P, c->R, c->S, c->W, c->G, nullptr}, FK_BICG_E));
             break;
         case DDAFFT_SOLVER_SIMPLE:
             TRY(q.mv(0, pro(PRO_COPY, c->P), epi(EK_SIM_R0, c->P, c->R, c->S, c->P), 0, FK_SIM_E));
@@ -1532,13 +1567,13 @@ int iteration(Seq& q, int solver, int o, float tau, int part = 0) {
     switch (solver) {
         case DDAFFT_SOLVER_CG: {
             ProArgs p = (o == 1) ? pro(PRO_COPY, c->S) : pro(PRO_LC2, c->R, c->S);
-            TRY(q.mv(o, snap(p), epi(EK_CG_W, c->S, c->W, nullptr, nullptr, c->R), 0, FK_CG_A));
-            TRY(q.upd(o, UpdArgs{UK_CG, c->P, c->R, c->S, c->W, nullptr, nullptr}, FK_CG_E));
+            TRY(q.mv(o, snap(p), epi(EK_CG_W, c->S, c->W, nullptr, nullptr, c->R), 0));
+            TRY(q.upd(FK_CG_A, EK_CG_W, UpdArgs{UK_CG, c->P, c->R, c->S, c->W, nullptr, nullptr}, FK_CG_E));
             break;
         }
         case DDAFFT_SOLVER_AA:
-            TRY(q.mv(o, snap(pro(PRO_COPY, c->S)), epi(EK_AA_W, c->S, c->W), 0, FK_AA_A));
-            TRY(q.upd(o, UpdArgs{UK_AA, c->P, c->R, c->S, c->W, nullptr, nullptr}, FK_AA_E));
+            TRY(q.mv(o, snap(pro(PRO_COPY, c->S)), epi(EK_AA_W, c->S, c->W), 0));
+            TRY(q.upd(FK_AA_A, EK_AA_W, UpdArgs{UK_AA, c->P, c->R, c->S, c->W, nullptr, nullptr}, FK_AA_E));
             TRY(q.mv(o, pro(PRO_COPY, c->R), epi(EK_AA_SUPD, c->R, nullptr, c->S), 1));
             break;
         case DDAFFT_SOLVER_BICGSTAB:
@@ -1546,8 +1581,8 @@ int iteration(Seq& q, int solver, int o, float tau, int part = 0) {
                 TRY(q.mv(o, snap(pro(PRO_LC4, c->R, c->S, c->H)), epi(EK_BICG_H, c->S, c->H, nullptr, nullptr, c->G), 0,
                          FK_BICG_A));
             if (part != 1) {
-                TRY(q.mv(o, pro(PRO_LC1, c->R, c->H), epi(EK_BICG_W, c->R, c->W), 0, FK_BICG_W));
-                TRY(q.upd(o, UpdArgs{UK_BICG, c->P, c->R, c->S, c->W, c->G, nullptr}, FK_BICG_E));
+                TRY(q.mv(o, pro(PRO_LC1, c->R, c->H), epi(EK_BICG_W, c->R, c->W), 0));
+                TRY(q.upd(FK_BICG_W, EK_BICG_W, UpdArgs{UK_BICG, c->P, c->R, c->S, c->W, c->G, nullptr}, FK_BICG_E));
             }
             break;
         case DDAFFT_SOLVER_SIMPLE:
@@ -1953,7 +1988,7 @@ int run_begin(Run& r) {
         s.stop_at = r.max_step + 1;
     }
     TRY(upload(c, c->st, s0.data(), r.nrhs * sizeof(SolveState)));
-    TRY(ensure_partials(c, (size_t)r.nrhs * std::max(max_epi_blocks(d), update_blocks(d)) * kSlots));
+    TRY(ensure_partials(c, (size_t)r.nrhs * step_partials(d)));
     TRY(flush_small(c));   // every staged input of the solve, in one copy
     if (c->pending_first_approx) {
         c->pending_first_approx = false;
@@ -2325,7 +2360,7 @@ int ddafft_solve_noalloc(ddafft_ctx* c, int nrhs, int solver, float tau, int max
         off = 0;
         res = 0;   // results, laid out as fin_layout lays them out
         obs_blocks(c, nrhs, ndirs, ffn, ffS, &cb, &fchunk);
-        n_part = std::max({(size_t)nrhs * std::max(max_epi_blocks(d), update_blocks(d)) * kSlots, (size_t)nrhs * cb * 2,
+        n_part = std::max({(size_t)nrhs * step_partials(d), (size_t)nrhs * cb * 2,
                            (size_t)nrhs * fchunk * std::max(ndirs, 1) * 6});
         n_hist = (size_t)c->nrhs_max * (max_step + 1);
         n_esc = (size_t)nrhs * ndirs * 3;

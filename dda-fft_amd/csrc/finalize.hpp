@@ -82,30 +82,65 @@ __device__ void end_step(SolveState& s, const FinArgs& fa, int rhs, int o, doubl
     }
 }
 
-// The fixed-order FP64 sum of one right-hand side's block partials and the
-// scalar step of its solver; run by every thread of one block.
-__device__ __forceinline__ void finalize_block(SolveState* __restrict__ st, int iter, const FinArgs& fa, int rhs,
-                                               double* red) {
-    double v[kSlots] = {0, 0, 0, 0, 0, 0};
+// The fixed-order FP64 sum of one right-hand side's block partials, by every
+// thread of a block of BT; the result is valid in thread 0.  (Blocks of 512
+// threads add only zeros to the sums of 256 while nblk <= 256.)
+template <int BT = kBlock>
+__device__ __forceinline__ void sum_partials(const FinArgs& fa, int rhs, double (&v)[kSlots], double* red) {
     const double* p = fa.partials + (long long)rhs * fa.nblk * kSlots;
-    // each thread sums partials b = tid, tid + 256, ... in that order; the
+    // each thread sums partials b = tid, tid + BT, ... in that order; the
     // loads of four of them are in flight together
     constexpr int kBatch = 4;
-    for (int b0 = threadIdx.x; b0 < fa.nblk; b0 += kBatch * kBlock) {
+    for (int b0 = threadIdx.x; b0 < fa.nblk; b0 += kBatch * BT) {
         double t[kBatch][kSlots];
 #pragma unroll
         for (int u = 0; u < kBatch; ++u) {
-            const int b = b0 + u * kBlock;
+            const int b = b0 + u * BT;
 #pragma unroll
             for (int q = 0; q < kSlots; ++q) t[u][q] = b < fa.nblk ? p[(long long)b * kSlots + q] : 0.0;
         }
 #pragma unroll
         for (int u = 0; u < kBatch; ++u)
-            if (b0 + u * kBlock < fa.nblk)
+            if (b0 + u * BT < fa.nblk)
 #pragma unroll
                 for (int q = 0; q < kSlots; ++q) v[q] += t[u][q];
     }
-    block_sum<kSlots>(v, red);
+    block_sum<kSlots, BT>(v, red);
+}
+
+// The scalar steps inside an iteration: they read fields of the state that
+// they do not write, and write only the coefficients named here.
+__device__ __forceinline__ void scalar_mid(int kind, const double (&v)[kSlots], SolveState& s) {
+    switch (kind) {
+        case FK_BICG_A:
+            ld_div(s.rho, s.rho_i, v[0], v[1], s.A, s.A_i);
+            s.cA = to_f(s.A, s.A_i);
+            s.pro_c1 = cneg(s.cA);
+            break;
+        case FK_BICG_W:
+            ld_div(v[0], v[1], v[2], v[3], s.W, s.W_i);
+            s.cW = to_f(s.W, s.W_i);
+            break;
+        case FK_CG_A:
+            s.den = v[0];
+            s.den_i = v[1];
+            ld_div(v[2], v[3], s.den, s.den_i, s.A, s.A_i);
+            s.cA = to_f(s.A, s.A_i);
+            break;
+        case FK_AA_A:
+            s.rA = (float)(-s.RR_1 / v[4]);
+            break;
+        default:
+            break;
+    }
+}
+
+// The scalar step of one right-hand side's solver; run by every thread of one
+// block.
+__device__ __forceinline__ void finalize_block(SolveState* __restrict__ st, int iter, const FinArgs& fa, int rhs,
+                                               double* red) {
+    double v[kSlots] = {0, 0, 0, 0, 0, 0};
+    sum_partials(fa, rhs, v, red);
     if (threadIdx.x != 0) return;
     SolveState& s = st[rhs];
     const double err = v[5] * fa.inv_ndip;
@@ -114,17 +149,12 @@ __device__ __forceinline__ void finalize_block(SolveState* __restrict__ st, int 
             s.rho_prev = s.rho = v[0];
             s.rho_prev_i = s.rho_i = v[1];
             break;
-        case FK_BICG_A: {
-            ld_div(s.rho, s.rho_i, v[0], v[1], s.A, s.A_i);
-            s.cA = to_f(s.A, s.A_i);
-            s.pro_c1 = cneg(s.cA);
+        case FK_BICG_A:
+        case FK_BICG_W:
+        case FK_CG_A:
+        case FK_AA_A:
+            scalar_mid(fa.kind, v, s);
             break;
-        }
-        case FK_BICG_W: {
-            ld_div(v[0], v[1], v[2], v[3], s.W, s.W_i);
-            s.cW = to_f(s.W, s.W_i);
-            break;
-        }
         case FK_BICG_E: {
             if (iter > 0) {
                 s.rho_prev = s.rho;
@@ -148,13 +178,6 @@ __device__ __forceinline__ void finalize_block(SolveState* __restrict__ st, int 
         case FK_SIM_E:
             end_step(s, fa, rhs, iter, err);
             break;
-        case FK_CG_A: {
-            s.den = v[0];
-            s.den_i = v[1];
-            ld_div(v[2], v[3], s.den, s.den_i, s.A, s.A_i);
-            s.cA = to_f(s.A, s.A_i);
-            break;
-        }
         case FK_CG_E: {
             double br, bi;
             ld_div(v[0], v[1], s.den, s.den_i, br, bi);
@@ -165,9 +188,6 @@ __device__ __forceinline__ void finalize_block(SolveState* __restrict__ st, int 
         }
         case FK_AA_0:
             s.RR_1 = v[4];
-            break;
-        case FK_AA_A:
-            s.rA = (float)(-s.RR_1 / v[4]);
             break;
         case FK_AA_E: {
             const double rr = v[4];

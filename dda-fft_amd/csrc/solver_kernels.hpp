@@ -106,51 +106,98 @@ struct UpdArgs {
     double* partials;  // [nrhs][gridDim.x][kSlots]
 };
 
-__global__ __launch_bounds__(kBlock) void k_update(Dims d, SolveState* __restrict__ st, UpdArgs ua,
-                                                   const int8_t* __restrict__ dipf) {
+// The update of one cell's component: p, r from their old values and s, w, g.
+__device__ __forceinline__ void update_cell(int kind, float2 ncA, float2 ncW, float rA, float2& p, float2& r, float2 s,
+                                            float2 w, float2 g, double (&acc)[kSlots]) {
+    if (kind == UK_BICG) {
+        const float2 t2 = cadd(p, cmul(ncA, s));
+        p = cadd(cmul(ncW, r), t2);
+        r = cadd(r, cmul(ncW, w));
+        dot_acc(r, g, acc[0], acc[1]);
+    } else if (kind == UK_CG) {
+        p = cadd(p, cmul(ncA, s));
+        r = cadd(r, cmul(ncA, w));
+        dot_acc(r, w, acc[0], acc[1]);
+    } else {
+        r = cadd(r, rmul(rA, w));
+        p = cadd(p, rmul(rA, s));
+        acc[4] += norm_term(r);
+    }
+}
+
+// MID: every block runs the scalar step ahead of the update itself, which
+// drops a launch of one block per right-hand side: each block adds the same
+// partials in the same order, and block 0 writes the coefficients to the
+// state, of whose fields none that it writes is read here.  The operands of
+// the thread's first cell are in flight meanwhile.  The update's own partials
+// go to another part of the buffer.
+template <bool MID>
+__global__ __launch_bounds__(kBlock) void k_update(Dims d, SolveState* st, UpdArgs ua, const int8_t* __restrict__ dipf,
+                                                   FinArgs fa) {
     __shared__ double red[kSlots * 16];
     const int rhs = blockIdx.y;
-    if (st[rhs].it >= st[rhs].stop_at) return;
-    const float2 ncA = cneg(st[rhs].cA), ncW = cneg(st[rhs].cW);
-    const float rA = st[rhs].rA;
-    const long long rb = (long long)rhs * 3 * d.n;
+    const SolveState& s = st[rhs];
+    if (s.it >= s.stop_at) return;
+    float2 ncA = cneg(s.cA), ncW = cneg(s.cW);
+    float rA = s.rA;
+    const long long rb = (long long)rhs * 3 * d.n, stride = (long long)gridDim.x * blockDim.x;
+    const long long k0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     double acc[kSlots] = {0, 0, 0, 0, 0, 0};
-    for (long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x; k < d.n;
-         k += (long long)gridDim.x * blockDim.x) {
-        // off the dipoles P is zero from the first approximation (or the
-        // adjoint source) on and nothing reads the other vectors
-        if (dipf[k] == 0) continue;
+    // off the dipoles P is zero from the first approximation (or the adjoint
+    // source) on and nothing reads the other vectors; a cell's 12 or 15
+    // operands are requested together (CG step at 64^3, 1 RHS 93 -> 91.3 us)
+    auto cell = [&](long long k, auto first) {
+        float2 p[3], r[3], sv[3], w[3], g[3];
+        const bool on = k < d.n && dipf[k] != 0;
+        if (on)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const long long ck = rb + q * d.n + k;
+                p[q] = ua.P[ck];
+                r[q] = ua.R[ck];
+                sv[q] = ua.S[ck];
+                w[q] = ua.W[ck];
+                g[q] = ua.kind == UK_BICG ? ua.G[ck] : make_float2(0.f, 0.f);
+            }
+        first();
+        if (!on) return;
         double nrm = 0;
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
             const long long ck = rb + q * d.n + k;
-            float2 p = ua.P[ck], r = ua.R[ck];
-            if (ua.kind == UK_BICG) {
-                const float2 t2 = cadd(p, cmul(ncA, ua.S[ck]));
-                p = cadd(cmul(ncW, r), t2);
-                r = cadd(r, cmul(ncW, ua.W[ck]));
-                dot_acc(r, ua.G[ck], acc[0], acc[1]);
-            } else if (ua.kind == UK_CG) {
-                const float2 w = ua.W[ck];
-                p = cadd(p, cmul(ncA, ua.S[ck]));
-                r = cadd(r, cmul(ncA, w));
-                dot_acc(r, w, acc[0], acc[1]);
-            } else {
-                r = cadd(r, rmul(rA, ua.W[ck]));
-                p = cadd(p, rmul(rA, ua.S[ck]));
-                acc[4] += norm_term(r);
-            }
-            ua.P[ck] = p;
-            ua.R[ck] = r;
-            nrm += norm_term(r);
+            update_cell(ua.kind, ncA, ncW, rA, p[q], r[q], sv[q], w[q], g[q], acc);
+            ua.P[ck] = p[q];
+            ua.R[ck] = r[q];
+            nrm += norm_term(r[q]);
         }
         acc[5] += sqrt(nrm);
+    };
+    if constexpr (MID) {
+        __shared__ float2 coef;
+        cell(k0, [&]() {
+            double v[kSlots] = {0, 0, 0, 0, 0, 0};
+            sum_partials(fa, rhs, v, red);
+            if (threadIdx.x == 0) {
+                SolveState t;
+                t.RR_1 = s.RR_1;
+                scalar_mid(fa.kind, v, t);
+                coef = fa.kind == FK_CG_A ? t.cA : fa.kind == FK_BICG_W ? t.cW : make_float2(t.rA, 0.f);
+                if (blockIdx.x == 0) scalar_mid(fa.kind, v, st[rhs]);
+            }
+            __syncthreads();
+            if (fa.kind == FK_CG_A) ncA = cneg(coef);
+            if (fa.kind == FK_BICG_W) ncW = cneg(coef);
+            if (fa.kind == FK_AA_A) rA = coef.x;
+        });
+        for (long long k = k0 + stride; k < d.n; k += stride) cell(k, [] {});
+    } else {
+        for (long long k = k0; k < d.n; k += stride) cell(k, [] {});
     }
     block_sum<kSlots>(acc, red);
     if (threadIdx.x == 0) {
-        double* p = ua.partials + ((long long)rhs * gridDim.x + blockIdx.x) * kSlots;
+        double* q = ua.partials + ((long long)rhs * gridDim.x + blockIdx.x) * kSlots;
 #pragma unroll
-        for (int q = 0; q < kSlots; ++q) p[q] = acc[q];
+        for (int e = 0; e < kSlots; ++e) q[e] = acc[e];
     }
 }
 
