@@ -2784,7 +2784,7 @@ int ddafft_gradient(ddafft_ctx* c, int npol, int nobj, int solver, float tau, in
         hipLaunchKernelGGL(k_adj_source, dim3(nblk, nadj), kBlock, 0, c->stream, d, g, c->occ, c->mv, aa);
         HIPCHECK(hipGetLastError());
     }
-    hipLaunchKernelGGL(k_adj_scale, 1, 64, 0, c->stream, c->partials, nblk, nadj,
+    hipLaunchKernelGGL(k_adj_scale, nadj, 64, 0, c->stream, c->partials, nblk,
                        reinterpret_cast<const double*>(c->gaux + off_na), reinterpret_cast<float*>(c->gaux + off_s),
                        reinterpret_cast<float*>(c->gaux + off_is));
     HIPCHECK(hipGetLastError());
