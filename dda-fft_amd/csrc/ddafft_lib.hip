@@ -1005,15 +1005,17 @@ int update_blocks(const Dims& d) { return (int)std::min<long long>((d.n + kBlock
 // blocks that each repeat it, it loses: 32x32x64, 4 RHS (1024 blocks) 82.9 ->
 // 85.7, 16 RHS 175 -> 187.
 constexpr int kMidBlocks = 256;
-bool mid_within(const Dims& d, int nblk) {
-    return nblk <= kMidBlocks && (long long)update_blocks(d) * d.nrhs <= 512;
+// It also takes room for both kernels' partials, which a solve within fixed
+// scratch may not have; the sums are the same either way.
+constexpr int kMidUpdates = 512;
+bool mid_within(const ddafft_ctx* c, const Dims& d, int nblk) {
+    const long long upd = (long long)update_blocks(d) * d.nrhs;
+    return nblk <= kMidBlocks && upd <= kMidUpdates &&
+           (size_t)(upd + (long long)nblk * d.nrhs) * kSlots <= c->partials_cap;
 }
 
-// Partial sums of a solve per right-hand side, in doubles: an epilogue's, or
-// an update's behind those of the epilogue that its scalar step reads.
-size_t step_partials(const Dims& d) {
-    return (size_t)std::max(max_epi_blocks(d), update_blocks(d) + std::min(max_epi_blocks(d), kMidBlocks)) * kSlots;
-}
+// Partial sums of a solve per right-hand side, in doubles.
+size_t step_partials(const Dims& d) { return (size_t)std::max(max_epi_blocks(d), update_blocks(d)) * kSlots; }
 
 }  // namespace
 
@@ -1496,7 +1498,7 @@ struct Seq {
         FinArgs f{};
         const int nblk = epi_blocks(c, epi_kind);
         ua.partials = c->partials;
-        const bool within = mid_within(d, nblk);
+        const bool within = mid_within(c, d, nblk);
         if (within) {
             TRY(fin_args(mid, nblk, c->partials, f));
             ua.partials += (size_t)nrhs * nblk * kSlots;
@@ -1988,7 +1990,8 @@ int run_begin(Run& r) {
         s.stop_at = r.max_step + 1;
     }
     TRY(upload(c, c->st, s0.data(), r.nrhs * sizeof(SolveState)));
-    TRY(ensure_partials(c, (size_t)r.nrhs * step_partials(d)));
+    const bool mid_room = !t_noalloc && (long long)update_blocks(d) * r.nrhs <= kMidUpdates;   // mid_within
+    TRY(ensure_partials(c, (size_t)r.nrhs * (step_partials(d) + (mid_room ? kMidBlocks * kSlots : 0))));
     TRY(flush_small(c));   // every staged input of the solve, in one copy
     if (c->pending_first_approx) {
         c->pending_first_approx = false;
