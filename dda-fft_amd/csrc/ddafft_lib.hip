@@ -171,7 +171,19 @@ char* scratch_address(int dev) {
 // Context
 // ---------------------------------------------------------------------------
 
-struct ddafft_ctx {
+// A direction set on the device and how it splits into groups that share z
+// (dir_groups).  The splits belong to the directions: they are kept, saved and
+// put back with them, as one.
+struct Directions {
+    float* dirs = nullptr;
+    int ndirs = 0, dirs_cap = 0;   // resident directions (dirs_cap in directions)
+    int ffg_n = 0, ffg_S = 1;      // ffg_n groups of ffg_S (at most kFFMembers), for the far field by columns
+    int ffs_n = 0, ffs_S = 1;      // groups of at most kFFDirs, for the S11 gradients' far field
+
+    void split(const float* host, int n);   // host: the n directions, nullptr where they share no groups
+};
+
+struct ddafft_ctx : Directions {
     int device = 0;
     hipStream_t stream = nullptr;
     Dims d{};
@@ -205,7 +217,6 @@ struct ddafft_ctx {
     float2* ffpc = nullptr;
     size_t ffpc_cap = 0;
     bool ff_s11 = false;      // such a call's forward solve is running
-    int ffs_n = 0, ffs_S = 1; // its split of the direction set, groups of at most kFFDirs
     long long ndip = 0;
     std::vector<long long> mat_count;  // dipoles per material index
     bool have_target = false;
@@ -231,8 +242,6 @@ struct ddafft_ctx {
     int hist_cap = 0;
     double* partials = nullptr;
     size_t partials_cap = 0;
-    float* dirs = nullptr;
-    int ndirs = 0, dirs_cap = 0;       // resident directions (dirs_cap in directions)
     std::vector<char> dir_pairs;       // per-RHS directions: do RHS 2q and 2q+1 share them?
     // gradients: forward dipoles kept for the adjoint, per-axis phase table,
     // small per-call arrays
@@ -250,7 +259,6 @@ struct ddafft_ctx {
     int ahat_mode = 0;                 // 0: full Â as the reference builds it; 1: one octant (Nyquist planes zeroed)
     int ff_mfma = -1;                  // far field on the matrix cores: -1 default, 0 off, 1 on
     int ff_group = -1;                 // far field by columns: -1 default (on), 0 off, 1 on
-    int ffg_n = 0, ffg_S = 1;          // the direction set as ffg_n groups of ffg_S sharing z (dir_groups)
     int ff_chunk_max = 0;              // set by an allocation-free solve: column chunks that its scratch has room for
     // launch schedule, 0 / -1: from the tuned table, else the built-in rule
     int x_blocks = 0;                  // X pass: blocks per launch up to which right-hand-side groups are spread
@@ -1395,6 +1403,11 @@ int dir_groups(const float* dirs, int ndirs, int most, int* S) {
 
 }  // namespace
 
+void Directions::split(const float* host, int n) {
+    ffg_n = dir_groups(host, n, kFFMembers, &ffg_S);
+    ffs_n = dir_groups(host, n, kFFDirs, &ffs_S);
+}
+
 int ddafft_set_directions(ddafft_ctx* c, int ndirs, const float* dirs) {
     if (!c || ndirs < 0 || (ndirs > 0 && !dirs)) return fail(DDAFFT_EINVAL, "bad directions");
     HIPCHECK(hipStreamSynchronize(c->stream));
@@ -1407,8 +1420,7 @@ int ddafft_set_directions(ddafft_ctx* c, int ndirs, const float* dirs) {
         c->dirs_cap = ndirs;
     }
     c->ndirs = ndirs;
-    c->ffg_n = dir_groups(dirs, ndirs, kFFMembers, &c->ffg_S);
-    c->ffs_n = dir_groups(dirs, ndirs, kFFDirs, &c->ffs_S);
+    c->split(dirs, ndirs);
     if (ndirs) {
         HIPCHECK(hipMemcpy(c->dirs, dirs, (size_t)ndirs * 3 * sizeof(float), hipMemcpyHostToDevice));
     }
@@ -2256,9 +2268,7 @@ int job_prepare(ddafft_ctx* c, const ddafft_job* j, int solver, int max_step, co
             }
             TRY(upload(c, c->dirs, j->dirs, per * sets * sizeof(float)));
             c->ndirs = j->dirs_per_rhs ? 0 : ndirs;   // per-RHS sets are not resident for later calls
-            const float* gd = j->dirs_per_rhs ? nullptr : j->dirs;   // rotated sets: no groups
-            c->ffg_n = dir_groups(gd, ndirs, kFFMembers, &c->ffg_S);
-            c->ffs_n = dir_groups(gd, ndirs, kFFDirs, &c->ffs_S);
+            c->split(j->dirs_per_rhs ? nullptr : j->dirs, ndirs);   // rotated sets: no groups
             if (j->dirs_per_rhs) {
                 *dir_stride = (long long)per;
                 c->dir_pairs.assign((size_t)(nrhs + 1) / 2, 0);
@@ -2408,12 +2418,11 @@ int ddafft_solve_noalloc(ddafft_ctx* c, int nrhs, int solver, float tau, int max
         double* hist; int hist_cap;
         float2* esc; int esc_cap;
         float2* fftab; size_t fftab_cap;
-        float* dirs; int dirs_cap, ndirs, ffg_n, ffg_S;
+        Directions dirs;
         float* seqbuf; size_t seqbuf_cap;
         char *dn, *dn_dev; size_t dn_cap;
-    } sv{c->partials, c->partials_cap, c->hist, c->hist_cap, c->esc, c->esc_cap, c->fftab, c->fftab_cap, c->dirs,
-         c->dirs_cap, c->ndirs, c->ffg_n, c->ffg_S, c->seqbuf, c->seqbuf_cap, c->dn, c->dn_dev,
-         c->dn_cap};
+    } sv{c->partials, c->partials_cap, c->hist, c->hist_cap, c->esc, c->esc_cap, c->fftab, c->fftab_cap, *c, c->seqbuf,
+         c->seqbuf_cap, c->dn, c->dn_dev, c->dn_cap};
     HIPCHECK(hipStreamSynchronize(c->stream));   // nothing of an earlier call still uses the old buffers
     char* sc = c->scratch;
     c->partials = reinterpret_cast<double*>(sc + o_part);
@@ -2448,11 +2457,7 @@ int ddafft_solve_noalloc(ddafft_ctx* c, int nrhs, int solver, float tau, int max
     c->esc_cap = sv.esc_cap;
     c->fftab = sv.fftab;
     c->fftab_cap = sv.fftab_cap;
-    c->dirs = sv.dirs;
-    c->dirs_cap = sv.dirs_cap;
-    c->ndirs = sv.ndirs;
-    c->ffg_n = sv.ffg_n;
-    c->ffg_S = sv.ffg_S;
+    static_cast<Directions&>(*c) = sv.dirs;
     c->seqbuf = sv.seqbuf;
     c->seqbuf_cap = sv.seqbuf_cap;
     c->dn = sv.dn;
