@@ -128,9 +128,11 @@ __device__ __forceinline__ void update_cell(int kind, float2 ncA, float2 ncW, fl
 // MID: every block runs the scalar step ahead of the update itself, which
 // drops a launch of one block per right-hand side: each block adds the same
 // partials in the same order, and block 0 writes the coefficients to the
-// state, of whose fields none that it writes is read here.  The operands of
-// the thread's first cell are in flight meanwhile.  The update's own partials
-// go to another part of the buffer.
+// state.  No block reads a field that block 0 may be writing: the coefficient
+// that the step gives comes from the block's own sum (`coef`), and from the
+// state come only it, stop_at, RR_1 and, for BiCGStab, whose step here gives
+// cW, cA.  The operands of the thread's first cell are in flight meanwhile.
+// The update's own partials go to another part of the buffer.
 template <bool MID>
 __global__ __launch_bounds__(kBlock) void k_update(Dims d, SolveState* st, UpdArgs ua, const int8_t* __restrict__ dipf,
                                                    FinArgs fa) {
@@ -138,8 +140,13 @@ __global__ __launch_bounds__(kBlock) void k_update(Dims d, SolveState* st, UpdAr
     const int rhs = blockIdx.y;
     const SolveState& s = st[rhs];
     if (s.it >= s.stop_at) return;
-    float2 ncA = cneg(s.cA), ncW = cneg(s.cW);
-    float rA = s.rA;
+    float2 ncA = make_float2(0.f, 0.f), ncW = ncA;
+    float rA = 0.f;
+    if (!MID || fa.kind == FK_BICG_W) ncA = cneg(s.cA);
+    if constexpr (!MID) {
+        ncW = cneg(s.cW);
+        rA = s.rA;
+    }
     const long long rb = (long long)rhs * 3 * d.n, stride = (long long)gridDim.x * blockDim.x;
     const long long k0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     double acc[kSlots] = {0, 0, 0, 0, 0, 0};
