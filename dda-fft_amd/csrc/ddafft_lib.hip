@@ -123,7 +123,10 @@ int dev_alloc(T** p, size_t count) {
     if (count == 0) return DDAFFT_OK;
     if (t_noalloc) return fail(DDAFFT_ESTATE, "internal: device allocation inside the allocation-free solve");
     hipError_t e = hipMalloc((void**)p, count * sizeof(T));
-    if (e != hipSuccess) return fail(DDAFFT_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // reported here: the next launch check must not find it again
+        return fail(DDAFFT_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    }
     return DDAFFT_OK;
 }
 
@@ -1285,16 +1288,20 @@ int ddafft_set_target(ddafft_ctx* c, const signed char* occ, int nmat, const int
     const size_t o_col = put(fcol.data(), fcol.size() * sizeof(int), fcol.size() * sizeof(int));
     const size_t o_pc = put(fpiece.data(), fpiece.size() * sizeof(int2), fpiece.size() * sizeof(int2));
     HIPCHECK(hipStreamSynchronize(c->stream));
+    // from here to the end the context has no target: if an allocation or a
+    // copy fails, later calls are refused and nothing points into the block
+    c->have_target = false;
     if (c->ffseg) hipFree(c->ffseg);
     c->ffseg = nullptr;
     c->nffpiece = c->nseg = 0;
+    c->occ = c->dipf = nullptr;
+    c->rows = nullptr;
+    c->mv = c->cells = c->ffcol = nullptr;
+    c->ffpiece = nullptr;
     if (total > c->target_cap) {
         if (c->target) hipFree(c->target);
         c->target = nullptr;
         c->target_cap = 0;
-        c->occ = c->dipf = nullptr;
-        c->rows = nullptr;
-        c->mv = nullptr;
         TRY(dev_alloc(&c->target, total));
         c->target_cap = total;
     }

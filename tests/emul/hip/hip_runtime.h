@@ -27,6 +27,7 @@
 #include <memory>
 #include <mutex>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #if defined(__SANITIZE_ADDRESS__)
@@ -296,7 +297,12 @@ constexpr unsigned hipEventDisableTiming = 2;
 constexpr unsigned hipHostMallocDefault = 0;
 
 inline const char* hipGetErrorString(hipError_t) { return "emulated HIP error"; }
-inline hipError_t hipGetLastError() { return hipSuccess; }
+namespace emul {
+inline hipError_t g_last_error = hipSuccess;   // kept until it is asked for, as the runtime keeps it
+inline long g_fail_malloc = -1;                // device allocations left before the one that fails (-1: none fails)
+}  // namespace emul
+extern "C" __attribute__((used)) inline void emul_fail_malloc(long after) { emul::g_fail_malloc = after; }
+inline hipError_t hipGetLastError() { return std::exchange(emul::g_last_error, hipSuccess); }
 inline hipError_t hipGetDeviceCount(int* n) {
     *n = 1;
     return hipSuccess;
@@ -306,6 +312,7 @@ inline hipError_t hipGetDevice(int* d) {
     return hipSuccess;
 }
 inline hipError_t hipMalloc(void** p, size_t bytes) {
+    if (emul::g_fail_malloc >= 0 && emul::g_fail_malloc-- == 0) return emul::g_last_error = hipErrorOutOfMemory;
     *p = std::malloc(bytes ? bytes : 1);
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }
