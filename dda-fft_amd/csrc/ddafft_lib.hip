@@ -184,6 +184,10 @@ struct Directions {
     int ffs_n = 0, ffs_S = 1;      // groups of at most kFFDirs, for the S11 gradients' far field
 
     void split(const float* host, int n);   // host: the n directions, nullptr where they share no groups
+    void drop() {                           // no set is resident
+        if (dirs) hipFree(dirs);
+        *this = Directions();
+    }
 };
 
 struct ddafft_ctx : Directions {
@@ -1419,9 +1423,7 @@ int ddafft_set_directions(ddafft_ctx* c, int ndirs, const float* dirs) {
     if (!c || ndirs < 0 || (ndirs > 0 && !dirs)) return fail(DDAFFT_EINVAL, "bad directions");
     HIPCHECK(hipStreamSynchronize(c->stream));
     if (ndirs > c->dirs_cap) {
-        if (c->dirs) hipFree(c->dirs);
-        c->dirs = nullptr;
-        c->dirs_cap = 0;
+        c->drop();
         int rc = dev_alloc(&c->dirs, (size_t)ndirs * 3);
         if (rc) return rc;
         c->dirs_cap = ndirs;
@@ -2267,9 +2269,7 @@ int job_prepare(ddafft_ctx* c, const ddafft_job* j, int solver, int max_step, co
             const int sets = j->dirs_per_rhs ? nrhs : 1;
             if ((long long)ndirs * sets > c->dirs_cap) {
                 HIPCHECK(hipStreamSynchronize(c->stream));
-                if (c->dirs) hipFree(c->dirs);
-                c->dirs = nullptr;
-                c->dirs_cap = 0;
+                c->drop();
                 TRY(dev_alloc(&c->dirs, per * sets));
                 c->dirs_cap = ndirs * sets;
             }

@@ -13,7 +13,7 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 EMUL = os.path.join(ROOT, "tests", "emul")
-CASES = ["set_target"]
+CASES = ["set_target", "directions"]
 
 
 @pytest.mark.skipif(os.environ.get("DDAFFT_EMUL") != "1", reason="set DDAFFT_EMUL=1 to run")
@@ -73,6 +73,33 @@ def set_target():
         ctx.set_target(full, [0, 1])
         ref = solve(ctx)
     assert np.array_equal(got["esc"], ref["esc"]) and got["cext"] == ref["cext"]
+
+
+def directions():
+    """A larger direction set that cannot be allocated, resident or brought by
+    a solve: the set that was resident is gone, and solves that ask for it are
+    refused until a set is given again."""
+    kd = np.float32(0.5)
+    alpha = alpha_of(kd)
+    dirs = np.array([[0, 0, 1], [1, 0, 0]], np.float32)
+    more = np.repeat(dirs, 8, 0)
+
+    def solve(ctx, **kw):
+        return ctx.solve("bicgstab", alpha, KINC, EINC, max_step=1, err_max=1e-9, **kw)[0]
+
+    with ddafft.Context(DIMS, kd, nrhs_max=2) as ctx:
+        ctx.set_target(np.ones(DIMS, np.int8), [0, 1])
+        for fails in (lambda: ctx.set_directions(more), lambda: solve(ctx, dirs=more)):
+            ctx.set_directions(dirs)
+            ref = solve(ctx)
+            ddafft._lib.emul_fail_malloc(0)
+            refused(fails, "hipMalloc")
+            refused(lambda: solve(ctx), "differs from the resident directions")
+            refused(lambda: solve(ctx, noalloc=True), "differs from the resident directions")
+            refused(lambda: ctx.gradient("bicgstab", alpha, alpha, np.array([1, 1.5]), KINC, EINC, np.ones((1, 4))),
+                    "bad directions")
+            ctx.set_directions(dirs)
+            assert np.array_equal(solve(ctx)["esc"], ref["esc"])
 
 
 if __name__ == "__main__":
