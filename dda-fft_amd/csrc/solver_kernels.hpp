@@ -547,8 +547,9 @@ __global__ __launch_bounds__(kBlock) void k_far_field_mfma(Dims d, const float2*
 // columns over a range of l.  One v_mfma_f32_16x16x4f32 takes 16 groups (rows)
 // x 4 l x 8 complex columns as 16 real ones (lane n < 8: real part of column
 // n, else the imaginary part of column n - 8):
-//   D += Re(Z) [Pr | Pi]  and  D += Im(Z) [-Pi | Pr]
-// (lane layout: A[l % 16][l / 16], B[l / 16][l % 16], D[4 (l / 16) + v][l % 16]).
+//   D1 += Re(Z) [Pr | Pi]  and  D2 += Im(Z) [-Pi | Pr],  T = D1 + D2
+// (two accumulators: half the chain of roundings; lane layout: A[l % 16][l / 16],
+// B[l / 16][l % 16], D[4 (l / 16) + v][l % 16]).
 // Lane group k of a wave takes the four l's 16 u + 4 k + s, s = 0 .. 3, of a
 // 16-point chunk u in four such products.  The chunk's moments are loaded as
 // whole 128-byte lines and change lanes through LDS (loaded straight into the
@@ -571,8 +572,14 @@ __global__ __launch_bounds__(kBlock) void k_far_field_mfma(Dims d, const float2*
 //   32x32x64 agglomerate, 8 sets of 19, 16 RHS     173 -> 21 (one launch)
 // At 256^3 the products alone are 1.1 ms of matrix-core time; the rest is the
 // VALU work of stage 2 and LDS and L1 accesses that the four waves of a SIMD
-// do not hide.  Error against 64-bit sums: no larger than before (FP64 from 8
-// columns up).
+// do not hide.  LDS leaves five waves per SIMD; saying so keeps the allocation
+// at 64 VGPRs (68 without: 64^3, 4 x 181, 1 RHS 30 -> 37 us).
+// RMS error against 64-bit sums over that of the per-direction kernel, which
+// adds 8 to 70 products per thread before FP64 (8 seeds, plane waves and
+// random moments in ellipsoids of 16^3 to 64x64x64 and 16x32x128 cells, one
+// direction a group): geometric mean 0.992, 0.94 to 1.04 (one accumulator:
+// 1.006, up to 1.13 for random moments at 16^3); sets in groups of three:
+// 0.97.  The phases' rounding, which both share, is most of it.
 // tab: [set][ni + nj + nl][S][ng] phases; cols: (i nj + j) of the columns that
 // hold dipoles, padded to 8 with -1; piece: {first column / 8, 16-point chunks
 // [lo, hi) as lo | hi << 16}, padded to 4 with {0, 0}.  Grid: x over chunks of
@@ -617,11 +624,9 @@ __global__ __launch_bounds__(kBlock) void k_ff_table(Dims d, Geometry g, const f
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_far_field_cols(Dims d, const float2* __restrict__ tab, int set_rhs,
-                                                           const int* __restrict__ cols,
-                                                           const int2* __restrict__ piece, int npiece, int ng, int S,
-                                                           int nchunk, int rhs_first, const float2* __restrict__ P,
-                                                           double* __restrict__ partials) {
+__global__ __launch_bounds__(kBlock) DDA_WAVES_PER_EU(4, 5) void k_far_field_cols(
+    Dims d, const float2* __restrict__ tab, int set_rhs, const int* __restrict__ cols, const int2* __restrict__ piece,
+    int npiece, int ng, int S, int nchunk, int rhs_first, const float2* __restrict__ P, double* __restrict__ partials) {
     typedef DDA_FLOAT4_MFMA f4;
     constexpr int NC = kFFWaves * kFFCols;    // columns of a batch: one piece per wave
     constexpr int CS = 3 * kFFGroups + 17;    // T's column stride: a wave's 8 columns start in different banks
@@ -679,9 +684,9 @@ __global__ __launch_bounds__(kBlock) void k_far_field_cols(Dims d, const float2*
 #pragma unroll
             for (int s = 0; s < 4; ++s) zv[s] = tab[zo + (unsigned)min(16 * u + 4 * k + s, d.nl - 1) * ndirs];
         };
-        f4 acc[3];
+        f4 acc[3], acc2[3];
 #pragma unroll
-        for (int v = 0; v < 3; ++v) acc[v] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int v = 0; v < 3; ++v) acc[v] = acc2[v] = f4{0.f, 0.f, 0.f, 0.f};
         if (u0 < u1) fetch(u0);
         for (int u = u0; u < u1; ++u) {
             float2 z[4];
@@ -702,7 +707,7 @@ __global__ __launch_bounds__(kBlock) void k_far_field_cols(Dims d, const float2*
                     b2[v] = imag ? p.x : -p.y;
                 }
 #pragma unroll
-                for (int v = 0; v < 3; ++v) acc[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(z[s].y, b2[v], acc[v], 0, 0, 0);
+                for (int v = 0; v < 3; ++v) acc2[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(z[s].y, b2[v], acc2[v], 0, 0, 0);
             }
         }
         // T[column][component][group], and the phase table's rows of the columns
@@ -710,7 +715,7 @@ __global__ __launch_bounds__(kBlock) void k_far_field_cols(Dims d, const float2*
 #pragma unroll
         for (int v = 0; v < 3; ++v)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) t[(v * kFFGroups + e) * 2] = acc[v][e];
+            for (int e = 0; e < 4; ++e) t[(v * kFFGroups + e) * 2] = acc[v][e] + acc2[v][e];
         if (m == 0) {   // T is zero where there is no column
             sy[wave * kFFCols + k] = (unsigned)(d.ni + (max(ca, 0) & (d.nj - 1))) * ndirs;
             sy[wave * kFFCols + k + 4] = (unsigned)(d.ni + (max(cb, 0) & (d.nj - 1))) * ndirs;
