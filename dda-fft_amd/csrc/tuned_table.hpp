@@ -3,7 +3,8 @@
 // sides per X-pass tile; x_blocks: X-pass launch size up to which groups of
 // right-hand sides are spread over blocks (1 << 30: each group its own
 // block); graph: iterations replayed as captured HIP graphs; fuse: z- and
-// y-forward transforms of an i-plane in one kernel.
+// y-forward transforms of an i-plane in one kernel (always, whatever stands
+// here, where the plane has at most 2^11 cells).
 #pragma once
 
 namespace ddafft {
@@ -17,7 +18,7 @@ struct TunedEntry {
 constexpr int kTunedBatchWidth = 12;
 
 constexpr TunedEntry kTuned[] = {
-    {32, 32, 32, 2, 1, 2048, 0, 0},   // X pass 11.8 us, solve 0.893 ms
+    {32, 32, 32, 2, 1, 2048, 0, 1},   // X pass 11.8 us, solve 0.893 ms
     {64, 64, 64, 2, 2, 1 << 30, 0, 0},   // X pass 42.4 us, solve 2.533 ms
     {128, 128, 128, 2, 2, 1 << 30, 1, 0},   // X pass 380.2 us, solve 8.411 ms
     {256, 256, 256, 2, 2, 1 << 30, 1, 0},   // X pass 4001.6 us, solve 83.154 ms

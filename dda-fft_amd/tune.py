@@ -7,7 +7,7 @@ Measures, on the GPU it runs on, for each (lattice, right-hand sides) case:
   A-hat read, and runs of groups per block (one group per block, or runs
   long enough to cut the launch to 8192 / 2048 blocks);
 - the z- and y-forward transforms as one kernel per i-plane against two
-  passes (planes up to 64 x 64);
+  passes (64 x 64 planes; smaller ones always run fused);
 - a whole BiCGStab solve with its iterations replayed from captured HIP
   graphs against launched kernel by kernel;
 - for the batched Monte-Carlo workload, the number of realizations in
@@ -63,6 +63,12 @@ def time_zy(ctx, nrhs, reps):
     return float(km[0] + km[1])
 
 
+def always_fused(dims):
+    """Planes whose forward and inverse passes the library always fuses (axes
+    of 8 points up, at most 2^11 cells)."""
+    return min(dims[1:]) >= 8 and dims[1] * dims[2] <= 2048
+
+
 def target(dims, x=5.0, m=1.5 + 0.01j):
     kd = np.float32(2.0 * x / dims[0])
     occ, _ = ddafft.target_ellipsoid(dims, min(1.0, dims[1] / dims[0]), min(1.0, dims[2] / dims[0]))
@@ -85,8 +91,8 @@ def tune_case(dims, nrhs, reps, log):
             best = (t, rb, xb)
     _, rb, xb = best
     ctx.set_tuning(x_rb=rb, x_blocks=xb)
-    fuse = 0
-    if dims[1] <= 64 and dims[2] <= 64:
+    fuse = 1 if always_fused(dims) else 0
+    if not fuse and dims[1] <= 64 and dims[2] <= 64:
         tz = {}
         for f in (0, 1, 0, 1):
             ctx.set_tuning(fuse_zy=f)
@@ -95,7 +101,8 @@ def tune_case(dims, nrhs, reps, log):
         fuse = 1 if tz[1] < tz[0] else 0
         log("%-14s R=%-2d z/y forward: two passes %.1f us, fused %.1f us -> fuse=%d" % (
             "x".join(map(str, dims)), nrhs, tz[0] * 1e3, tz[1] * 1e3, fuse))
-    ctx.set_tuning(fuse_zy=fuse)
+    if not always_fused(dims):   # else as the library does by itself: 0 would split the passes
+        ctx.set_tuning(fuse_zy=fuse)
     # graphs against launches on a whole solve of nrhs right-hand sides
     kinc = np.array([0, 0, 1], np.float32)
     einc = np.array([np.eye(3)[r % 2] for r in range(nrhs)], np.complex64)
@@ -152,7 +159,8 @@ def write_table(entries, width, path):
              "// sides per X-pass tile; x_blocks: X-pass launch size up to which groups of",
              "// right-hand sides are spread over blocks (1 << 30: each group its own",
              "// block); graph: iterations replayed as captured HIP graphs; fuse: z- and",
-             "// y-forward transforms of an i-plane in one kernel.",
+             "// y-forward transforms of an i-plane in one kernel (always, whatever stands",
+             "// here, where the plane has at most 2^11 cells).",
              "#pragma once", "", "namespace ddafft {", "",
              "struct TunedEntry {", "    int ni, nj, nl, nrhs, x_rb, x_blocks, graph, fuse;", "};", "",
              "// realizations in flight in ddafft_solve_batch for the batched Monte-Carlo",
