@@ -266,7 +266,9 @@ struct ddafft_ctx : Directions {
     int ahat_mode = 0;                 // 0: full Â as the reference builds it; 1: one octant (Nyquist planes zeroed)
     int ff_mfma = -1;                  // far field on the matrix cores: -1 default, 0 off, 1 on
     int ff_group = -1;                 // far field by columns: -1 default (on), 0 off, 1 on
-    int ff_chunk_max = 0;              // set by an allocation-free solve: column chunks that its scratch has room for
+    // set by an allocation-free solve whose scratch has no room for more:
+    int ff_chunk_max = 0;              // far-field column chunks at most (0: as many as the rule says)
+    bool yzi_off = false;              // the inverse passes apart (fewer partial sums where planes have 8 rows)
     // launch schedule, 0 / -1: from the tuned table, else the built-in rule
     int x_blocks = 0;                  // X pass: blocks per launch up to which right-hand-side groups are spread
     int x_rb = 0;                      // X pass: right-hand sides per tile
@@ -546,9 +548,8 @@ bool zyf_launch(ddafft_ctx* c, const Dims& d, const ProArgs& pa, SolveState* st,
 // 101.0; 32x32x64, 16 RHS 189.5 -> 175.7; 64x128x8, 4 RHS 123 -> 95); planes of
 // twice that (132 KB, one block) lost where it counts: 64^3, 2 RHS 125 -> 129,
 // 64x32x128, 6 RHS 343 -> 353.
-bool yzi_on(const ddafft_ctx* c, int kind) {
-    return one_component(kind) && small_plane(c->d) && c->fuse_zy != 0;
-}
+bool yzi_fits(const ddafft_ctx* c) { return small_plane(c->d) && c->fuse_zy != 0 && !c->yzi_off; }
+bool yzi_on(const ddafft_ctx* c, int kind) { return one_component(kind) && yzi_fits(c); }
 
 bool yzi_launch(ddafft_ctx* c, const Dims& d, const float2* b3, SolveState* st, const EpiArgs& ea, int C, hipStream_t s) {
     const dim3 grid(d.ni, C);
@@ -567,7 +568,9 @@ bool yzi_launch(ddafft_ctx* c, const Dims& d, const float2* b3, SolveState* st, 
 
 // Blocks of a matvec's epilogue per right-hand side (its partial sums).
 int epi_blocks(const ddafft_ctx* c, int kind) { return yzi_on(c, kind) ? 3 * c->d.ni : zi_blocks(c->d); }
-int max_epi_blocks(const Dims& d) { return std::max(zi_blocks(d), 3 * d.ni); }
+int max_epi_blocks(const ddafft_ctx* c) {
+    return yzi_fits(c) ? std::max(zi_blocks(c->d), 3 * c->d.ni) : zi_blocks(c->d);
+}
 
 // One matvec of nrhs right-hand sides: ZF -> YF (or the fused ZYF) -> X ->
 // YI -> ZI (or the fused YZI).
@@ -1030,7 +1033,9 @@ bool mid_within(const ddafft_ctx* c, const Dims& d, int nblk) {
 }
 
 // Partial sums of a solve per right-hand side, in doubles.
-size_t step_partials(const Dims& d) { return (size_t)std::max(max_epi_blocks(d), update_blocks(d)) * kSlots; }
+size_t step_partials(const ddafft_ctx* c) {
+    return (size_t)std::max(max_epi_blocks(c), update_blocks(c->d)) * kSlots;
+}
 
 }  // namespace
 
@@ -1135,7 +1140,7 @@ int ddafft_create(int ni, int nj, int nl, float kd, int nrhs_max, ddafft_ctx** o
     // at least 512 KB: room for the far field's partial sums of most direction
     // sets, which would otherwise be allocated by the first solve
     if (!rc)
-        rc = ensure_partials(c, std::max<size_t>((size_t)nrhs_max * std::max<size_t>(step_partials(c->d), 1024 * kSlots), (size_t)1 << 16));
+        rc = ensure_partials(c, std::max<size_t>((size_t)nrhs_max * std::max<size_t>(step_partials(c), 1024 * kSlots), (size_t)1 << 16));
     if (rc) {
         ddafft_destroy(c);
         return rc;
@@ -2012,7 +2017,7 @@ int run_begin(Run& r) {
     }
     TRY(upload(c, c->st, s0.data(), r.nrhs * sizeof(SolveState)));
     const bool mid_room = !t_noalloc && (long long)update_blocks(d) * r.nrhs <= kMidUpdates;   // mid_within
-    TRY(ensure_partials(c, (size_t)r.nrhs * (step_partials(d) + (mid_room ? kMidBlocks * kSlots : 0))));
+    TRY(ensure_partials(c, (size_t)r.nrhs * (step_partials(c) + (mid_room ? kMidBlocks * kSlots : 0))));
     TRY(flush_small(c));   // every staged input of the solve, in one copy
     if (c->pending_first_approx) {
         c->pending_first_approx = false;
@@ -2374,13 +2379,23 @@ int ddafft_solve_noalloc(ddafft_ctx* c, int nrhs, int solver, float tau, int max
         off += (b + 255) & ~(size_t)255;
         return o;
     };
-    // the plan of the scratch; the far field's columns in fewer chunks where its partial sums do not fit
-    c->ff_chunk_max = 0;
+    // the reference-order sums' terms, at least (they get all of the rest)
+    const size_t seq_min =
+        c->sum_mode ? std::max((size_t)2 * nrhs * c->ncells, (size_t)nrhs * std::max(ndirs, 1) * 6) : 0;
+    // the plan of the scratch; where the partial sums do not fit, the far
+    // field's columns in fewer chunks, then the inverse passes apart
+    struct Limits {   // they hold for this call only
+        ddafft_ctx* c;
+        ~Limits() {
+            c->ff_chunk_max = 0;
+            c->yzi_off = false;
+        }
+    } limits{c};
     for (;;) {
         off = 0;
         res = 0;   // results, laid out as fin_layout lays them out
         obs_blocks(c, nrhs, ndirs, ffn, ffS, &cb, &fchunk);
-        n_part = std::max({(size_t)nrhs * step_partials(d), (size_t)nrhs * cb * 2,
+        n_part = std::max({(size_t)nrhs * step_partials(c), (size_t)nrhs * cb * 2,
                            (size_t)nrhs * fchunk * std::max(ndirs, 1) * 6});
         n_hist = (size_t)c->nrhs_max * (max_step + 1);
         n_esc = (size_t)nrhs * ndirs * 3;
@@ -2399,18 +2414,21 @@ int ddafft_solve_noalloc(ddafft_ctx* c, int nrhs, int solver, float tau, int max
         o_tab = take(n_tab * sizeof(float2));
         o_dirs = take(n_dirs * sizeof(float));
         o_res = take(res);
-        if (off <= kScratchBytes || fchunk <= 1 || !ff_cols_on(c, ndirs, ffn, ffS)) break;
-        c->ff_chunk_max = fchunk / 2;
+        if (off + seq_min * sizeof(float) <= kScratchBytes) break;
+        if (fchunk > 1 && ff_cols_on(c, ndirs, ffn, ffS)) {
+            c->ff_chunk_max = fchunk / 2;
+        } else if (yzi_fits(c) && max_epi_blocks(c) > std::max(zi_blocks(d), update_blocks(d))) {
+            c->yzi_off = true;
+            c->ff_chunk_max = 0;
+        } else {
+            break;
+        }
     }
-    struct Unlimit {   // the cap holds for this call only
-        ddafft_ctx* c;
-        ~Unlimit() { c->ff_chunk_max = 0; }
-    } unlimit{c};
     size_t o_seq = 0, n_seq = 0;
     if (c->sum_mode) {   // the sequential-sum terms get the rest
         o_seq = take(0);
         n_seq = off < kScratchBytes ? (kScratchBytes - off) / sizeof(float) : 0;
-        if (n_seq < (size_t)2 * nrhs * c->ncells || n_seq < (size_t)nrhs * std::max(ndirs, 1) * 6)
+        if (n_seq < seq_min)
             return fail(DDAFFT_EINVAL, "the reference-order sums of this solve exceed the allocation-free scratch");
     }
     if (off > kScratchBytes || res > sizeof(c->noalloc_dn))

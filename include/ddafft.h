@@ -103,13 +103,14 @@ int ddafft_solve(ddafft_ctx* ctx, int nrhs, int solver, float tau, int max_step,
 /* ddafft_solve that allocates nothing.  No counterpart in the reference: it
  * is for callers that cannot allocate memory during a solve (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).
- * Same arguments and results as ddafft_solve, bit for bit (except the far
- * field where its partial sums do not fit the scratch: then fewer of them,
- * within about 1e-7).  Its
+ * Same arguments and results as ddafft_solve, bit for bit, except where the
+ * partial sums do not fit the scratch: then the far field has fewer of them
+ * (within about 1e-7), and lattices with n_j = 8 run their inverse passes
+ * apart, as DDAFFT_TUNE_FUSE_ZY 0 does.  Its
  * scratch (block partials, discrepancy history, far-field partials and phase
  * tables, per-call directions, results on their way back, reference-order
- * sum terms) lives in a fixed 32 MiB device array, one per GPU, that every such call on that GPU
- * shares: calls that overlap on one GPU race.  A solve whose
+ * sum terms) lives in a fixed 32 MiB device array, one per GPU, that every such
+ * call on that GPU shares: calls that overlap on one GPU race.  A solve whose
  * scratch would exceed it fails with DDAFFT_EINVAL and a message giving the
  * size needed; results are limited to 1 MiB per call.  Inputs are copied from
  * the caller's memory (no page-locked staging is allocated). */
