@@ -884,11 +884,15 @@ int upload_begin(ddafft_ctx* c, size_t bytes) {
     return pinned_reserve(c, &c->up, &c->up_cap, bytes);
 }
 
-int field_in(ddafft_ctx* c, const float* host_aos, float2* dev_soa, float2* staging) {
+// masked (may be nullptr): also a copy that is zero off the dipoles
+int field_in(ddafft_ctx* c, const float* host_aos, float2* dev_soa, float2* staging, float2* masked = nullptr) {
     const long long n = c->d.n;
+    const int grid = (int)std::min<long long>((n + kBlock - 1) / kBlock, 4096);
     HIPCHECK(hipMemcpyAsync(staging, host_aos, (size_t)n * 3 * sizeof(float2), hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(k_aos_to_soa, (int)std::min<long long>((n + kBlock - 1) / kBlock, 4096), kBlock, 0, c->stream, n, staging,
-                                                                                                     dev_soa);
+    if (masked)
+        hipLaunchKernelGGL(k_aos_to_soa_masked, grid, kBlock, 0, c->stream, n, staging, c->dipf, dev_soa, masked);
+    else
+        hipLaunchKernelGGL(k_aos_to_soa, grid, kBlock, 0, c->stream, n, staging, dev_soa);
     HIPCHECK(hipGetLastError());
     return DDAFFT_OK;
 }
@@ -2923,7 +2927,9 @@ int ddafft_far_field(ddafft_ctx* c, const float* p, int ndirs, const float* dirs
     if (!c || !p || !dirs || !esc || ndirs < 1) return fail(DDAFFT_EINVAL, "bad argument");
     if (!c->have_target) return fail(DDAFFT_ESTATE, "set_target first");
     TRY(ddafft_set_directions(c, ndirs, dirs));
-    TRY(field_in(c, p, c->P, c->Y));
+    // the columns' sums run over every cell they span: on a copy that is zero off the dipoles
+    const bool cols = ff_cols_on(c, ndirs, c->ffg_n, c->ffg_S);
+    TRY(field_in(c, p, c->P, c->Y, cols ? c->X : nullptr));
     // cross sections are computed alongside; their values are discarded
     std::vector<float> zero_alpha((size_t)2 * c->nmat, 0.f);
     TRY(upload(c, c->alpha, zero_alpha.data(), zero_alpha.size() * sizeof(float)));
@@ -2931,10 +2937,7 @@ int ddafft_far_field(ddafft_ctx* c, const float* p, int ndirs, const float* dirs
     const float e[6] = {1.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     TRY(upload(c, c->einc, e, sizeof(e)));
     TRY(upload_incidence(c, 1, kz));
-    // the columns' sums run over every cell they span: a copy that is zero off the dipoles
-    hipLaunchKernelGGL(k_mask_field, update_blocks(c->d), kBlock, 0, c->stream, c->d, c->dipf, c->P, c->X);
-    HIPCHECK(hipGetLastError());
-    return observables(c, 1, e, ndirs, c->dirs, 0, esc, nullptr, nullptr, c->X);
+    return observables(c, 1, e, ndirs, c->dirs, 0, esc, nullptr, nullptr, cols ? c->X : c->P);
 }
 
 int ddafft_profile(ddafft_ctx* c, int enable, double* pass_ms, long long* matvecs) {
