@@ -224,7 +224,10 @@ def large_run(cpu=False):
 def matvec_scaling(reps=50):
     """Average duration of each matvec pass (HIP events, ddafft_time_matvec)
     for 1..16 right-hand sides sharing one operator, with the algorithmic
-    GB/s of each pass."""
+    GB/s of each pass.  Where a pass runs fused with its neighbour, its own
+    event pair encloses nothing (about 5 us, less than any pass with its
+    events): a dash stands for its rate, and the neighbour's counts both
+    passes' bytes without the buffer between them."""
     print("# lattice nrhs | total_us us_per_rhs | zf yf x yi zi (us) | zf yf x yi zi (GB/s) | matvec GB/s")
     for dims, rmax in (((32, 32, 32), 16), ((64, 64, 64), 16), ((128, 128, 128), 4)):
         n = int(np.prod(dims))
@@ -235,10 +238,18 @@ def matvec_scaling(reps=50):
         while r <= rmax:
             km, tot = ctx.time_matvec(r, reps)
             by = matvec_bytes(n, r)
-            gbs = [by[k] / (t * 1e-3) / 1e9 for k, t in zip(("zf", "yf", "x", "yi", "zi"), km)]
+            names = ("zf", "yf", "x", "yi", "zi")
+            rate = dict(zip(names, (by[k] / (t * 1e-3) / 1e9 for k, t in zip(names, km))))
+            for a, b in (("zf", "yf"), ("yi", "zi")):
+                empty = [k for k in (a, b) if km[names.index(k)] < 5.5e-3]
+                if len(empty) == 1:
+                    full = b if empty[0] == a else a
+                    between = 2 * 48 * n * r   # B1 or B4, written and read
+                    rate[full] = (by[a] + by[b] - between) / (km[names.index(full)] * 1e-3) / 1e9
+                    rate[empty[0]] = None
             print("%s %2d | %8.1f %8.1f | %s | %s | %6.0f" % (
                 "x".join(map(str, dims)), r, tot * 1e3, tot * 1e3 / r, " ".join("%6.1f" % (v * 1e3) for v in km),
-                " ".join("%5.0f" % g for g in gbs), sum(by.values()) / (tot * 1e-3) / 1e9), flush=True)
+                " ".join("    -" if rate[k] is None else "%5.0f" % rate[k] for k in names), sum(by.values()) / (tot * 1e-3) / 1e9), flush=True)
             r *= 2
         ctx.close()
 

@@ -542,8 +542,8 @@ bool zyf_launch(ddafft_ctx* c, const Dims& d, const ProArgs& pa, SolveState* st,
 
 // Whether a matvec's inverse y and z passes run fused (k_yzi): plane shapes it
 // is built for and an epilogue that one component at a time can finish.  One
-// block holds all of the plane's padded lines, so it is ahead as far as they
-// fit 66 KB of LDS, two blocks per CU (CG step, MI355X, YI + ZI against YZI:
+// block holds all of the plane's padded lines, so it is ahead as far as two
+// such blocks fit a CU (67 to 73 KB of LDS at 2^11 cells; CG step, MI355X, YI + ZI against YZI:
 // 16^3, 2 RHS 39.9 -> 36.2 us; 32^3, 2 RHS 48.7 -> 46.6; 32^3, 16 RHS 114.4 ->
 // 101.0; 32x32x64, 16 RHS 189.5 -> 175.7; 64x128x8, 4 RHS 123 -> 95); planes of
 // twice that (132 KB, one block) lost where it counts: 64^3, 2 RHS 125 -> 129,

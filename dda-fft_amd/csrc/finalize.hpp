@@ -83,29 +83,27 @@ __device__ void end_step(SolveState& s, const FinArgs& fa, int rhs, int o, doubl
 }
 
 // The fixed-order FP64 sum of one right-hand side's block partials, by every
-// thread of a block of BT; the result is valid in thread 0.  (Blocks of 512
-// threads add only zeros to the sums of 256 while nblk <= 256.)
-template <int BT = kBlock>
+// thread of a block of kBlock; the result is valid in thread 0.
 __device__ __forceinline__ void sum_partials(const FinArgs& fa, int rhs, double (&v)[kSlots], double* red) {
     const double* p = fa.partials + (long long)rhs * fa.nblk * kSlots;
-    // each thread sums partials b = tid, tid + BT, ... in that order; the
+    // each thread sums partials b = tid, tid + kBlock, ... in that order; the
     // loads of four of them are in flight together
     constexpr int kBatch = 4;
-    for (int b0 = threadIdx.x; b0 < fa.nblk; b0 += kBatch * BT) {
+    for (int b0 = threadIdx.x; b0 < fa.nblk; b0 += kBatch * kBlock) {
         double t[kBatch][kSlots];
 #pragma unroll
         for (int u = 0; u < kBatch; ++u) {
-            const int b = b0 + u * BT;
+            const int b = b0 + u * kBlock;
 #pragma unroll
             for (int q = 0; q < kSlots; ++q) t[u][q] = b < fa.nblk ? p[(long long)b * kSlots + q] : 0.0;
         }
 #pragma unroll
         for (int u = 0; u < kBatch; ++u)
-            if (b0 + u * BT < fa.nblk)
+            if (b0 + u * kBlock < fa.nblk)
 #pragma unroll
                 for (int q = 0; q < kSlots; ++q) v[q] += t[u][q];
     }
-    block_sum<kSlots, BT>(v, red);
+    block_sum<kSlots>(v, red);
 }
 
 // The scalar steps inside an iteration: they read fields of the state that

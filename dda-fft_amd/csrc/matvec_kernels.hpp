@@ -460,8 +460,9 @@ __global__ __launch_bounds__((ZyfShape<NJ, NL>::BT)) void k_zyf(Dims d, ProArgs 
 }
 
 // ZYF for planes of at most 2^11 cells: both parities of the z and of the y
-// frequencies at once, 2 n_j z lines and then 4 n_l y lines in LDS (66 KB at
-// most), where k_zyf runs them one after another.  The short chain is what
+// frequencies at once, 2 n_j z lines and then 4 n_l y lines in LDS (74 KB
+// with the twiddles at 8 x 256, 64 to 69 KB in the other shapes of 2^11
+// cells), where k_zyf runs them one after another.  The short chain is what
 // counts here: these planes give a block little work and a launch few blocks
 // (zyf_launch has the rule and the figures).
 template <int NJ, int NL>

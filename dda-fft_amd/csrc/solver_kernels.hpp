@@ -769,10 +769,12 @@ __global__ __launch_bounds__(kBlock) DDA_WAVES_PER_EU(4, 5) void k_far_field_col
 // The far field that an adjoint source is built from (gradients of S11), for
 // direction sets of groups that share z: BiCGStab multiplies the last bits of
 // its source by up to 1e4 within a few steps near a breakdown, so those calls
-// keep these float sums, whose bits their gradients have had, rather than the
-// faster column form's (which is as exact, but rounds otherwise).  The l-sums
-// are formed once per group, as there; group g holds the directions g,
-// g + ngroups, ..., g + (S - 1) ngroups.
+// keep these float sums, with which their gradients were checked, rather than
+// the faster column form's (which is as exact, but rounds otherwise).  The FP64
+// partials of the chunks are added by k_far_field_sum, four runs of them apart;
+// another order there reaches the float result only at a rounding boundary.
+// The l-sums are formed once per group, as there; group g holds the directions
+// g, g + ngroups, ..., g + (S - 1) ngroups.
 // The dipole list is cut into segments of at most kFFSeg consecutive dipoles
 // of one (i, j) column (seg: {first dipole, (i nj + j) << 6 | count}).
 // Stage 1: one thread per segment sums its T for the block's G groups, from
