@@ -18,16 +18,16 @@ struct TunedEntry {
 constexpr int kTunedBatchWidth = 12;
 
 constexpr TunedEntry kTuned[] = {
-    {32, 32, 32, 2, 1, 2048, 0, 1},   // X pass 11.8 us, solve 0.893 ms
-    {64, 64, 64, 2, 2, 1 << 30, 0, 0},   // X pass 42.4 us, solve 2.533 ms
-    {128, 128, 128, 2, 2, 1 << 30, 1, 0},   // X pass 380.2 us, solve 8.411 ms
-    {256, 256, 256, 2, 2, 1 << 30, 1, 0},   // X pass 4001.6 us, solve 83.154 ms
-    {32, 32, 32, 16, 2, 1 << 30, 0, 1},   // X pass 34.5 us, solve 2.210 ms
-    {32, 32, 64, 16, 2, 1 << 30, 0, 1},   // X pass 69.2 us, solve 4.040 ms
-    {64, 64, 64, 16, 2, 1 << 30, 1, 1},   // X pass 295.1 us, solve 15.458 ms
-    {32, 32, 64, 2, 2, 1 << 30, 0, 1},   // X pass 16.7 us, solve 1.055 ms
-    {64, 64, 64, 4, 2, 1 << 30, 0, 0},   // X pass 90.6 us, solve 4.521 ms
-    {128, 128, 128, 4, 2, 1 << 30, 0, 0},   // X pass 708.0 us, solve 16.209 ms
+    {32, 32, 32, 2, 1, 2048, 0, 1},   // X pass 11.7 us, solve 0.695 ms
+    {64, 64, 64, 2, 2, 1 << 30, 0, 0},   // X pass 41.4 us, solve 2.225 ms
+    {128, 128, 128, 2, 2, 1 << 30, 1, 0},   // X pass 371.4 us, solve 7.908 ms
+    {256, 256, 256, 2, 2, 1 << 30, 1, 0},   // X pass 3262.3 us, solve 66.691 ms
+    {32, 32, 32, 16, 2, 1 << 30, 0, 1},   // X pass 33.5 us, solve 1.817 ms
+    {32, 32, 64, 16, 2, 1 << 30, 0, 1},   // X pass 59.6 us, solve 2.978 ms
+    {64, 64, 64, 16, 2, 1 << 30, 1, 1},   // X pass 292.8 us, solve 14.756 ms
+    {32, 32, 64, 2, 2, 1 << 30, 0, 1},   // X pass 15.7 us, solve 0.934 ms
+    {64, 64, 64, 4, 2, 1 << 30, 0, 0},   // X pass 83.7 us, solve 4.115 ms
+    {128, 128, 128, 4, 2, 1 << 30, 0, 0},   // X pass 692.1 us, solve 15.295 ms
 };
 
 }  // namespace ddafft
